@@ -1,0 +1,84 @@
+"""The label fields' device layout (9^3 corner values a slot, a record a brick) against
+the oracle, which reads the stored layout voxel by voxel: every query the same bits at
+points in brick interiors, on brick faces and edges, at the grid's sides and outside it,
+for labels the cell's brick lists and labels it does not.
+"""
+import numpy as np
+import pytest
+
+from conftest import Fixture, bits
+from trussnet_amd._abi import Nodes, RelaxParams
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def tn():
+    from trussnet_amd import relax
+
+    if relax.device_count() < 1:
+        pytest.fail("no HIP device visible")
+    return relax
+
+
+def _points(shape, vs, seed):
+    """Uniform points reaching out of the grid, and points whose coordinates sit at and
+    beside brick faces (voxels 8 k - 1 .. 8 k + 1, half voxels between)."""
+    rng = np.random.default_rng(seed)
+    n = np.array(shape[::-1])
+    free = rng.uniform(-2.5, n + 1.5, (6000, 3))
+    near = 8 * rng.integers(0, np.maximum(2, n // 8 + 1), (6000, 3)) + rng.choice(
+        [-1.5, -1.0, -0.75, -0.5, -0.25, 0.0, 0.3, 0.5, 1.0], (6000, 3))
+    ends = rng.choice([-1.0, -0.5, 0.0, 1.0], (500, 3)) + rng.integers(0, 2, (500, 3)) * (n - 1)
+    return (np.concatenate([free, near, ends]) * np.array(vs)).astype(np.float32)
+
+
+@pytest.mark.parametrize("shape,vs,blocks,nlab", [
+    ((24, 16, 32), (1.0, 1.0, 1.0), 6, 3),      # whole bricks
+    ((17, 9, 25), (0.9, 1.1, 1.3), 5, 4),       # one voxel over a brick along each axis
+    ((7, 8, 15), (2.0, 0.5, 1.0), 3, 5),        # less than a brick
+    ((1, 1, 1), (1.0, 1.0, 1.0), 1, 2),
+    ((20, 23, 31), (1.0, 1.0, 1.0), 2, 60),     # more labels near a brick than it lists
+])
+def test_queries_equal_the_oracle(tn, oracle_lib, shape, vs, blocks, nlab):
+    from trussnet_amd import gridbuild
+
+    rng = np.random.default_rng(7)
+    cells = [(s + blocks - 1) // blocks for s in shape]
+    lab = rng.integers(0, nlab, cells).astype(np.uint16)
+    for ax in range(3):
+        lab = np.repeat(lab, blocks, axis=ax)
+    lab = np.ascontiguousarray(lab[:shape[0], :shape[1], :shape[2]])
+    grid = gridbuild.build(lab, vs, device=0)
+    X = _points(shape, vs, 3)
+    one = Nodes(np.zeros((1, 3)), np.zeros(1), np.zeros(1), np.full((1, 2), 0xFFFF))
+    with tn.Plan(grid, one, RelaxParams()) as plan:
+        for a, b in ((0, 1), (1, 2), (nlab - 1, 0), (nlab + 5, 1), (0xFFFE, 0)):
+            got = plan.field_points(a, b, X)
+            want = oracle_lib.field_points(grid, a, b, X)
+            for g, w, name in zip(got, want, ("phi", "psi", "grad", "label", "second")):
+                assert np.array_equal(bits(g), bits(w)), (shape, a, b, name)
+
+
+def test_stored_layout_where_the_slots_do_not_fit(tn):
+    """A relaxation that just fits the no-allocation entry point's memory has no room left
+    for the slots and reads the stored layout: the same bits."""
+    case = Fixture("spheres64")
+    s = case.seeds
+    reps = 90
+    P, lab, typ, part = np.tile(s.P, (reps, 1)), np.tile(s.lab, reps), np.tile(s.typ, reps), np.tile(s.part, (reps, 1))
+    prm = RelaxParams(max_iters=3, dptol=0.0)
+
+    def run(n):
+        try:
+            return tn.relax_noalloc(case.grid, Nodes(P[:n], lab[:n], typ[:n], part[:n]), prm, device=0)
+        except tn.DeviceError:
+            return None
+
+    lo, hi = 1000, s.n * reps
+    while hi - lo > 500:   # the largest count that fits, to 0.25 MB
+        mid = (lo + hi) // 2
+        lo, hi = (mid, hi) if run(mid) is not None else (lo, mid)
+    got, _ = run(lo)
+    want, _ = tn.relax(case.grid, Nodes(P[:lo], lab[:lo], typ[:lo], part[:lo]), prm, device=0)
+    assert got.equal(want)

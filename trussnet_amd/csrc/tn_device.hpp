@@ -50,6 +50,10 @@ struct Field {
     const float* __restrict__ gI;    // gray-scale mode: the intensity per voxel
     const float* __restrict__ gTW;   // gray-scale mode: [t_0..t_{m-1}, W_0..W_{m-1}]
     int gm;                          // gray-scale mode: m > 0 thresholds (0: a label volume)
+    // a label volume's fields laid out for the device's queries (tn_apron.hpp), or null
+    const float* __restrict__ ap;
+    const uint4* __restrict__ rec;
+    static constexpr bool kPlain = false;   // (PlainField: a label volume with ap and rec)
     // this struct's copy in device memory. Out-of-line functions take it instead of a
     // reference: a reference to the kernel argument would move the whole struct into
     // scratch memory and turn the kernel's loads through its pointers into flat loads.
@@ -769,6 +773,10 @@ __device__ __noinline__ float4 psi_grad_point(const Field* fp, int a, int b, P3 
     return psi_grad_at(f, a, b, p, pc);
 }
 
+__device__ __forceinline__ float4 psi_grad_once(const Field& f, int a, int b, P3 p) {
+    return psi_grad_point(f.self, a, b, p);
+}
+
 // The labels of p's brick (v2m_labels_near, src/opencl/v2m_seed_body.cl:42-59) as
 // a brick index and a count: bl_lab[b*16 + s] for s < n (b = -1: outside the grid,
 // the one label 0).
@@ -980,13 +988,21 @@ __device__ __forceinline__ OwnerPsi owner_psi_at(const Field& f, int a, P3 p) {
     return r;
 }
 
+}  // namespace tnd
+
+#include "tn_apron.hpp"
+
+namespace tnd {
+
 __device__ __forceinline__ P3 along(P3 p, float sg, float t, P3 u) {
     return p3(p.x + sg * t * u.x, p.y + sg * t * u.y, p.z + sg * t * u.z);
 }
 
 // v2m_bisect_dir, src/opencl/v2m_seed_body.cl:255-320 (doubling probes, then Illinois).
+// One loop over both phases, so that the field is evaluated at one place of the code.
 // On success the returned point is the last point probed, so pc then holds its cell.
-__device__ __forceinline__ P3ok bracket_along(const Field& f, int a, int b, P3 p, P3 u, float v0, float rad, float tg,
+template <class F>
+__device__ __forceinline__ P3ok bracket_along(const F& f, int a, int b, P3 p, P3 u, float v0, float rad, float tg,
                                               PsiCell& pc) {
     P3ok r;
     r.p = p;
@@ -994,33 +1010,36 @@ __device__ __forceinline__ P3ok bracket_along(const Field& f, int a, int b, P3 p
     if (v0 == 0.0f) {
         return r;
     }
+    r.ok = 0;
     const float sg = v0 > 0.0f ? -1.0f : 1.0f;
     float t0 = 0.0f, t1 = -1.0f, f0 = v0, f1 = 0.0f;
     float t = (tg > 0.0f && tg < rad) ? tg : 0.25f * rad;
-    for (int k = 0; k < 8; ++k) {
+    bool bracketed = false;
+    int left = 8, side = 0;   // probes left in this phase
+#pragma clang loop unroll(disable)
+    while (left > 0) {
         const float v = psi_at(f, a, b, along(p, sg, t, u), pc);
-        if ((v > 0.0f) != (v0 > 0.0f) || v == 0.0f) {
+        --left;
+        if (!bracketed) {
+            if ((v > 0.0f) != (v0 > 0.0f) || v == 0.0f) {
+                t1 = t;
+                f1 = v;
+                if (t1 < 0.0f) {
+                    return r;
+                }
+                bracketed = true;
+                left = 8;
+            } else {
+                t0 = t;
+                f0 = v;
+                if (t >= rad) {
+                    return r;
+                }
+                t = fminf(2.0f * t, rad);
+                continue;
+            }
+        } else if ((v > 0.0f) == (f1 > 0.0f)) {
             t1 = t;
-            f1 = v;
-            break;
-        }
-        t0 = t;
-        f0 = v;
-        if (t >= rad) {
-            break;
-        }
-        t = fminf(2.0f * t, rad);
-    }
-    if (t1 < 0.0f) {
-        r.ok = 0;
-        return r;
-    }
-    int side = 0;
-    for (int it = 0; it < 8 && f1 != 0.0f && fabsf(t1 - t0) > 1e-4f * rad; ++it) {
-        const float tm = (f0 != f1) ? t1 - f1 * (t1 - t0) / (f1 - f0) : 0.5f * (t0 + t1);
-        const float v = psi_at(f, a, b, along(p, sg, tm, u), pc);
-        if ((v > 0.0f) == (f1 > 0.0f)) {
-            t1 = tm;
             f1 = v;
             if (side == -1) {
                 f0 *= 0.5f;
@@ -1029,20 +1048,27 @@ __device__ __forceinline__ P3ok bracket_along(const Field& f, int a, int b, P3 p
         } else {
             t0 = t1;
             f0 = f1;
-            t1 = tm;
+            t1 = t;
             f1 = v;
             side = 1;
         }
+        if (!(f1 != 0.0f && fabsf(t1 - t0) > 1e-4f * rad)) {
+            break;
+        }
+        t = (f0 != f1) ? t1 - f1 * (t1 - t0) / (f1 - f0) : 0.5f * (t0 + t1);
     }
-    r.p.x = p.x + sg * t1 * u.x;
-    r.p.y = p.y + sg * t1 * u.y;
-    r.p.z = p.z + sg * t1 * u.z;
+    if (!bracketed) {
+        return r;
+    }
+    r.ok = 1;
+    r.p = along(p, sg, t1, u);
     return r;
 }
 
 // v2m_project1, src/opencl/v2m_seed_body.cl:324-335 (ok = 0: p unchanged), with the
 // a|b cell cache of the caller
-__device__ __forceinline__ P3ok onto_interface_at(const Field& f, int a, int b, P3 p, float rad, PsiCell& pc) {
+template <class F>
+__device__ __forceinline__ P3ok onto_interface_at(const F& f, int a, int b, P3 p, float rad, PsiCell& pc) {
     const float4 g = psi_grad_at(f, a, b, p, pc);
     const float gn = sqrtf(g.x * g.x + g.y * g.y + g.z * g.z);
     if (gn < 1e-9f) {
@@ -1055,84 +1081,100 @@ __device__ __forceinline__ P3ok onto_interface_at(const Field& f, int a, int b, 
     return bracket_along(f, a, b, p, u, g.w, rad, 1.5f * fabsf(g.w) / gn, pc);
 }
 
-__device__ __noinline__ P3ok onto_interface(const Field* fp, int a, int b, P3 p, float rad) {
-    const Field f = *fp;
+template <class F>
+__device__ __forceinline__ P3ok onto_interface(const F& f, int a, int b, P3 p, float rad) {
     PsiCell pc;
     psi_cell_init(pc);
     return onto_interface_at(f, a, b, p, rad, pc);
 }
 
-// v2m_project2 (gm == 0), src/opencl/v2m_seed_body.cl:342-420 (ok = 0: p unchanged)
-__device__ __noinline__ P3ok onto_junction(const Field* fp, int a, int b, int c, P3 p, float rad) {
-    const Field f = *fp;
-    P3ok fail;
-    fail.p = p;
-    fail.ok = 0;
+// v2m_project2, src/opencl/v2m_seed_body.cl:342-420 (ok = 0: p unchanged)
+template <class F>
+__device__ __forceinline__ P3ok onto_junction_at(const F& f, int a, int b, int c, P3 p, float rad) {
+    P3ok r;
+    r.p = p;
+    r.ok = 0;
     P3 q = p;
     PsiCell pab, pac;   // the a|b and a|c cells: each projection ends where its cache points
     psi_cell_init(pab);
     psi_cell_init(pac);
-    if (f.gm < 0) {
-        // shape fields: of the three pairs' constraints, the two with the most
-        // independent gradients, their shared label first (src/opencl/v2m_seed_body.cl:345-375)
-        const float4 gab = shape_psi(fp, a, b, q, 1), gac = shape_psi(fp, a, c, q, 1), gbc = shape_psi(fp, b, c, q, 1);
-        const float xa[3] = { gab.y * gac.z - gab.z * gac.y, gab.z * gac.x - gab.x * gac.z, gab.x * gac.y - gab.y * gac.x };
-        const float xb[3] = { gab.y * gbc.z - gab.z * gbc.y, gab.z * gbc.x - gab.x * gbc.z, gab.x * gbc.y - gab.y * gbc.x };
-        const float xc[3] = { gac.y * gbc.z - gac.z * gbc.y, gac.z * gbc.x - gac.x * gbc.z, gac.x * gbc.y - gac.y * gbc.x };
-        const float na = xa[0] * xa[0] + xa[1] * xa[1] + xa[2] * xa[2], nb = xb[0] * xb[0] + xb[1] * xb[1] + xb[2] * xb[2],
-                    nc = xc[0] * xc[0] + xc[1] * xc[1] + xc[2] * xc[2];
-        if (nb > na && nb >= nc) {   // pivot b
-            const int t = a;
-            a = b;
-            b = t;
-        } else if (nc > na && nc > nb) {   // pivot c
-            const int t = a;
-            a = c;
-            c = b;
-            b = t;
+    if constexpr (!F::kPlain) {
+        if (f.gm < 0) {
+            // shape fields: of the three pairs' constraints, the two with the most
+            // independent gradients, their shared label first (src/opencl/v2m_seed_body.cl:345-375)
+            const float4 gab = shape_psi(f.self, a, b, q, 1), gac = shape_psi(f.self, a, c, q, 1),
+                         gbc = shape_psi(f.self, b, c, q, 1);
+            const float xa[3] = { gab.y * gac.z - gab.z * gac.y, gab.z * gac.x - gab.x * gac.z, gab.x * gac.y - gab.y * gac.x };
+            const float xb[3] = { gab.y * gbc.z - gab.z * gbc.y, gab.z * gbc.x - gab.x * gbc.z, gab.x * gbc.y - gab.y * gbc.x };
+            const float xc[3] = { gac.y * gbc.z - gac.z * gbc.y, gac.z * gbc.x - gac.x * gbc.z, gac.x * gbc.y - gac.y * gbc.x };
+            const float na = xa[0] * xa[0] + xa[1] * xa[1] + xa[2] * xa[2], nb = xb[0] * xb[0] + xb[1] * xb[1] + xb[2] * xb[2],
+                        nc = xc[0] * xc[0] + xc[1] * xc[1] + xc[2] * xc[2];
+            if (nb > na && nb >= nc) {   // pivot b
+                const int t = a;
+                a = b;
+                b = t;
+            } else if (nc > na && nc > nb) {   // pivot c
+                const int t = a;
+                a = c;
+                c = b;
+                b = t;
+            }
         }
     }
-    for (int it = 0; it < 3; ++it) {
+    // three rounds onto a|b, then along the curve's normal plane onto a|c; a last a|b
+#pragma clang loop unroll(disable)
+    for (int it = 0;; ++it) {
         const P3ok r1 = onto_interface_at(f, a, b, q, rad, pab);
         if (!r1.ok) {
-            return fail;
+            return r;
         }
         q = r1.p;
+        if (it == 3) {
+            break;
+        }
         const float4 g1 = psi_grad_at(f, a, b, q, pab);
         const float4 g2 = psi_grad_at(f, a, c, q, pac);
         const float v2 = g2.w;
         const float a11 = g1.x * g1.x + g1.y * g1.y + g1.z * g1.z;
         if (a11 < 1e-18f) {
-            return fail;
+            return r;
         }
         const float pr = (g1.x * g2.x + g1.y * g2.y + g1.z * g2.z) / a11;
         P3 u = p3(g2.x - pr * g1.x, g2.y - pr * g1.y, g2.z - pr * g1.z);
         const float un = sqrtf(u.x * u.x + u.y * u.y + u.z * u.z);
         if (un < 1e-9f) {
-            return fail;
+            return r;
         }
         u.x /= un;
         u.y /= un;
         u.z /= un;
         const P3ok r2 = bracket_along(f, a, c, q, u, v2, rad, 1.5f * fabsf(v2) / un, pac);
         if (!r2.ok) {
-            return fail;
+            return r;
         }
         q = r2.p;
     }
-    const P3ok r3 = onto_interface_at(f, a, b, q, rad, pab);
-    if (!r3.ok) {
-        return fail;
-    }
-    q = r3.p;
     const float m2 = (q.x - p.x) * (q.x - p.x) + (q.y - p.y) * (q.y - p.y) + (q.z - p.z) * (q.z - p.z);
     if (m2 > rad * rad) {
-        return fail;
+        return r;
     }
-    P3ok r;
     r.p = q;
     r.ok = 1;
     return r;
+}
+
+__device__ __noinline__ P3ok onto_junction_call(const Field* fp, int a, int b, int c, P3 p, float rad) {
+    const Field f = *fp;
+    return onto_junction_at(f, a, b, c, p, rad);
+}
+
+template <class F>
+__device__ __forceinline__ P3ok onto_junction(const F& f, int a, int b, int c, P3 p, float rad) {
+    if constexpr (F::kPlain) {
+        return onto_junction_at(f, a, b, c, p, rad);
+    } else {
+        return onto_junction_call(f.self, a, b, c, p, rad);
+    }
 }
 
 // ---- hash ------------------------------------------------------------------------------
@@ -1239,14 +1281,20 @@ __device__ __forceinline__ float4 bar_force(const float4* __restrict__ X, const 
 // ---- the trapped move --------------------------------------------------------------------
 
 // v2m_crossing, src/opencl/v2m_particle_body.cl:188-212
-__device__ __forceinline__ P3 segment_crossing_at(const Field& f, int a, int b, P3 p, P3 q, PsiCell& pc) {
+template <class F>
+__device__ __forceinline__ P3 segment_crossing_at(const F& f, int a, int b, P3 p, P3 q, PsiCell& pc) {
     float t0 = 0.0f, t1 = 1.0f;
-    float v0 = psi_at(f, a, b, p, pc);
-    float v1 = psi_at(f, a, b, q, pc);
-    for (int it = 0; it < 6; ++it) {
+    float v0 = 0.0f, v1 = 0.0f;
+    // the two ends, then six halvings, at one place of the code
+#pragma clang loop unroll(disable)
+    for (int it = -2; it < 6; ++it) {
         const float tm = 0.5f * (t0 + t1);
-        const float vm = psi_at(f, a, b, p3(p.x + tm * (q.x - p.x), p.y + tm * (q.y - p.y), p.z + tm * (q.z - p.z)), pc);
-        if (vm > 0.0f) {
+        const P3 x = it == -2 ? p : (it == -1 ? q : p3(p.x + tm * (q.x - p.x), p.y + tm * (q.y - p.y), p.z + tm * (q.z - p.z)));
+        const float vm = psi_at(f, a, b, x, pc);
+        if (it < 0) {
+            v0 = it == -2 ? vm : v0;
+            v1 = vm;
+        } else if (vm > 0.0f) {
             t0 = tm;
             v0 = vm;
         } else {
@@ -1259,7 +1307,8 @@ __device__ __forceinline__ P3 segment_crossing_at(const Field& f, int a, int b, 
 }
 
 // v2m_tangential, src/opencl/v2m_particle_body.cl:215-229: v less its part along n_ab at p
-__device__ __forceinline__ P3 drop_normal_at(const Field& f, int a, int b, P3 p, P3 v, PsiCell& pc) {
+template <class F>
+__device__ __forceinline__ P3 drop_normal_at(const F& f, int a, int b, P3 p, P3 v, PsiCell& pc) {
     const float4 g = psi_grad_at(f, a, b, p, pc);
     const float gn2 = g.x * g.x + g.y * g.y + g.z * g.z;
     if (gn2 < 1e-12f) {
@@ -1269,68 +1318,90 @@ __device__ __forceinline__ P3 drop_normal_at(const Field& f, int a, int b, P3 p,
     return p3(v.x - vn * g.x, v.y - vn * g.y, v.z - vn * g.z);
 }
 
-// v2m_third_label, src/opencl/v2m_particle_body.cl:232-260. The brick test runs
-// inline; the field comparisons (a third label is near: rare) are a call.
-__device__ __noinline__ int competing_label_near(const Field* fp, int a, int b, P3 q, BrickLabels bl) {
-    const Field f = *fp;
-    const float pa = phi_point(f, a, q);
-    int c = kNoLab;
-    float pc = 0.5f * pa;
-    const PointCell cell = point_cell(f, q, bl);
+// The other labels at q (of the labels of its brick): whether one competes with a|b
+// (v2m_third_label, src/opencl/v2m_particle_body.cl:232-260: the strongest above half of
+// phi_a), and whether one dominates a, b and c (v2m_valid_on fails, :266-291: above the
+// weakest of theirs by 0.02; c = kNoLab or -1: of a and b; with kNoLab a label of that
+// number competes but does not dominate, as in the reference).
+struct OtherLabels {
+    int third;       // the competing label, or kNoLab
+    int dominated;
+};
+
+__device__ __forceinline__ bool others_near(const BrickLabels& bl, int a, int b, int c) {
+    int other = 0;
     for (int s = 0; s < bl.n; ++s) {
-        const int l = brick_label(f, bl, s);
-        if (l != a && l != b) {
-            const float w = f.gm < 0 ? phi_point(f, l, q) : label_phi(f, cell, s, l);
-            if (w > pc) {
-                pc = w;
-                c = l;
+        const int l = bl.b < 0 ? 0 : list_label(bl.list, s);
+        other |= l != a && l != b && (l != c || c == kNoLab);
+    }
+    return other != 0;
+}
+
+template <class F>
+__device__ __forceinline__ OtherLabels weigh_others(const F& f, int a, int b, int c, P3 q, const BrickLabels& bl) {
+    OtherLabels r;
+    r.third = kNoLab;
+    r.dominated = 0;
+    float pa, mine, top;
+    auto weigh = [&](int l, float w) {
+        if (w > top) {
+            top = w;
+            r.third = l;
+        }
+        r.dominated |= l != c && w > mine + 0.02f;
+    };
+    if constexpr (F::kPlain) {
+        const ApronCell cell = apron_point(f, q, bl);
+        pa = apron_phi(f, cell, -1, a);
+        mine = fminf(pa, apron_phi(f, cell, -1, b));
+        if (c != kNoLab && c >= 0) {
+            mine = fminf(mine, apron_phi(f, cell, -1, c));
+        }
+        top = 0.5f * pa;
+        for (int s = 0; s < bl.n; ++s) {
+            const int l = bl.b < 0 ? 0 : list_label(bl.list, s);
+            if (l != a && l != b && (l != c || c == kNoLab)) {
+                weigh(l, apron_phi(f, cell, s, l));
+            }
+        }
+    } else {
+        pa = phi_point(f, a, q);
+        mine = fminf(pa, phi_point(f, b, q));
+        if (c != kNoLab && c >= 0) {
+            mine = fminf(mine, phi_point(f, c, q));
+        }
+        top = 0.5f * pa;
+        const PointCell cell = point_cell(f, q, bl);
+        for (int s = 0; s < bl.n; ++s) {
+            const int l = brick_label(f, bl, s);
+            if (l != a && l != b && (l != c || c == kNoLab)) {
+                weigh(l, f.gm < 0 ? phi_point(f, l, q) : label_phi(f, cell, s, l));
             }
         }
     }
-    return c;
+    return r;
 }
 
-__device__ __forceinline__ int competing_label(const Field& f, int a, int b, P3 q) {
-    const BrickLabels bl = brick_labels_at(f, q);
-    int other = 0;
-    for (int s = 0; s < bl.n; ++s) {
-        const int l = brick_label(f, bl, s);
-        other |= l != a && l != b;
-    }
-    if (!other) {
-        return kNoLab;
-    }
-    return competing_label_near(f.self, a, b, q, bl);
-}
-
-// v2m_valid_on, src/opencl/v2m_particle_body.cl:266-291 (the same split)
-__device__ __noinline__ int labels_dominate_near(const Field* fp, int a, int b, int c, P3 q, BrickLabels bl) {
+__device__ __noinline__ OtherLabels weigh_others_call(const Field* fp, int a, int b, int c, P3 q, BrickLabels bl) {
     const Field f = *fp;
-    float mine = fminf(phi_point(f, a, q), phi_point(f, b, q));
-    if (c != kNoLab) {
-        mine = fminf(mine, phi_point(f, c, q));
-    }
-    const PointCell cell = point_cell(f, q, bl);
-    for (int s = 0; s < bl.n; ++s) {
-        const int l = brick_label(f, bl, s);
-        if (l != a && l != b && l != c && (f.gm < 0 ? phi_point(f, l, q) : label_phi(f, cell, s, l)) > mine + 0.02f) {
-            return 0;
+    return weigh_others(f, a, b, c, q, bl);
+}
+
+// kInline: no out-of-line call (whose register budget would bound a lean kernel)
+template <bool kInline, class F>
+__device__ __forceinline__ OtherLabels other_labels(const F& f, int a, int b, int c, P3 q) {
+    const BrickLabels bl = brick_labels_at(f, q);
+    OtherLabels r;
+    r.third = kNoLab;
+    r.dominated = 0;
+    if (others_near(bl, a, b, c)) {
+        if constexpr (F::kPlain || kInline) {
+            r = weigh_others(f, a, b, c, q, bl);
+        } else {
+            r = weigh_others_call(f.self, a, b, c, q, bl);
         }
     }
-    return 1;
-}
-
-__device__ __forceinline__ int labels_dominate(const Field& f, int a, int b, int c, P3 q) {
-    const BrickLabels bl = brick_labels_at(f, q);
-    int other = 0;
-    for (int s = 0; s < bl.n; ++s) {
-        const int l = brick_label(f, bl, s);
-        other |= l != a && l != b && l != c;
-    }
-    if (!other) {
-        return 1;
-    }
-    return labels_dominate_near(f.self, a, b, c, q, bl);
+    return r;
 }
 
 constexpr float kDeferred = -1.0f;   // trapped_step<true>: the node needs the general path
@@ -1347,67 +1418,14 @@ struct NodeState {
     int b, c;       // partners as stored: part[2i], part[2i+1]
 };
 
-// v2m_move_step (smooth mode), src/opencl/v2m_particle_body.cl:659-833: apply the
-// capped step s with interface trapping. Returns |dp| / h (0: the node stayed;
-// its type and partners may still have changed, as in the reference).
-// The general tail below for an interior or interface node, without its out-of-line
-// calls: one pass over the labels of q's brick evaluates both v2m_third_label
-// (competing_label_near) and v2m_valid_on (labels_dominate_near) at q, with the same
-// values. A third label found (the node would try to join a junction) returns
-// kDeferred. Otherwise the step fails if it is too long or another label dominates
-// at q (the second third-label search then finds none either: same labels, same
-// point), and ends as the general tail ends if not.
-__device__ __forceinline__ float lean_tail(const Field& f, float h, float maxstep, float snap, int a, int typ0,
-                                           int ty, int b, P3 p, P3 q, NodeState& ns) {
-    bool dominated = false;
-    if (ty == TN_INTERFACE) {
-        const BrickLabels bl = brick_labels_at(f, q);
-        int other = 0;
-        for (int s = 0; s < bl.n; ++s) {
-            const int l = brick_label(f, bl, s);
-            other |= l != a && l != b;
-        }
-        if (other) {
-            const PointCell cell = point_cell(f, q, bl);
-            const float pa = phi_point(f, a, q), pb = phi_point(f, b, q);
-            const float mine = fminf(pa, pb);
-            float pc = 0.5f * pa;
-            int cc = kNoLab;
-            for (int s = 0; s < bl.n; ++s) {
-                const int l = brick_label(f, bl, s);
-                if (l != a && l != b) {
-                    const float w = f.gm < 0 ? phi_point(f, l, q) : label_phi(f, cell, s, l);
-                    if (w > pc) {
-                        pc = w;
-                        cc = l;
-                    }
-                    dominated = dominated || w > mine + 0.02f;
-                }
-            }
-            if (cc != kNoLab) {
-                return kDeferred;
-            }
-        }
-    }
-    const float lim = (maxstep + fmaxf(snap, 0.5f)) * h;
-    const float m2 = dist2(q, p);
-    if (!(m2 <= lim * lim)) {
-        if (typ0 == TN_INTERIOR) {
-            ns.b = kNoLab;
-        }
-        return 0.0f;
-    }
-    if (ty != TN_INTERIOR && dominated) {
-        ns.ty = typ0 == TN_INTERIOR ? TN_INTERIOR : ty;
-        if (ns.ty == TN_INTERIOR) {
-            ns.b = kNoLab;
-        }
-        return 0.0f;
-    }
+// The end of v2m_move_step for a step that lands: the new state and |dp| / h
+template <class F>
+__device__ __forceinline__ float land(const F& f, float h, P3 p, P3 q, int ty, NodeState& ns) {
+    const float mv = sqrtf(dist2(q, p));
     ns.p = q;
     ns.ty = ty;
     ns.hn = size_at(f, q.x, q.y, q.z);
-    return sqrtf(m2) / h;
+    return mv / h;
 }
 
 // Step modes: the general path, or a lean one for nodes known to be interface
@@ -1417,8 +1435,18 @@ __device__ __forceinline__ float lean_tail(const Field& f, float h, float maxste
 // untouched; the caller hands such a node to the general path.
 constexpr int kGeneral = 0, kLeanInterface = 1, kLeanInterior = 2;
 
-template <int kMode>
-__device__ __forceinline__ float trapped_step(const Field& f, float h, P3 s, float maxstep, float snap, int a,
+// v2m_move_step (smooth mode), src/opencl/v2m_particle_body.cl:659-833: apply the
+// capped step s with interface trapping. Returns |dp| / h (0: the node stayed;
+// its type and partners may still have changed, as in the reference).
+//
+// The reference searches for a third label, joins a junction and tests its labels at up
+// to two places each. Here the junction projection, by far the longest part, stands at
+// one place in a loop of at most two rounds: an interface node that found no junction to
+// join (or could not be projected onto it) and is dominated would only repeat the search
+// at the same point with the same result, so the second round is left to an interior
+// node that joined a junction whose labels are dominated there.
+template <int kMode, class F>
+__device__ __forceinline__ float trapped_step(const F& f, float h, P3 s, float maxstep, float snap, int a,
                                               NodeState& ns) {
     const P3 p = ns.p;
     P3 q;
@@ -1428,121 +1456,160 @@ __device__ __forceinline__ float trapped_step(const Field& f, float h, P3 s, flo
     int b = ns.b;             // the locals b, c of the reference; ns.b / ns.c are the stored part[]
     const int c = ns.c;
 
-    if (kMode != kLeanInterface && ty == TN_INTERIOR) {
-        q = p3(p.x + s.x, p.y + s.y, p.z + s.z);
-        const int2 own = owner_at(f, q);
-        const int l = own.x, sec = own.y;
-        if (l != a) {
-            b = l;
-            PsiCell pc;   // crossing, glide and projection stay near the crossing point
-            psi_cell_init(pc);
-            const P3 x = segment_crossing_at(f, a, b, p, q, pc);
-            const P3 r = drop_normal_at(f, a, b, x, p3(q.x - x.x, q.y - x.y, q.z - x.z), pc);
-            q = p3(x.x + r.x, x.y + r.y, x.z + r.z);
-            const P3ok pr = onto_interface_at(f, a, b, q, 0.5f * h, pc);
-            q = pr.ok ? pr.p : x;
-            ty = TN_INTERFACE;
-            ns.b = b;
-        } else if (sec != kNoLab && snap > 0.0f) {
-            PsiCell pc;
-            psi_cell_init(pc);
-            const float4 gq = psi_grad_at(f, a, sec, q, pc);
-            const float v = gq.w;
-            const float gn = sqrtf(gq.x * gq.x + gq.y * gq.y + gq.z * gq.z);
-            if (gn > 1e-9f && v / gn < snap * h) {
-                const P3ok pr = onto_interface_at(f, a, sec, q, 1.2f * snap * h, pc);
-                if (pr.ok) {
-                    q = pr.p;
-                    ty = TN_INTERFACE;
-                    b = sec;
-                    ns.b = sec;
+    if (kMode != kGeneral || ty <= TN_INTERFACE) {
+        PsiCell pc;   // crossing, glide and projection probe the same few cells
+        psi_cell_init(pc);
+        // where the interface projection starts, its reach and its pair (project: to be done)
+        bool project = true;
+        P3 x = p, r = s;
+        float rad = 0.5f * h;
+        if (kMode != kLeanInterface && ty == TN_INTERIOR) {
+            q = p3(p.x + s.x, p.y + s.y, p.z + s.z);
+            const int2 own = owner_at(f, q);
+            const int l = own.x, sec = own.y;
+            if (l != a) {   // across the interface: glide from the crossing
+                b = l;
+                x = segment_crossing_at(f, a, b, p, q, pc);
+                r = p3(q.x - x.x, q.y - x.y, q.z - x.z);
+                ns.b = b;
+            } else {
+                project = false;
+                if (sec != kNoLab && snap > 0.0f) {
+                    const float4 gq = psi_grad_at(f, a, sec, q, pc);
+                    const float gn = sqrtf(gq.x * gq.x + gq.y * gq.y + gq.z * gq.z);
+                    if (gn > 1e-9f && gq.w / gn < snap * h) {   // close to it: snap
+                        b = sec;
+                        rad = 1.2f * snap * h;
+                        project = true;
+                        ty = TN_JUNCTION;   // (marks the snap until the projection is done)
+                    }
                 }
             }
         }
-    } else if (kMode == kLeanInterface || ty == TN_INTERFACE) {
-        PsiCell pc;   // the glide and its projection probe the same few cells
-        psi_cell_init(pc);
-        s = drop_normal_at(f, a, b, p, s, pc);
-        q = p3(p.x + s.x, p.y + s.y, p.z + s.z);
-        const P3ok pr = onto_interface_at(f, a, b, q, 0.5f * h, pc);
-        if (!pr.ok) {
-            return 0.0f;
+        if (project) {
+            const bool snapped = kMode != kLeanInterface && ty == TN_JUNCTION;
+            if (!snapped) {
+                r = drop_normal_at(f, a, b, x, r, pc);
+                q = p3(x.x + r.x, x.y + r.y, x.z + r.z);
+            }
+            const P3ok pr = onto_interface_at(f, a, b, q, rad, pc);
+            if (kMode == kLeanInterface || typ0 == TN_INTERFACE) {
+                if (!pr.ok) {
+                    return 0.0f;
+                }
+                q = pr.p;
+            } else if (snapped) {
+                ty = TN_INTERIOR;
+                if (pr.ok) {
+                    q = pr.p;
+                    ty = TN_INTERFACE;
+                    ns.b = b;
+                } else {
+                    b = ns.b;
+                }
+            } else {
+                q = pr.ok ? pr.p : x;
+                ty = TN_INTERFACE;
+            }
         }
-        q = pr.p;
     } else {
-        const float4 g1 = psi_grad_point(f.self, a, b, p);
-        const float4 g2 = psi_grad_point(f.self, a, c, p);
+        const float4 g1 = psi_grad_once(f, a, b, p);
+        const float4 g2 = psi_grad_once(f, a, c, p);
         const float t0 = g1.y * g2.z - g1.z * g2.y;
         const float t1 = g1.z * g2.x - g1.x * g2.z;
         const float t2 = g1.x * g2.y - g1.y * g2.x;
         const float tl2 = t0 * t0 + t1 * t1 + t2 * t2;
         const float st = tl2 > 1e-20f ? (s.x * t0 + s.y * t1 + s.z * t2) / tl2 : 0.0f;
         q = p3(p.x + st * t0, p.y + st * t1, p.z + st * t2);
-        const P3ok pr = onto_junction(f.self, a, b, c, q, 0.5f * h);
-        if (!pr.ok) {
-            return 0.0f;
-        }
-        q = pr.p;
     }
 
+    OtherLabels near;   // at q, of the node's labels there
+    near.third = kNoLab;
+    near.dominated = 0;
     if (kMode != kGeneral) {
-        return lean_tail(f, h, maxstep, snap, a, typ0, ty, b, p, q, ns);
-    }
-
-    if (ty == TN_INTERFACE) {
-        const int cc = competing_label(f, a, b, q);
-        if (cc != kNoLab) {
-            const P3ok pr = onto_junction(f.self, a, b, cc, q, 0.5f * h);
-            if (pr.ok) {
-                q = pr.p;
-                ty = TN_JUNCTION;
-                ns.c = cc;
+        if (ty == TN_INTERFACE) {
+            near = other_labels<true>(f, a, b, -1, q);
+            if (near.third != kNoLab) {
+                return kDeferred;
             }
         }
-    }
-
-    {
         const float lim = (maxstep + fmaxf(snap, 0.5f)) * h;
-        const float m2 = dist2(q, p);
-        if (!(m2 <= lim * lim)) {
+        if (!(dist2(q, p) <= lim * lim)) {
             if (typ0 == TN_INTERIOR) {
                 ns.b = kNoLab;
             }
             return 0.0f;
         }
+        if (ty != TN_INTERIOR && near.dominated) {
+            ns.ty = typ0 == TN_INTERIOR ? TN_INTERIOR : ty;
+            if (ns.ty == TN_INTERIOR) {
+                ns.b = kNoLab;
+            }
+            return 0.0f;
+        }
+        return land(f, h, p, q, ty, ns);
     }
 
-    if (ty != TN_INTERIOR && !labels_dominate(f, a, ns.b, ty >= TN_JUNCTION ? ns.c : kNoLab, q)) {
-        if (ty == TN_INTERFACE || typ0 == TN_INTERIOR) {
-            const int cc = competing_label(f, a, ns.b, q);
-            int joined = 0;
-            if (cc != kNoLab) {
-                const P3ok pr = onto_junction(f.self, a, ns.b, cc, q, 0.5f * h);
-                if (pr.ok && labels_dominate(f, a, ns.b, cc, pr.p)) {
-                    q = pr.p;
-                    joined = 1;
-                }
-            }
-            if (joined) {
+#pragma clang loop unroll(disable)
+    for (int round = 0; round < 2; ++round) {
+        int jc = c;
+        bool join = typ0 >= TN_JUNCTION;
+        if (ty == TN_INTERFACE || round) {
+            near = other_labels<false>(f, a, ns.b, kNoLab, q);
+            jc = near.third;
+            join = jc != kNoLab;
+        }
+        bool joined = false;
+        if (join) {
+            const P3ok pr = onto_junction(f, a, ns.b, jc, q, 0.5f * h);
+            joined = pr.ok != 0;
+            if (joined && !round) {
+                q = pr.p;
                 ty = TN_JUNCTION;
-                ns.c = cc;
-            } else {
-                ns.ty = typ0 == TN_INTERIOR ? TN_INTERIOR : ty;
-                if (ns.ty == TN_INTERIOR) {
-                    ns.b = kNoLab;
+                ns.c = jc;
+            } else if (joined) {
+                joined = other_labels<false>(f, a, ns.b, jc, pr.p).dominated == 0;
+                if (joined) {
+                    q = pr.p;
+                    ns.c = jc;
                 }
+            } else if (typ0 >= TN_JUNCTION) {
                 return 0.0f;
             }
-        } else {
+        }
+        if (round) {
+            if (!joined) {
+                ns.ty = TN_INTERIOR;
+                ns.b = kNoLab;
+                return 0.0f;
+            }
+            break;
+        }
+        const float lim = (maxstep + fmaxf(snap, 0.5f)) * h;
+        if (!(dist2(q, p) <= lim * lim)) {
+            if (typ0 == TN_INTERIOR) {
+                ns.b = kNoLab;
+            }
+            return 0.0f;
+        }
+        if (ty >= TN_JUNCTION) {
+            near.dominated = other_labels<false>(f, a, ns.b, ns.c, q).dominated;
+        }
+        if (ty == TN_INTERIOR || !near.dominated) {
+            break;
+        }
+        if (ty == TN_INTERFACE) {
+            ns.ty = typ0 == TN_INTERIOR ? TN_INTERIOR : ty;
+            if (ns.ty == TN_INTERIOR) {
+                ns.b = kNoLab;
+            }
+            return 0.0f;
+        }
+        if (typ0 != TN_INTERIOR) {
             return 0.0f;
         }
     }
-
-    const float mv = sqrtf(dist2(q, p));
-    ns.p = q;
-    ns.ty = ty;
-    ns.hn = size_at(f, q.x, q.y, q.z);
-    return mv / h;
+    return land(f, h, p, q, ty, ns);
 }
 
 // ---- the voxel trap: the exact staircase of the label volume ---------------------------

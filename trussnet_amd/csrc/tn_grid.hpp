@@ -1299,7 +1299,7 @@ int tn_seed_count_from_grid(const tn_grid* g, const tn_relax_params* prm, int64_
         g->seeds.reset();
         DevMem mem;
         mem.device = g->mem.device;
-        const Seeds s = seeding_core(g->f, g->grade, g->info.hmin, g->info.hmax, prm, mem);
+        const Seeds s = seeding_core(g->f, g->info.nslot, g->grade, g->info.hmin, g->info.hmax, prm, mem);
         // keep the nodes (not the seeding's work arrays) for tn_seed_from_grid
         auto c = std::make_unique<tn_grid::SeedCache>();
         c->mem.device = g->mem.device;
@@ -1337,7 +1337,7 @@ int tn_seed_from_grid(const tn_grid* g, const tn_relax_params* prm, int64_t n, f
         // (deterministic: the same nodes)
         std::unique_ptr<tn_grid::SeedCache> cached = std::move(g->seeds);
         const bool hit = cached && std::memcmp(&cached->prm, prm, sizeof *prm) == 0;
-        const Seeds s = hit ? cached->s : seeding_core(g->f, g->grade, g->info.hmin, g->info.hmax, prm, mem);
+        const Seeds s = hit ? cached->s : seeding_core(g->f, g->info.nslot, g->grade, g->info.hmin, g->info.hmax, prm, mem);
         arg_check(s.n == n, "seeding: the output holds " + std::to_string(n) + " nodes, the seeding made " +
                                 std::to_string(s.n) + " (tn_seed_count_from_grid)");
         if (s.n == 0) {
@@ -1365,7 +1365,7 @@ int tn_plan_create_from_grid(const tn_grid* g, const tn_relax_params* prm, const
         int64_t nkeys = 0;
         const tnd::Hash H = make_hash_geom(I.nx, I.ny, I.nz, vs, I.hmin, I.hmax, g->hbig, prm, &nkeys);
         // the plan keeps its own copy of the grid (device to device)
-        *out = plan_build(prm, seeds, g->mem.device, H, nkeys, [&](DevMem& mem) {
+        *out = plan_build(prm, seeds, g->mem.device, H, nkeys, I.nslot, [&](DevMem& mem) {
             const size_t nv = (size_t)I.nx * I.ny * I.nz, nb = (size_t)I.nbx * I.nby * I.nbz;
             auto dup = [&](auto* src, size_t count) {
                 using T = std::remove_const_t<std::remove_pointer_t<decltype(src)>>;

@@ -1446,14 +1446,10 @@ __device__ __forceinline__ void block_append2(bool fa, bool fb, int i, int32_t* 
     }
 }
 
-// kPlain: every grid of the launch is a label volume (gm == 0). The compiler then
-// drops the gray-scale and shape-field branches of the field queries, and the hot
-// kernels keep their register budget; other grids take the kPlain = false variants.
-template <bool kPlain>
-__device__ __forceinline__ void k_move_easy_body(Field f, MoveArgs ma, Ctl* __restrict__ ctl, int n, const float4* __restrict__ F, float4* __restrict__ X, float4* __restrict__ V, uint8_t* __restrict__ typ, uint32_t* __restrict__ part, const uint16_t* __restrict__ lab, float* __restrict__ mv, float* __restrict__ pw, int32_t* __restrict__ queue, int32_t* __restrict__ queue_int, const uint8_t* __restrict__ skip, int bid, int nblk) {
-    if (kPlain) {
-        __builtin_assume(f.gm == 0);
-    }
+// F: PlainField when every grid of the launch is a label volume with its apron slots
+// (tn_apron.hpp): the kernel then holds no other field mode; Field for the others.
+template <class F>
+__device__ __forceinline__ void k_move_easy_body(F f, MoveArgs ma, Ctl* __restrict__ ctl, int n, const float4* __restrict__ Fo, float4* __restrict__ X, float4* __restrict__ V, uint8_t* __restrict__ typ, uint32_t* __restrict__ part, const uint16_t* __restrict__ lab, float* __restrict__ mv, float* __restrict__ pw, int32_t* __restrict__ queue, int32_t* __restrict__ queue_int, const uint8_t* __restrict__ skip, int bid, int nblk) {
     const int g = bid * kBlock + threadIdx.x;
     int i = 0;
     bool surf = false, inner = false;   // the two lean queues
@@ -1463,7 +1459,7 @@ __device__ __forceinline__ void k_move_easy_body(Field f, MoveArgs ma, Ctl* __re
     const int sk = in ? skip[g] : 1;
     const int ty0 = in ? typ[g] : 0;
     const float4 x = in ? X[g] : make_float4(0.0f, 0.0f, 0.0f, 1.0f);
-    const float4 Fi = in ? F[g] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float4 Fi = in ? Fo[g] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const float4 Vi = in && ma.fire ? V[g] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const int a = in ? lab[g] : 0;
     const uint32_t pp = in ? part[g] : 0u;
@@ -1527,9 +1523,9 @@ __device__ __forceinline__ void k_move_easy_body(Field f, MoveArgs ma, Ctl* __re
     block_append2(surf, inner, i, &ctl->nmove, queue, &ctl->nmove_int, queue_int);
 }
 
-template <bool kPlain>
-__global__ __launch_bounds__(kBlock) void k_move_easy(Field f, MoveArgs ma, Ctl* __restrict__ ctl, int n, const float4* __restrict__ F, float4* __restrict__ X, float4* __restrict__ V, uint8_t* __restrict__ typ, uint32_t* __restrict__ part, const uint16_t* __restrict__ lab, float* __restrict__ mv, float* __restrict__ pw, int32_t* __restrict__ queue, int32_t* __restrict__ queue_int, const uint8_t* __restrict__ skip) {
-    k_move_easy_body<kPlain>(f, ma, ctl, n, F, X, V, typ, part, lab, mv, pw, queue, queue_int, skip, blockIdx.x,
+template <class F>
+__global__ __launch_bounds__(kBlock) void k_move_easy(F f, MoveArgs ma, Ctl* __restrict__ ctl, int n, const float4* __restrict__ Fo, float4* __restrict__ X, float4* __restrict__ V, uint8_t* __restrict__ typ, uint32_t* __restrict__ part, const uint16_t* __restrict__ lab, float* __restrict__ mv, float* __restrict__ pw, int32_t* __restrict__ queue, int32_t* __restrict__ queue_int, const uint8_t* __restrict__ skip) {
+    k_move_easy_body(f, ma, ctl, n, Fo, X, V, typ, part, lab, mv, pw, queue, queue_int, skip, blockIdx.x,
                              gridDim.x);
 }
 
@@ -1549,9 +1545,9 @@ constexpr int kLeanSpread = TN_LEAN_SPREAD;
 #endif
 
 // v2m_move for queued node i; true: handed back (a lean mode, a third label near)
-template <int kMode>
-__device__ __forceinline__ bool move_node(const Field& f, const MoveArgs& ma, const Ctl* __restrict__ ctl, int i,
-                                          const float4* __restrict__ F, float4* __restrict__ X,
+template <int kMode, class F>
+__device__ __forceinline__ bool move_node(const F& f, const MoveArgs& ma, const Ctl* __restrict__ ctl, int i,
+                                          const float4* __restrict__ Fo, float4* __restrict__ X,
                                           float4* __restrict__ V, uint8_t* __restrict__ typ,
                                           uint32_t* __restrict__ part, const uint16_t* __restrict__ lab,
                                           float* __restrict__ mv, float* __restrict__ pw) {
@@ -1566,7 +1562,7 @@ __device__ __forceinline__ bool move_node(const Field& f, const MoveArgs& ma, co
     ns.b = (int)(pp & 0xFFFF);
     ns.c = (int)(pp >> 16);
     float m = 0.0f;
-    const NodeStep st = node_step(ma, ctl, F[i], V, i, h);   // queued nodes are never corners
+    const NodeStep st = node_step(ma, ctl, Fo[i], V, i, h);   // queued nodes are never corners
     if (st.moves) {
         m = trapped_step<kMode>(f, h, p3(st.s[0], st.s[1], st.s[2]), ma.maxstep, ma.snap, lab[i], ns);
         if (kMode != kGeneral && m == kDeferred) {
@@ -1677,11 +1673,8 @@ __global__ __launch_bounds__(kBlock) void k_move_voxel_wave(Field f, MoveArgs ma
 // whole trapped step (junction nodes and the handed-back ones). Each node's move
 // reads and writes only that node's state, so the passes over disjoint queues may
 // run concurrently.
-template <int kMode, bool kPlain>
-__device__ __forceinline__ void k_move_body(Field f, MoveArgs ma, Ctl* __restrict__ ctl, const int32_t* __restrict__ queue, const float4* __restrict__ F, float4* __restrict__ X, float4* __restrict__ V, uint8_t* __restrict__ typ, uint32_t* __restrict__ part, const uint16_t* __restrict__ lab, float* __restrict__ mv, float* __restrict__ pw, const int32_t* __restrict__ qcount, int32_t* __restrict__ defer_count, int32_t* __restrict__ defer_queue, uint8_t* __restrict__ sticky, int bid, int nblk) {
-    if (kPlain) {
-        __builtin_assume(f.gm == 0);
-    }
+template <int kMode, class F>
+__device__ __forceinline__ void k_move_body(F f, MoveArgs ma, Ctl* __restrict__ ctl, const int32_t* __restrict__ queue, const float4* __restrict__ Fo, float4* __restrict__ X, float4* __restrict__ V, uint8_t* __restrict__ typ, uint32_t* __restrict__ part, const uint16_t* __restrict__ lab, float* __restrict__ mv, float* __restrict__ pw, const int32_t* __restrict__ qcount, int32_t* __restrict__ defer_count, int32_t* __restrict__ defer_queue, uint8_t* __restrict__ sticky, int bid, int nblk) {
     // A fixed grid strides over the queue, whose length only the device knows. A
     // short queue's nodes follow long, divergent paths (projections onto interfaces
     // and junction curves), and a wave executes every path its lanes take, so they
@@ -1709,7 +1702,7 @@ __device__ __forceinline__ void k_move_body(Field f, MoveArgs ma, Ctl* __restric
         int i = 0;
         if (slot >= 0 && g < count) {
             i = queue[g];
-            defer = move_node<kMode>(f, ma, ctl, i, F, X, V, typ, part, lab, mv, pw);
+            defer = move_node<kMode>(f, ma, ctl, i, Fo, X, V, typ, part, lab, mv, pw);
         }
         if (kLean) {   // every lane of the wave is here
             wave_append(defer, i, defer_count, defer_queue);
@@ -1720,9 +1713,9 @@ __device__ __forceinline__ void k_move_body(Field f, MoveArgs ma, Ctl* __restric
     }
 }
 
-template <int kMode, bool kPlain>
-__global__ __launch_bounds__(kBlock, TN_MOVE_WAVES) void k_move(Field f, MoveArgs ma, Ctl* __restrict__ ctl, const int32_t* __restrict__ queue, const float4* __restrict__ F, float4* __restrict__ X, float4* __restrict__ V, uint8_t* __restrict__ typ, uint32_t* __restrict__ part, const uint16_t* __restrict__ lab, float* __restrict__ mv, float* __restrict__ pw, const int32_t* __restrict__ qcount, int32_t* __restrict__ defer_count, int32_t* __restrict__ defer_queue, uint8_t* __restrict__ sticky) {
-    k_move_body<kMode, kPlain>(f, ma, ctl, queue, F, X, V, typ, part, lab, mv, pw, qcount, defer_count, defer_queue,
+template <int kMode, class F>
+__global__ __launch_bounds__(kBlock, TN_MOVE_WAVES) void k_move(F f, MoveArgs ma, Ctl* __restrict__ ctl, const int32_t* __restrict__ queue, const float4* __restrict__ Fo, float4* __restrict__ X, float4* __restrict__ V, uint8_t* __restrict__ typ, uint32_t* __restrict__ part, const uint16_t* __restrict__ lab, float* __restrict__ mv, float* __restrict__ pw, const int32_t* __restrict__ qcount, int32_t* __restrict__ defer_count, int32_t* __restrict__ defer_queue, uint8_t* __restrict__ sticky) {
+    k_move_body<kMode>(f, ma, ctl, queue, Fo, X, V, typ, part, lab, mv, pw, qcount, defer_count, defer_queue,
                                sticky, blockIdx.x, gridDim.x);
 }
 
@@ -1857,7 +1850,8 @@ __global__ __launch_bounds__(kBlock) void k_stats(const float4* __restrict__ X, 
 
 // phi_a (v2m_phi_f), psi_ab and its gradient (v2m_psi_grad), the owner and the
 // runner-up (v2m_label_of) at X[3k..3k+2]; any output may be null.
-__global__ __launch_bounds__(kBlock) void k_field_points(Field f, int a, int b, int m, const float* __restrict__ X,
+template <class F>
+__global__ __launch_bounds__(kBlock) void k_field_points(F f, int a, int b, int m, const float* __restrict__ X,
                                                          float* __restrict__ phi, float* __restrict__ psi,
                                                          float* __restrict__ grad, int32_t* __restrict__ label,
                                                          int32_t* __restrict__ second) {
@@ -1870,7 +1864,7 @@ __global__ __launch_bounds__(kBlock) void k_field_points(Field f, int a, int b, 
         phi[k] = phi_point(f, a, p);
     }
     if (psi || grad) {
-        const float4 g = psi_grad_point(f.self, a, b, p);
+        const float4 g = psi_grad_once(f, a, b, p);
         if (psi) {
             psi[k] = g.w;
         }
@@ -2079,7 +2073,7 @@ __global__ __launch_bounds__(kBlock) void kg_force(const PlanIter* __restrict__ 
                  P.sticky, bid_, nb_);
 }
 
-template <bool kPlain>
+template <class F>
 __global__ __launch_bounds__(kBlock) void kg_move_easy(const PlanIter* __restrict__ tab,
                                                        const int32_t* __restrict__ bplan,
                                                        const int32_t* __restrict__ bfirst) {
@@ -2089,13 +2083,13 @@ __global__ __launch_bounds__(kBlock) void kg_move_easy(const PlanIter* __restric
                           bid_);
         return;
     }
-    k_move_easy_body<kPlain>(P.f, P.ma, P.ctl, P.n, P.F, P.X, P.V, P.typ, P.part, P.lab, P.mv, P.pw, P.mq, P.mqi, P.flag,
+    k_move_easy_body(as_field<F>(P.f), P.ma, P.ctl, P.n, P.F, P.X, P.V, P.typ, P.part, P.lab, P.mv, P.pw, P.mq, P.mqi, P.flag,
                              bid_, nb_);
 }
 
 // the four move passes: kQueue 0 = the general queue, 1 = interior (lean), 2 =
 // interface (lean), 3 = the handed-back nodes (general)
-template <int kQueue, bool kPlain>
+template <int kQueue, class F>
 __global__ __launch_bounds__(kBlock, TN_MOVE_WAVES) void kg_move(const PlanIter* __restrict__ tab,
                                                                  const int32_t* __restrict__ bplan,
                                                                  const int32_t* __restrict__ bfirst) {
@@ -2113,7 +2107,7 @@ __global__ __launch_bounds__(kBlock, TN_MOVE_WAVES) void kg_move(const PlanIter*
                                        : (kQueue == 1 ? &P.ctl->nmove_int
                                                       : (kQueue == 2 ? &P.ctl->nmove : &P.ctl->nmove_def));
     const bool lean = kMode != kGeneral;
-    k_move_body<kMode, kPlain>(P.f, P.ma, P.ctl, queue, P.F, P.X, P.V, P.typ, P.part, P.lab, P.mv, P.pw, count,
+    k_move_body<kMode>(as_field<F>(P.f), P.ma, P.ctl, queue, P.F, P.X, P.V, P.typ, P.part, P.lab, P.mv, P.pw, count,
                        lean ? &P.ctl->nmove_def : nullptr, lean ? P.mqd : nullptr, lean ? P.sticky : nullptr, bid_,
                        nb_);
 }

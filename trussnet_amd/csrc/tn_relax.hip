@@ -267,6 +267,15 @@ struct DevMem {
         chunk_left -= bytes;
         return p;
     }
+    // raw() for a buffer that its caller can do without: null where there is no room
+    void* spare(size_t bytes) {
+        try {
+            return raw(bytes);
+        } catch (const TnError&) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
     template <class T>
     T* alloc(size_t count) {
         return static_cast<T*>(raw(count * sizeof(T)));
@@ -316,12 +325,42 @@ tnd::Field upload_grid(const tn_grid_view* g, DevMem& mem) {
     f.phi = mem.upload(g->phi, (size_t)g->nslot * TN_SLOT);
     f.h = mem.upload(g->h, nv);
     f.gm = g->gm;
+    f.ap = nullptr;
+    f.rec = nullptr;
     f.gI = f.gm > 0 ? mem.upload(g->gI, nv) : nullptr;
     f.gTW = f.gm > 0 ? mem.upload(g->gTW, 2 * (size_t)f.gm) : (f.gm < 0 ? mem.upload(g->gTW, (size_t)g->ngTW) : nullptr);
     tnd::Field* self = mem.alloc<tnd::Field>(1);
     f.self = self;
     TN_HIP(hipMemcpy(self, &f, sizeof f, hipMemcpyHostToDevice));
     return f;
+}
+
+// The apron slots and brick records of a label volume's grid (tn_apron.hpp), put into mem
+// and f (f.self's copy too, on the stream s). Nothing for the other field modes, nor where
+// mem has no room for them: the kernels over the stored layout then run.
+// own_self: f.self is this Field's alone.
+void add_apron(tnd::Field& f, int64_t nslot, DevMem& mem, hipStream_t s, bool own_self) {
+    f.ap = nullptr;
+    f.rec = nullptr;
+    if (f.gm != 0) {
+        return;
+    }
+    const int64_t nb = (int64_t)f.nbx * f.nby * f.nbz;
+    const size_t slots = (size_t)std::max<int64_t>(nslot, 1) * tnd::kApSlot * sizeof(float);
+    float* ap = static_cast<float*>(mem.spare(slots));
+    uint4* rec = ap ? static_cast<uint4*>(mem.spare((size_t)nb * 4 * sizeof(uint4))) : nullptr;
+    if (!rec) {
+        return;
+    }
+    tnd::k_brick_rec<<<blocks_for(nb, 256), 256, 0, s>>>(f.bl_cnt, f.bl_lab, f.bl_slot, (int)nb, rec);
+    tnd::k_apron<<<(unsigned)nb, 256, 0, s>>>(f, ap);
+    TN_HIP(hipGetLastError());
+    f.ap = ap;
+    f.rec = rec;
+    if (own_self) {
+        TN_HIP(hipMemcpyAsync(const_cast<tnd::Field*>(f.self), &f, sizeof f, hipMemcpyHostToDevice, s));
+        TN_HIP(hipStreamSynchronize(s));
+    }
 }
 
 // Kernel classes of the per-kernel device timings.
@@ -637,9 +676,9 @@ struct tn_plan {
             enqueue_iteration_tail(nb);
             return;
         }
-        // (label volumes: the move kernels compiled without the other field modes)
-        auto moves = [&](auto plain) {
-            constexpr bool kP = decltype(plain)::value;
+        // (label volumes: the move kernels over their apron slots, with no other field mode)
+        auto moves = [&](const auto& f) {
+            using FT = std::decay_t<decltype(f)>;
             // The queued nodes: the junction nodes' general pass starts on a side stream as
             // soon as the forces are done, beside k_move_easy; then the two lean passes at
             // once over the queues k_move_easy fills, each bounded by its slowest node, then
@@ -651,13 +690,13 @@ struct tn_plan {
                 TN_HIP(hipStreamWaitEvent(s0, ev_force, 0));
             }
             hipEvent_t tr = timer.begin(KC_MOVE_REST, s0);
-            tnk::k_move<tnd::kGeneral, kP><<<g2, tnk::kBlock, 0, s0>>>(f, ma, dCtl, dMoveQ2, dF, dX, dV, dTyp, dPart, dLab, dMv,
+            tnk::k_move<tnd::kGeneral, FT><<<g2, tnk::kBlock, 0, s0>>>(f, ma, dCtl, dMoveQ2, dF, dX, dV, dTyp, dPart, dLab, dMv,
                                                                    dPw, &dCtl->nmove_rest, nullptr, nullptr, nullptr);
             timer.end(KC_MOVE_REST, tr, s0);
             if (overlap_moves) {
                 TN_HIP(hipEventRecord(ev_rest, s0));
             }
-            tnk::k_move_easy<kP><<<nb, tnk::kBlock, 0, stream>>>(f, ma, dCtl, n, dF, dX, dV, dTyp, dPart, dLab, dMv,
+            tnk::k_move_easy<FT><<<nb, tnk::kBlock, 0, stream>>>(f, ma, dCtl, n, dF, dX, dV, dTyp, dPart, dLab, dMv,
                                                              dPw, dMoveQ, dMoveQi, dFlag);
             timer.end(KC_MOVE_EASY, t);
             if (overlap_moves) {
@@ -665,7 +704,7 @@ struct tn_plan {
                 TN_HIP(hipStreamWaitEvent(s1, ev_easy, 0));
             }
             t = timer.begin(KC_MOVE_INT, s1);
-            tnk::k_move<tnd::kLeanInterior, kP><<<g1, tnk::kBlock, 0, s1>>>(f, ma, dCtl, dMoveQi, dF, dX, dV, dTyp, dPart, dLab,
+            tnk::k_move<tnd::kLeanInterior, FT><<<g1, tnk::kBlock, 0, s1>>>(f, ma, dCtl, dMoveQi, dF, dX, dV, dTyp, dPart, dLab,
                                                                         dMv, dPw, &dCtl->nmove_int, &dCtl->nmove_def,
                                                                         dMoveQd, dSticky);
             timer.end(KC_MOVE_INT, t, s1);
@@ -673,7 +712,7 @@ struct tn_plan {
                 TN_HIP(hipEventRecord(ev_int, s1));
             }
             t = timer.begin(KC_MOVE);
-            tnk::k_move<tnd::kLeanInterface, kP><<<g1, tnk::kBlock, 0, stream>>>(f, ma, dCtl, dMoveQ, dF, dX, dV, dTyp, dPart,
+            tnk::k_move<tnd::kLeanInterface, FT><<<g1, tnk::kBlock, 0, stream>>>(f, ma, dCtl, dMoveQ, dF, dX, dV, dTyp, dPart,
                                                                              dLab, dMv, dPw, &dCtl->nmove, &dCtl->nmove_def,
                                                                              dMoveQd, dSticky);
             timer.end(KC_MOVE, t);
@@ -681,17 +720,17 @@ struct tn_plan {
                 TN_HIP(hipStreamWaitEvent(stream, ev_int, 0));
             }
             t = timer.begin(KC_MOVE_DEF);
-            tnk::k_move<tnd::kGeneral, kP><<<g2, tnk::kBlock, 0, stream>>>(f, ma, dCtl, dMoveQd, dF, dX, dV, dTyp, dPart, dLab,
+            tnk::k_move<tnd::kGeneral, FT><<<g2, tnk::kBlock, 0, stream>>>(f, ma, dCtl, dMoveQd, dF, dX, dV, dTyp, dPart, dLab,
                                                                        dMv, dPw, &dCtl->nmove_def, nullptr, nullptr, nullptr);
             timer.end(KC_MOVE_DEF, t);
             if (overlap_moves) {
                 TN_HIP(hipStreamWaitEvent(stream, ev_rest, 0));
             }
         };
-        if (f.gm == 0) {
-            moves(std::true_type{});
+        if (f.ap) {
+            moves(tnd::as_field<tnd::PlainField>(f));
         } else {
-            moves(std::false_type{});
+            moves(f);
         }
         enqueue_iteration_tail(nb);
     }
@@ -851,11 +890,11 @@ struct tn_plan {
 namespace {
 
 // A plan on device dev: make_grid(mem) puts the grid into the plan's memory and
-// returns its Field; H and nkeys are the hash geometry. With an arena, the plan
+// returns its Field; H and nkeys are the hash geometry, nslot the grid's phi slots. With an arena, the plan
 // allocates nothing (DevMem::set_arena; tn_plan::noalloc).
 template <class MakeGrid>
 tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int dev, const tnd::Hash& H, int64_t nkeys,
-                    MakeGrid make_grid, void* arena = nullptr, size_t arena_cap = 0) {
+                    int64_t nslot, MakeGrid make_grid, void* arena = nullptr, size_t arena_cap = 0) {
         TN_HIP(hipSetDevice(dev));
         std::unique_ptr<tn_plan> p(new tn_plan);
         p->device = dev;
@@ -889,7 +928,7 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
         const int n = p->n;
         p->mem.device = dev;
         p->f = make_grid(p->mem);
-        const tnd::Field& f = p->f;
+        tnd::Field& f = p->f;
         // node state
         p->dX0 = p->alloc<float4>(n);
         p->dX = p->alloc<float4>(n);
@@ -981,6 +1020,10 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
             TN_HIP(hipMemcpy(p->dPart0, part.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
             TN_HIP(hipMemcpy(p->dTyp0, seeds->typ, n, hipMemcpyHostToDevice));
             TN_HIP(hipMemcpy(p->dLab0, seeds->lab, sizeof(uint16_t) * n, hipMemcpyHostToDevice));
+        }
+        // (after every buffer that the plan cannot do without)
+        if (n > 0 && !prm->voxel_trap) {
+            add_apron(f, nslot, p->mem, p->stream, true);
         }
         p->reset();
         return p.release();
@@ -1208,7 +1251,12 @@ int64_t junction_pass(float ghmax, const tnd::Field& f, const tnk::SeedArgs& sa,
         jc.key = mem.alloc<int32_t>((size_t)7 * m3);
         jc.ok = mem.alloc<int32_t>((size_t)m3 + 1);
         tnk::k_fill_i32<<<blocks_for(m3 + 1, tnk::kBlock), tnk::kBlock>>>(jc.ok, m3 + 1, 0);
-        tnk::k_junction_cand<<<blocks_for(m3, tnk::kBlock), tnk::kBlock>>>(f, sa, cellfac, vg, list, jc);
+        if (f.ap) {
+            tnk::k_junction_cand<<<blocks_for(m3, tnk::kBlock), tnk::kBlock>>>(tnd::as_field<tnd::PlainField>(f), sa,
+                                                                               cellfac, vg, list, jc);
+        } else {
+            tnk::k_junction_cand<<<blocks_for(m3, tnk::kBlock), tnk::kBlock>>>(f, sa, cellfac, vg, list, jc);
+        }
         const int nc = ops.scan(jc.ok, m3);
         if (nc > 0) {
             // the candidates (in vertex order), compacted
@@ -1299,8 +1347,8 @@ int64_t junction_pass(float ghmax, const tnd::Field& f, const tnk::SeedArgs& sa,
     return total;
 }
 
-Seeds seeding_core(const tnd::Field& f, const uint8_t* d_grade, float hmin, float hmax, const tn_relax_params* prm,
-                   DevMem& mem);
+Seeds seeding_core(const tnd::Field& f, int64_t nslot, const uint8_t* d_grade, float hmin, float hmax,
+                   const tn_relax_params* prm, DevMem& mem);
 
 // v2m_h_at (src/opencl/v2m_particle_body.cl:30-36) on the host's copy of the sizing
 float host_h_at(const tn_grid_view* g, const float* p) {
@@ -1596,18 +1644,32 @@ Seeds run_seeding(const tn_grid_view* g, const uint8_t* grade, const tn_relax_pa
     mem.device = dev;
     const tnd::Field f = upload_grid(g, mem);
     const uint8_t* d_grade = mem.upload(grade, (size_t)g->nx * g->ny * g->nz);
-    const Seeds s = seeding_core(f, d_grade, g->hmin, g->hmax, prm, mem);
+    const Seeds s = seeding_core(f, g->nslot, d_grade, g->hmin, g->hmax, prm, mem);
     // seed_cpu (src/v2m_particles.cpp:625-635): the shape input's feature nodes last
     return g->nfeat > 0 ? add_feature_nodes(g, f, s, mem) : s;
 }
 
 // seed_cpu on a grid already on the device (f, its grades d_grade), scratch in mem
-Seeds seeding_core(const tnd::Field& f, const uint8_t* d_grade, float hmin, float hmax, const tn_relax_params* prm,
-                   DevMem& mem) {
+Seeds seeding_core(const tnd::Field& stored, int64_t nslot, const uint8_t* d_grade, float hmin, float hmax,
+                   const tn_relax_params* prm, DevMem& mem) {
     arg_check(prm != nullptr, "seeding: null argument");
     arg_check(prm->nseed >= 1 && prm->nseed <= 64, "seeding: nseed out of range");
     arg_check(prm->jseed >= 0.0f && std::isfinite(prm->jseed), "seeding: jseed must be finite and >= 0");
     SeedOps ops{ mem };
+    // (the copy of the Field in device memory, which other calls share, keeps no slots: they
+    // go with this call's memory, and only kernels without out-of-line calls read them)
+    tnd::Field f = stored;
+    if (!prm->voxel_trap) {
+        add_apron(f, nslot, mem, nullptr, false);
+    }
+    // run k(F): over the apron slots where there are any
+    auto over_field = [&](auto&& k) {
+        if (f.ap) {
+            k(tnd::as_field<tnd::PlainField>(f));
+        } else {
+            k(f);
+        }
+    };
     const tnd::Field* g = &f;   // (its dims)
     const int64_t nv = (int64_t)g->nx * g->ny * g->nz;
     // v2m_seed_spacing (src/opencl/v2m_seed_body.cl:445-447), with the host's powf
@@ -1639,7 +1701,9 @@ Seeds seeding_core(const tnd::Field& f, const uint8_t* d_grade, float hmin, floa
         }
     }
     int32_t* offs = ops.counts(nv);
-    tnk::k_seed_count<<<blocks_for(nv, tnk::kBlock), tnk::kBlock>>>(f, sa, offs);
+    over_field([&](const auto& f) {
+        tnk::k_seed_count<<<blocks_for(nv, tnk::kBlock), tnk::kBlock>>>(f, sa, offs);
+    });
     const int32_t total = ops.scan(offs, nv);
     const bool junctions = prm->jseed > 0.0f;
     Seeds lat;
@@ -1651,9 +1715,11 @@ Seeds seeding_core(const tnd::Field& f, const uint8_t* d_grade, float hmin, floa
     lat.part = mem.alloc<uint16_t>(2 * cap);
     lat.part3 = mem.alloc<uint16_t>(cap);
     if (total > 0) {
-        tnk::k_seed_fill<<<blocks_for(nv, tnk::kBlock), tnk::kBlock>>>(f, sa, offs, lat.P, lat.lab);
-        tnk::k_seed_classify<<<blocks_for(total, tnk::kBlock), tnk::kBlock>>>(f, total, lat.P, lat.lab, lat.typ,
-                                                                              lat.part);
+        over_field([&](const auto& f) {
+            tnk::k_seed_fill<<<blocks_for(nv, tnk::kBlock), tnk::kBlock>>>(f, sa, offs, lat.P, lat.lab);
+            tnk::k_seed_classify<<<blocks_for(total, tnk::kBlock), tnk::kBlock>>>(f, total, lat.P, lat.lab, lat.typ,
+                                                                                  lat.part);
+        });
         TN_HIP(hipMemset(lat.part3, 0xFF, sizeof(uint16_t) * total));   // kNoLab
         TN_HIP(hipGetLastError());
     }
@@ -1680,9 +1746,9 @@ template <class Plans>
 void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
     const int count = (int)plans.size();
     hipStream_t bs = plans[0]->stream;
-    bool all_plain = true;   // every grid a label volume
+    bool all_plain = true;   // every smooth move over a label volume's apron slots
     for (int k = 0; k < count; ++k) {
-        all_plain = all_plain && plans[k]->f.gm == 0;
+        all_plain = all_plain && (plans[k]->f.ap || (plans[k]->prm.voxel_trap && plans[k]->f.gm == 0));
     }
     std::vector<hipStream_t> own(count);
     for (int k = 0; k < count; ++k) {
@@ -1809,34 +1875,34 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
         // The general pass over every volume's junction queue runs on a side stream from
         // the forces on, beside the easy and lean passes (they move disjoint nodes, as in
         // a single plan's iteration); the pass over the handed-back nodes follows them.
-        auto moves = [&](auto plain) {
-            constexpr bool kP = decltype(plain)::value;
+        auto moves = [&](auto field) {
+            using FT = decltype(field);
             TN_HIP(hipEventRecord(fork_ev, bs));
             TN_HIP(hipStreamWaitEvent(gs, fork_ev, 0));
             if (tuning) {
                 TN_HIP(hipEventRecord(tune_ev[0], gs));
             }
-            kg_move<0, kP><<<nblocks[kShGen], kBlock, 0, gs>>>(dtab, bplan[kShGen], bfirst[kShGen]);
+            kg_move<0, FT><<<nblocks[kShGen], kBlock, 0, gs>>>(dtab, bplan[kShGen], bfirst[kShGen]);
             if (tuning) {
                 TN_HIP(hipEventRecord(tune_ev[1], gs));
             }
             TN_HIP(hipEventRecord(join_ev, gs));
-            kg_move_easy<kP><<<nblocks[kShNodes], kBlock, 0, bs>>>(dtab, bplan[kShNodes], bfirst[kShNodes]);
-            kg_move<1, kP><<<nblocks[kShLean], kBlock, 0, bs>>>(dtab, bplan[kShLean], bfirst[kShLean]);
-            kg_move<2, kP><<<nblocks[kShLean], kBlock, 0, bs>>>(dtab, bplan[kShLean], bfirst[kShLean]);
+            kg_move_easy<FT><<<nblocks[kShNodes], kBlock, 0, bs>>>(dtab, bplan[kShNodes], bfirst[kShNodes]);
+            kg_move<1, FT><<<nblocks[kShLean], kBlock, 0, bs>>>(dtab, bplan[kShLean], bfirst[kShLean]);
+            kg_move<2, FT><<<nblocks[kShLean], kBlock, 0, bs>>>(dtab, bplan[kShLean], bfirst[kShLean]);
             if (tuning) {
                 TN_HIP(hipEventRecord(tune_ev[2], bs));
             }
-            kg_move<3, kP><<<nblocks[kShGen], kBlock, 0, bs>>>(dtab, bplan[kShGen], bfirst[kShGen]);
+            kg_move<3, FT><<<nblocks[kShGen], kBlock, 0, bs>>>(dtab, bplan[kShGen], bfirst[kShGen]);
             if (tuning) {
                 TN_HIP(hipEventRecord(tune_ev[3], bs));
             }
             TN_HIP(hipStreamWaitEvent(bs, join_ev, 0));
         };
         if (all_plain) {
-            moves(std::true_type{});
+            moves(tnd::PlainField{});
         } else {
-            moves(std::false_type{});
+            moves(tnd::Field{});
         }
         kg_stats<<<nblocks[kShParts], kBlock, 0, bs>>>(dtab, bplan[kShParts], bfirst[kShParts]);
         kg_control<<<nblocks[kShOne], kBlock, 0, bs>>>(dtab, bplan[kShOne], bfirst[kShOne]);
@@ -2367,7 +2433,7 @@ int tn_plan_create(const tn_grid_view* g, const tn_relax_params* prm, const tn_n
         const int dev = pick_device(device);
         int64_t nkeys = 0;
         const tnd::Hash H = make_hash(g, prm, &nkeys);
-        *out = plan_build(prm, seeds, dev, H, nkeys, [&](DevMem& mem) { return upload_grid(g, mem); });
+        *out = plan_build(prm, seeds, dev, H, nkeys, g->nslot, [&](DevMem& mem) { return upload_grid(g, mem); });
     });
 }
 
@@ -2575,8 +2641,15 @@ int tn_plan_field_points(tn_plan* p, int32_t a, int32_t b, int64_t m, const floa
         float* dgrad = grad ? mem.alloc<float>((size_t)3 * m) : nullptr;
         int32_t* dlab = label ? mem.alloc<int32_t>(m) : nullptr;
         int32_t* dsec = second ? mem.alloc<int32_t>(m) : nullptr;
-        tnk::k_field_points<<<blocks_for(m, tnk::kBlock), tnk::kBlock, 0, p->stream>>>(p->f, a, b, (int)m, dX, dphi,
-                                                                                       dpsi, dgrad, dlab, dsec);
+        auto query = [&](const auto& f) {
+            tnk::k_field_points<<<blocks_for(m, tnk::kBlock), tnk::kBlock, 0, p->stream>>>(f, a, b, (int)m, dX, dphi, dpsi,
+                                                                                           dgrad, dlab, dsec);
+        };
+        if (p->f.ap) {
+            query(tnd::as_field<tnd::PlainField>(p->f));
+        } else {
+            query(p->f);
+        }
         TN_HIP(hipGetLastError());
         TN_HIP(hipStreamSynchronize(p->stream));
         auto down = [&](void* h, const void* d, size_t bytes) {
@@ -2686,7 +2759,7 @@ int tn_relax_noalloc(const tn_grid_view* g, const tn_relax_params* prm, tn_nodes
         TN_HIP(hipGetLastError());
         int64_t nkeys = 0;
         const tnd::Hash H = make_hash(g, prm, &nkeys);
-        std::unique_ptr<tn_plan> p(plan_build(prm, nd, dev, H, nkeys, [&](DevMem& mem) { return upload_grid(g, mem); },
+        std::unique_ptr<tn_plan> p(plan_build(prm, nd, dev, H, nkeys, g->nslot, [&](DevMem& mem) { return upload_grid(g, mem); },
                                               base, TN_NOALLOC_SCRATCH_BYTES));
         if (p->n > 0) {   // plan_build left it reset: seeds in place, first rebuild done
             p->run_iters(p->prm.max_iters);

@@ -51,8 +51,8 @@ __device__ __forceinline__ int voxel_owner(const Field& f, P3 p) {
 
 // v2m_seed_voxel, src/opencl/v2m_seed_body.cl:449-495. Write: store the kept
 // points from slot `out` on. Returns the number kept.
-template <bool kWrite>
-__device__ int seed_voxel(const Field& f, const SeedArgs& sa, int i, int j, int k, float* __restrict__ P,
+template <bool kWrite, class F>
+__device__ __forceinline__ int seed_voxel(const F& f, const SeedArgs& sa, int i, int j, int k, float* __restrict__ P,
                           uint16_t* __restrict__ lab, int out) {
     const size_t v = vox(f, i, j, k);
     if (f.L[v] == 0) {
@@ -90,7 +90,8 @@ __device__ int seed_voxel(const Field& f, const SeedArgs& sa, int i, int j, int 
     return n;
 }
 
-__global__ __launch_bounds__(kBlock) void k_seed_count(Field f, SeedArgs sa, int32_t* __restrict__ cnt) {
+template <class F>
+__global__ __launch_bounds__(kBlock) void k_seed_count(F f, SeedArgs sa, int32_t* __restrict__ cnt) {
     const int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int64_t nv = (int64_t)f.nx * f.ny * f.nz;
     if (v >= nv) {
@@ -100,7 +101,8 @@ __global__ __launch_bounds__(kBlock) void k_seed_count(Field f, SeedArgs sa, int
     cnt[v] = seed_voxel<false>(f, sa, i, j, k, nullptr, nullptr, 0);
 }
 
-__global__ __launch_bounds__(kBlock) void k_seed_fill(Field f, SeedArgs sa, const int32_t* __restrict__ offs,
+template <class F>
+__global__ __launch_bounds__(kBlock) void k_seed_fill(F f, SeedArgs sa, const int32_t* __restrict__ offs,
                                                       float* __restrict__ P, uint16_t* __restrict__ lab) {
     const int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int64_t nv = (int64_t)f.nx * f.ny * f.nz;
@@ -114,7 +116,8 @@ __global__ __launch_bounds__(kBlock) void k_seed_fill(Field f, SeedArgs sa, cons
 // v2m_seed_classify, src/opencl/v2m_seed_body.cl:503-594. (The size at the node is
 // the nearest voxel's, clamped to the grid like v2m_h_at; a lattice point lies in
 // its voxel's box, so the clamp never changes it.)
-__global__ __launch_bounds__(kBlock) void k_seed_classify(Field f, int n, float* __restrict__ P,
+template <class F>
+__global__ __launch_bounds__(kBlock) void k_seed_classify(F f, int n, float* __restrict__ P,
                                                           const uint16_t* __restrict__ lab, uint8_t* __restrict__ typ,
                                                           uint16_t* __restrict__ part) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
@@ -145,12 +148,12 @@ __global__ __launch_bounds__(kBlock) void k_seed_classify(Field f, int n, float*
         return;
     }
     const float hs = size_at(f, p.x, p.y, p.z);
-    const float4 g = psi_grad_point(f.self, a, b, p);
+    const float4 g = psi_grad_once(f, a, b, p);
     const float gn = sqrtf(g.x * g.x + g.y * g.y + g.z * g.z);
     if (gn < 1e-9f || fabsf(g.w) / gn > 0.5f * hs) {
         return;
     }
-    const P3ok pr = onto_interface(f.self, a, b, p, 0.6f * hs);
+    const P3ok pr = onto_interface(f, a, b, p, 0.6f * hs);
     if (!pr.ok) {
         return;
     }
@@ -171,7 +174,7 @@ __global__ __launch_bounds__(kBlock) void k_seed_classify(Field f, int n, float*
     }
     int pc_lab = kNoLab;
     if (c != kNoLab && pc > 0.5f * pa) {
-        const P3ok pj = onto_junction(f.self, a, b, c, q, 0.5f * hs);
+        const P3ok pj = onto_junction(f, a, b, c, q, 0.5f * hs);
         if (pj.ok) {
             q = pj.p;
             ty = TN_JUNCTION;
@@ -300,7 +303,8 @@ struct JunctionCands {
 
 // v2m_junction_vertex, src/opencl/v2m_particle_body.cl:302-352, for one 3-label
 // vertex of the list
-__global__ __launch_bounds__(kBlock) void k_junction_cand(Field f, SeedArgs sa, float cellfac, VertexGrid vg,
+template <class F>
+__global__ __launch_bounds__(kBlock) void k_junction_cand(F f, SeedArgs sa, float cellfac, VertexGrid vg,
                                                           const int32_t* __restrict__ list, JunctionCands jc) {
     const int s = blockIdx.x * kBlock + threadIdx.x;
     if (s >= jc.m) {
@@ -330,12 +334,12 @@ __global__ __launch_bounds__(kBlock) void k_junction_cand(Field f, SeedArgs sa, 
         }
     }
     const float vmin = fminf(fminf(f.vx, f.vy), f.vz);
-    const P3ok pj = onto_junction(f.self, a, o[0], o[1], x, vmin);
+    const P3ok pj = onto_junction(f, a, o[0], o[1], x, vmin);
     if (!pj.ok) {
         return;
     }
     x = pj.p;
-    if (!labels_dominate(f, a, o[0], o[1], x)) {
+    if (other_labels<false>(f, a, o[0], o[1], x).dominated) {
         return;
     }
     const int vi = (int)floorf(over_vx(f, x.x) + 0.5f), vj = (int)floorf(over_vy(f, x.y) + 0.5f),
