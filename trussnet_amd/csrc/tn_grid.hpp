@@ -801,14 +801,6 @@ __global__ void k_fill_u8(uint8_t* __restrict__ a, int64_t n, uint8_t x) {
     }
 }
 
-__global__ void k_pos_minmax(const float* __restrict__ a, int64_t n, int32_t* __restrict__ mm) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && a[i] > 0.0f) {   // positive floats order as their bits
-        atomicMin(&mm[0], (int32_t)__float_as_uint(a[i]));
-        atomicMax(&mm[1], (int32_t)__float_as_uint(a[i]));
-    }
-}
-
 }  // namespace tng
 
 // ---- the host driver ------------------------------------------------------------------
@@ -975,16 +967,8 @@ int tn_grid_build(const tn_volume_view* vol, const tn_grid_params* prm, int32_t 
         const float* d_hvox = nullptr;
         if (vol->hvox) {   // the user's field: the grades span its sizes too
             d_hvox = tmp.upload(vol->hvox, (size_t)nv);
-            int32_t* mm = tmp.alloc<int32_t>(2);
-            const int32_t init[2] = { 0x7F800000, 0 };
-            TN_HIP(hipMemcpy(mm, init, sizeof init, hipMemcpyHostToDevice));
-            tng::k_pos_minmax<<<nbv, 256>>>(d_hvox, nv, mm);
-            int32_t got[2];
-            TN_HIP(hipMemcpy(got, mm, sizeof got, hipMemcpyDeviceToHost));
-            if (got[1] > 0) {
-                float lo, hi;
-                std::memcpy(&lo, &got[0], 4);
-                std::memcpy(&hi, &got[1], 4);
+            const auto [lo, hi] = device_minmax<true>(d_hvox, nv, tmp.alloc<int32_t>(2), nullptr);
+            if (hi > 0.0f) {
                 hmax = std::max(hmax, hi);
                 hmin = std::min(hmin, lo);
             }
@@ -1221,13 +1205,7 @@ int tn_grid_build(const tn_volume_view* vol, const tn_grid_params* prm, int32_t 
         }
         mark("grade");
         {   // the largest h (the hash's pruning test), and the Field completed for seeding
-            int32_t* mm = tmp.alloc<int32_t>(2);
-            const int32_t init[2] = { 0x7F800000, 0 };
-            TN_HIP(hipMemcpy(mm, init, sizeof init, hipMemcpyHostToDevice));
-            tng::k_pos_minmax<<<nbv, 256>>>(h, nv, mm);
-            int32_t got[2];
-            TN_HIP(hipMemcpy(got, mm, sizeof got, hipMemcpyDeviceToHost));
-            std::memcpy(&G->hbig, &got[1], 4);
+            G->hbig = device_minmax<true>(h, nv, tmp.alloc<int32_t>(2), nullptr).second;
             f.gm = I.gm;
             f.gI = G->gI;
             f.gTW = G->dTW;
@@ -1365,7 +1343,7 @@ int tn_plan_create_from_grid(const tn_grid* g, const tn_relax_params* prm, const
         int64_t nkeys = 0;
         const tnd::Hash H = make_hash_geom(I.nx, I.ny, I.nz, vs, I.hmin, I.hmax, g->hbig, prm, &nkeys);
         // the plan keeps its own copy of the grid (device to device)
-        *out = plan_build(prm, seeds, g->mem.device, H, nkeys, I.nslot, [&](DevMem& mem) {
+        *out = plan_build(prm, seeds, g->mem.device, H, nkeys, I.nslot, false, [&](DevMem& mem) {
             const size_t nv = (size_t)I.nx * I.ny * I.nz, nb = (size_t)I.nbx * I.nby * I.nbz;
             auto dup = [&](auto* src, size_t count) {
                 using T = std::remove_const_t<std::remove_pointer_t<decltype(src)>>;

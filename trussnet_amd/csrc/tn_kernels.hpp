@@ -95,6 +95,53 @@ __device__ __forceinline__ int block_excl_scan(int v, int* lds4, int* total) {
     return base + x - v;
 }
 
+// ---- smallest and largest of an array ---------------------------------------------
+
+// mm[0]: the smallest of a, mm[1]: the largest of a and 0 (kPositive: of its positive
+// values), as float bits in signed-integer order; start from { +inf's bits, 0 }. NaNs are
+// passed over. Each block reduces its share in registers and adds one pair of atomics: an
+// atomic a value, all to two words, took 5.9 ms for 16.8 M values where this streams them
+// in 0.03 ms.
+__device__ __forceinline__ int32_t ordered_bits(float v) {
+    const int32_t b = (int32_t)__float_as_uint(v);
+    return b ^ ((b >> 31) & 0x7FFFFFFF);
+}
+
+template <bool kPositive>
+__global__ __launch_bounds__(kBlock) void k_minmax(const float* __restrict__ a, int64_t n, int32_t* __restrict__ mm) {
+    __shared__ float lds[2][kBlock / kWave];
+    float lo = __builtin_huge_valf(), hi = 0.0f;
+    const int64_t step = (int64_t)gridDim.x * kBlock;
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += step) {
+        const float v = a[i];
+        if (!kPositive || v > 0.0f) {
+            lo = fminf(lo, v);
+            hi = fmaxf(hi, v);
+        }
+    }
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, d, kWave));
+        hi = fmaxf(hi, __shfl_xor(hi, d, kWave));
+    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        lds[0][w] = lo;
+        lds[1][w] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < kBlock / kWave; ++k) {
+            lo = fminf(lo, lds[0][k]);
+            hi = fmaxf(hi, lds[1][k]);
+        }
+        atomicMin(&mm[0], ordered_bits(lo));
+        atomicMax(&mm[1], ordered_bits(hi));
+    }
+}
+
+constexpr int kMinmaxGrid = 1024;   // blocks at most (4 a CU)
+
 // ---- exclusive scan (int32), tiles of 4096 ----------------------------------------
 
 constexpr int kScanItems = 16;

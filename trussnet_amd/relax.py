@@ -281,7 +281,9 @@ class Plan:
         return st.as_dict()
 
     def download(self) -> Nodes:
-        out = self.seeds.copy()
+        sd = self.seeds
+        out = Nodes(np.empty_like(sd.P), sd.lab.copy(), np.empty_like(sd.typ), np.empty_like(sd.part),
+                    None if sd.part3 is None else sd.part3.copy())
         nv = out.view()
         _check(lib().tn_plan_download(self._h, C.byref(nv)))
         return out
