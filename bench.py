@@ -60,7 +60,8 @@ def log(*a):
 
 # Algorithmic HBM bytes per item (node, or cell for the scan) of each kernel class
 # (K = mean list length). Neighbour and field gathers count as reuse, not traffic.
-def item_bytes(kbar: float, radix_passes: int) -> dict:
+# (radix_passes: the passes of an earlier sort; nothing depends on it.)
+def item_bytes(kbar: float, radix_passes: int = 0) -> dict:
     return {
         "force": 37 + 4 * kbar,       # P,h 16 + typ 1 + nnb 4 + nbr 4K read; F 16 written
         "move": 104,                  # queue 4, F 16, P,h 16, V 16, typ 1, part 4, lab 2 read; P,h 16, V 16, typ 1,
@@ -73,9 +74,9 @@ def item_bytes(kbar: float, radix_passes: int) -> dict:
         "neighbors": 23 + 4 * kbar,   # P,h 16, typ 1, lab 2 read; nbr 4K + nnb 4 written
         "keys": 24,                   # P 12 + h 4 read; key 4 written; count 4
         "scan": 8,                    # per cell: read + write
-        "radix_sort": 20 * radix_passes,
-        "permute": 134,               # sorted 4, X 16, V 16, typ 1, part 4, lab 2, id 4 read; the same 47 written,
-                                      # Ps 16, P0 16, Ms 8, slot_of 4
+        "radix_sort": 16,             # the gathering by cell: key 4, place 4, cell start 4 read; slot 4 written
+        "permute": 142,               # slot 4, key 4, X 16, V 16, typ 1, part 4, lab 2, id 4 read; the same 43 and
+                                      # the key 4 written, Ps 16, P0 16, Ms 8, slot_of 4
     }
 
 
@@ -100,7 +101,7 @@ CLASS_KERNELS = {
     "force": ["k_force"], "move_easy": ["k_move_easy"], "move": ["k_move<1>"], "move_int": ["k_move<2>"],
     "move_rest": ["k_move<0>"], "move_def": ["k_move<0>"],
     "stats": ["k_stats"],
-    "neighbors": ["k_truss"], "refresh": ["k_refresh_list", "k_truss_node"], "permute": ["k_permute"],
+    "neighbors": ["k_truss"], "refresh": ["k_truss_node"], "permute": ["k_permute"],
     "keys": ["k_fill_i32", "k_keys"],
     "control": ["k_control"],
 }
@@ -126,10 +127,11 @@ def by_kernel(timings: dict, per_item: dict, queues: dict | None = None) -> dict
 
 def kernel_key(full: str) -> str:
     """A trace's kernel name as CLASS_KERNELS writes it: no namespace, no arguments, and
-    the label-volume flag of the move kernels' template dropped ("void
-    tnk::k_move<0, true>(...)" -> "k_move<0>", "k_move_easy<true>" -> "k_move_easy")."""
-    name = full.split("(")[0].split("::")[-1]
-    for flag in ("true", "false"):
+    the field type (or flag) of the move kernels' template dropped ("void
+    tnk::k_move<0, tnd::PlainField>(...)" -> "k_move<0>", "k_move_easy<true>" ->
+    "k_move_easy")."""
+    name = full.split("(")[0].replace("tnd::", "").split("::")[-1]
+    for flag in ("true", "false", "PlainField", "Field"):
         if name.endswith(f", {flag}>"):
             name = name[: -len(f", {flag}>")] + ">"
         elif name.endswith(f"<{flag}>"):
@@ -597,14 +599,13 @@ def main() -> int:
     # The warmup times every kernel class, to find the dominant kernel; the timed steps
     # record events around that kernel's launches only (every class's events together
     # cost about 4% of the step).
-    passes = 0 if plan.hash.nkeys <= 1 else (int(plan.hash.nkeys - 1).bit_length() + 7) // 8
     plan.set_timing(True)
     for w in range(args.warmup):
         st = plan.run()
         log(f"warmup {w}: {st['iters']} iterations, {st['rebuilds']} rebuilds")
     warm = plan.timings() if args.warmup else {}
     if warm:
-        agg = by_kernel(warm, item_bytes(24.0, passes))
+        agg = by_kernel(warm, item_bytes(24.0))
         top = max(agg, key=lambda k: agg[k]["ms"])
         plan.set_timing(tuple(agg[top]["classes"]))
         log(f"timed steps: events around {top} only (the dominant kernel of the warmup)")
@@ -634,7 +635,7 @@ def main() -> int:
                     f"{items / cnt:11.0f} items/launch")
     # roofline of the dominant kernel (the timed classes merged by kernel: the general
     # move pass runs twice an iteration, as two classes), from the timed steps' events
-    per_item = item_bytes(kbar, passes)
+    per_item = item_bytes(kbar)
 
     def kernel_roofline(kernels: dict, kname: str, steps: int) -> dict:
         a = kernels[kname]

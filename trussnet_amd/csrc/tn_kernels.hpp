@@ -44,6 +44,7 @@ struct Ctl {
     int32_t nmove_int;     // interior nodes queued for the trapped step (crossing or in snap range)
     int32_t nmove_rest;    // other nodes queued for the general trapped step (this iteration)
     int32_t nmove_def;     // nodes a lean pass handed to the general step (this iteration)
+    int32_t moved_rest;    // nmove_rest as of the end of the moves (the count itself is then cleared)
     // FIRE (FireCtl, src/v2m_particles.h:47-76)
     float dt0, dt, dtmax, alpha;
     int32_t npos;
@@ -146,6 +147,7 @@ constexpr int kMinmaxGrid = 1024;   // blocks at most (4 a CU)
 
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kBlock * kScanItems;
+constexpr int kScanTiles = 1024;   // tiles whose sums every block may add up itself (4 a thread)
 
 __global__ __launch_bounds__(kBlock) void k_scan_reduce(const int32_t* __restrict__ in, int64_t m,
                                                         int32_t* __restrict__ bsum) {
@@ -189,19 +191,32 @@ __global__ __launch_bounds__(kBlock) void k_scan_top(int32_t* __restrict__ bsum,
     }
 }
 
+// kTop: bsum holds the tiles' sums, not their scan, and each block adds up the ones
+// before its own (at most kScanTiles of them: a launch fewer, and cheaper than the one
+// block that would scan them)
+template <bool kTop>
 __global__ __launch_bounds__(kBlock) void k_scan_down(const int32_t* in, int32_t* out, int64_t m,
                                                       const int32_t* __restrict__ bsum) {
     __shared__ int lds4[4];
     const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
     int v[kScanItems];
-    int s = 0;
+    int s = 0, before = 0;
+    if (kTop) {
+        int part = 0;
+        for (unsigned k = threadIdx.x; k < blockIdx.x; k += kBlock) {
+            part += bsum[k];
+        }
+        block_excl_scan(part, lds4, &before);
+    } else {
+        before = bsum[blockIdx.x];
+    }
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         v[k] = base + k < m ? in[base + k] : 0;
         s += v[k];
     }
     int tot;
-    int run = bsum[blockIdx.x] + block_excl_scan(s, lds4, &tot);
+    int run = before + block_excl_scan(s, lds4, &tot);
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         if (base + k < m) {
@@ -215,9 +230,12 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(const int32_t* in, int32_t
 
 // X.w is v2m_h_at at the node (set with every move), the size the rebuild takes.
 // The nodes sit in cell order from the previous rebuild, so neighbouring lanes
-// mostly share a key: each run of equal keys in a wave adds its length at once.
+// mostly share a key: each run of equal keys in a wave adds its length at once, and its
+// nodes take the places in their cell that the count stood at (in arrival order: k_permute
+// puts a cell's nodes in slot order).
 __global__ __launch_bounds__(kBlock) void k_keys(Hash H, const float4* __restrict__ X, int n, float tskin,
-                                                 int32_t* __restrict__ key, int32_t* __restrict__ cnt) {
+                                                 int32_t* __restrict__ key, int32_t* __restrict__ cnt,
+                                                 int32_t* __restrict__ place) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     const int lane = threadIdx.x & (kWave - 1);
     const bool valid = i < n;
@@ -231,10 +249,25 @@ __global__ __launch_bounds__(kBlock) void k_keys(Hash H, const float4* __restric
     const bool head = valid && (lane == 0 || prev != k);
     const uint64_t heads = __ballot(head);
     const int nvalid = __popcll(__ballot(valid));   // the valid lanes are a prefix
+    int at = 0;
     if (head) {
         const uint64_t later = lane == kWave - 1 ? 0ull : heads & (~0ull << (lane + 1));
         const int end = later ? __ffsll((long long)later) - 1 : nvalid;
-        atomicAdd(&cnt[k], end - lane);
+        at = atomicAdd(&cnt[k], end - lane);
+    }
+    if (valid) {   // (lane 0 is a head: every lane has one at or below it)
+        const int first = 63 - __clzll((long long)(heads & (~0ull >> (kWave - 1 - lane))));
+        place[i] = __shfl(at, first, kWave) + lane - first;
+    }
+}
+
+// The slots gathered by cell: slot i to its cell's start plus its place there.
+__global__ __launch_bounds__(kBlock) void k_place(const int32_t* __restrict__ key, const int32_t* __restrict__ place,
+                                                  const int32_t* __restrict__ cstart, int n,
+                                                  int32_t* __restrict__ bycell) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) {
+        bycell[cstart[key[i]] + place[i]] = i;
     }
 }
 
@@ -248,6 +281,7 @@ __global__ __launch_bounds__(kBlock) void k_keys(Hash H, const float4* __restric
 // counting sort of the slots by brick position: a cell's slots stay contiguous.
 
 constexpr int kBrickEdge = 4;
+static_assert(kBrickEdge == 4, "k_brick_count takes a position apart in 2-bit fields");
 
 struct BrickMap {
     int nb[TN_MAXLEV][3];   // bricks per axis at each level
@@ -268,13 +302,30 @@ __device__ __forceinline__ int brick_pos(const Hash& H, const BrickMap& B, int k
     return B.off[L] + brick * (kBrickEdge * kBrickEdge * kBrickEdge) + within;
 }
 
-// the node count of each cell at its brick-order position (positions of no cell stay 0)
+// the node count of each brick-order position's cell (0 at a position of no cell and at
+// the end), every position written
 __global__ __launch_bounds__(kBlock) void k_brick_count(Hash H, BrickMap B, const int32_t* __restrict__ cstart,
                                                         int32_t* __restrict__ cnt) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k < H.nkeys) {
-        cnt[brick_pos(H, B, k)] = cstart[k + 1] - cstart[k];
+    const int pos = blockIdx.x * kBlock + threadIdx.x;
+    if (pos > B.size) {
+        return;
     }
+    int c = 0;
+    if (pos < B.size) {
+        int L = 0;
+        while (L + 1 < H.nlev && pos >= B.off[L + 1]) {
+            ++L;
+        }
+        const int within = (pos - B.off[L]) & 63, brick = (pos - B.off[L]) >> 6;
+        const int bx = brick % B.nb[L][0], by = (brick / B.nb[L][0]) % B.nb[L][1], bz = brick / (B.nb[L][0] * B.nb[L][1]);
+        const int cx = bx * kBrickEdge + (within & 3), cy = by * kBrickEdge + ((within >> 2) & 3),
+                  cz = bz * kBrickEdge + (within >> 4);
+        if (cx < H.dim[L][0] && cy < H.dim[L][1] && cz < H.dim[L][2]) {
+            const int k = H.off[L] + cx + H.dim[L][0] * (cy + H.dim[L][1] * cz);
+            c = cstart[k + 1] - cstart[k];
+        }
+    }
+    cnt[pos] = c;
 }
 
 // the slots in brick order: slot s goes to its cell's start in that order plus its rank
@@ -373,8 +424,15 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const int32_t* __restr
 
 // ---- renumbering in cell order ---------------------------------------------------------
 
-// Slot t takes the node of old slot sorted[t]; Ps and P0 (the positions as of this
-// rebuild) and Ms (id, typ | lab << 8) are written in the new order.
+// The nodes renumbered in cell order, a cell's nodes by their old slots: the stable sort
+// by key. bycell holds each cell's old slots in arrival order (k_place), and a node's rank
+// among them (read from LDS) is its place: two launches where the radix sort this
+// replaces took three passes of five (2.5 M nodes: 126 us of sorting and 66 of renumbering
+// a rebuild before, 11 and 80 now; 3 k nodes: 37 and 6, now 6 and 7). The rank costs a
+// read for every node of the cell: where the voxel trap stacks nodes up (hundreds in a
+// cell) the two take 131 us at 495 k nodes against 97 before, of 2.9 ms a rebuild.
+// Ps and P0 (the positions as of this rebuild) and Ms (id, typ | lab << 8) are written in
+// the new order, and keyS the nodes' keys.
 struct NodeArrays {
     float4* X;
     float4* V;
@@ -385,13 +443,36 @@ struct NodeArrays {
     uint8_t* sticky;   // handed back to the general move pass before (may be null)
 };
 
-__global__ __launch_bounds__(kBlock) void k_permute(const int32_t* __restrict__ sorted, int n, NodeArrays in,
+__global__ __launch_bounds__(kBlock) void k_permute(const int32_t* __restrict__ bycell,
+                                                    const int32_t* __restrict__ key,
+                                                    const int32_t* __restrict__ cstart, int n, NodeArrays in,
                                                     NodeArrays out, float4* __restrict__ Ps,
                                                     float4* __restrict__ P0, int2* __restrict__ Ms,
-                                                    int32_t* __restrict__ slot_of) {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t < n) {
-        const int s = sorted[t];
+                                                    int32_t* __restrict__ slot_of, int32_t* __restrict__ keyS) {
+    constexpr int kSide = kBlock / 2;
+    __shared__ int near[2 * kBlock];   // bycell around the block: most cells' slots
+    const int p = blockIdx.x * kBlock + threadIdx.x, n0 = blockIdx.x * kBlock - kSide, n1 = n0 + 2 * kBlock;
+    for (int j = threadIdx.x; j < 2 * kBlock; j += kBlock) {
+        near[j] = n0 + j >= 0 && n0 + j < n ? bycell[n0 + j] : 0;
+    }
+    __syncthreads();
+    if (p < n) {
+        const int s = near[kSide + threadIdx.x];
+        const int k = key[s];
+        const int b = cstart[k], e = cstart[k + 1];
+        const int b1 = max(b, n0), e1 = min(e, n1);
+        int t = b;
+#pragma unroll 4
+        for (int q = b1; q < e1; ++q) {
+            t += near[q - n0] < s ? 1 : 0;
+        }
+        for (int q = b; q < b1; ++q) {   // a long cell's slots beyond the window
+            t += bycell[q] < s ? 1 : 0;
+        }
+        for (int q = e1; q < e; ++q) {
+            t += bycell[q] < s ? 1 : 0;
+        }
+        keyS[t] = k;
         const float4 x = in.X[s];
         out.X[t] = x;
         Ps[t] = x;
@@ -1135,7 +1216,9 @@ __device__ __forceinline__ void k_truss_node_body(Hash H, TrussIn in, int n, con
     __shared__ float cd[kRefreshCap];
     __shared__ int cj[kRefreshCap];
     const int lane = threadIdx.x;
-    const int m = ctl->nrefresh;
+    // after k_control: a rebuild (which rebuilds every list and sets P0 = P) or the end of
+    // the loop follows, so no refreshed list would ever be read
+    const int m = ctl->rebuild || ctl->done ? 0 : ctl->nrefresh;
     const float tskin = in.t + in.skin;
     for (int q = bid; q < m; q += nblk) {
         const int i = list[q];   // the node's slot
@@ -1229,43 +1312,6 @@ __global__ __launch_bounds__(kWave) void k_truss_node(Hash H, TrussIn in, int n,
     k_truss_node_body(H, in, n, list, ctl, nbrT, nnb, P0, blockIdx.x, gridDim.x);
 }
 
-// the slots of the nodes flagged for an own-list refresh, appended block by block
-// (in slot order, which is cell order as of the last rebuild, within a block)
-__device__ __forceinline__ void k_refresh_list_body(const uint8_t* __restrict__ flag, int n, Ctl* __restrict__ ctl, int32_t* __restrict__ list, int bid, int nblk) {
-    __shared__ int woff[kBlock / kWave];
-    __shared__ int base;
-    // k_control has run: a rebuild (which rebuilds every list and sets P0 = P) or the
-    // end of the loop follows, so no refreshed list would ever be read
-    if (ctl->rebuild || ctl->done) {
-        return;
-    }
-    const int s = bid * kBlock + threadIdx.x;
-    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x >> 6;
-    const bool f = s < n && flag[s];
-    const uint64_t mask = __ballot(f);
-    if (lane == 0) {
-        woff[w] = __popcll(mask);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int tot = 0;
-        for (int k = 0; k < kBlock / kWave; ++k) {
-            const int c = woff[k];
-            woff[k] = tot;
-            tot += c;
-        }
-        base = tot ? atomicAdd(&ctl->nrefresh, tot) : 0;
-    }
-    __syncthreads();
-    if (f) {
-        list[base + woff[w] + __popcll(mask & lanemask_lt())] = s;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_refresh_list(const uint8_t* __restrict__ flag, int n, Ctl* __restrict__ ctl, int32_t* __restrict__ list) {
-    k_refresh_list_body(flag, n, ctl, list, blockIdx.x, gridDim.x);
-}
-
 // ---- node counts by type: interface, junction, interior, corner ------------------------
 
 __device__ __forceinline__ int type_rank(int t) {
@@ -1334,6 +1380,13 @@ __device__ __forceinline__ void wave_append(bool flag, int i, int32_t* count, in
 __device__ __forceinline__ void k_force_body(const float4* __restrict__ X, const uint8_t* __restrict__ typ, const int32_t* __restrict__ nbrT, const int32_t* __restrict__ nnb, float fscale, float fsurf, int n, float4* __restrict__ F, Ctl* __restrict__ ctl, int32_t* __restrict__ queue_rest, uint8_t* __restrict__ skip, const uint8_t* __restrict__ sticky, int bid, int nblk) {
     const int i = bid * kBlock + threadIdx.x;
     bool junction = false;
+    if (i == 0) {   // the counts that the iteration's later kernels fill
+        ctl->nhalf = 0;
+        ctl->nrefresh = 0;
+        ctl->nmove = 0;
+        ctl->nmove_int = 0;
+        ctl->nmove_def = 0;
+    }
     if (i < n) {
         F[i] = bar_force(X, typ, nbrT, nnb, fscale, fsurf, i, n);
         if (queue_rest) {
@@ -1794,10 +1847,15 @@ constexpr int kHistThr = 35;   // exponents -21..13
 constexpr int kStatsBlocks = 2048;   // k_stats' grid at most (8 blocks per CU)
 
 // Per iteration: the histogram, the largest move, the count past skin/2, the
-// flags of the nodes past a full skin (their lists are refreshed), and FIRE's
+// nodes past a full skin (listed: their own lists are refreshed), and FIRE's
 // power partial sums (src/v2m_particles.cpp:849-937). Counts are reduced per
-// wave with ballots before any atomic.
-__device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const float4* __restrict__ P0, const float* __restrict__ mv, const float* __restrict__ pw, int n, float skin, int fire, const float* __restrict__ thr, Ctl* __restrict__ ctl, uint8_t* __restrict__ refresh, double2* __restrict__ partials, int bid, int nblk) {
+// wave with ballots before any atomic, and the listed nodes gathered in LDS, so that a
+// block takes its place in the list once (a pass of its own over a flag a node, as
+// before, cost 8 us an iteration at 2.5 M nodes and a launch at any size).
+__device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const float4* __restrict__ P0, const float* __restrict__ mv, const float* __restrict__ pw, int n, float skin, int fire, const float* __restrict__ thr, Ctl* __restrict__ ctl, int32_t* __restrict__ refresh, double2* __restrict__ partials, int bid, int nblk) {
+    constexpr int kHeld = 4 * kBlock;
+    __shared__ int held[kHeld];   // nodes to list
+    __shared__ int nheld, held_at;
     __shared__ uint32_t lh[32];
     __shared__ uint32_t lmax;
     __shared__ int lhalf;
@@ -1809,17 +1867,41 @@ __device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const
     if (tid == 0) {
         lmax = 0;
         lhalf = 0;
+        nheld = 0;
+        if (bid == 0) {   // (the moves are done: the queue is free for the next k_force)
+            ctl->moved_rest = ctl->nmove_rest;
+            ctl->nmove_rest = 0;
+        }
     }
+    // every thread of the block: the held nodes into the list
+    auto list_held = [&]() {
+        const int m = nheld;
+        if (tid == 0) {
+            held_at = atomicAdd(&ctl->nrefresh, m);
+        }
+        __syncthreads();
+        for (int e = tid; e < m; e += kBlock) {
+            refresh[held_at + e] = held[e];
+        }
+        __syncthreads();
+        if (tid == 0) {
+            nheld = 0;
+        }
+        __syncthreads();
+    };
     double bs = 0.0, ba = 0.0;   // this block's power partial sums (thread 0), chunk by chunk
     // chunks of kBlock nodes, grid-strided: each block adds its counts to the control
     // block once, and its partial sums have a fixed shape
     for (int c = bid; (int64_t)c * kBlock < n; c += nblk) {
         __syncthreads();   // lps of the previous chunk has been read
+        if (nheld > kHeld - kBlock) {
+            list_held();
+        }
         const int i = c * kBlock + tid;
         double ps = 0.0, pa = 0.0;
         int bin = -1;
         uint32_t mbits = 0;
-        bool half = false;
+        bool half = false, far = false;
         if (i < n) {
             const float m = mv[i];
             bin = hist_bin(m, thr);
@@ -1828,12 +1910,23 @@ __device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const
             const float ex = x.x - x0.x, ey = x.y - x0.y, ez = x.z - x0.z;
             const float h = x.w;
             const float m2 = ex * ex + ey * ey + ez * ez, s2 = skin * skin * h * h;
-            const bool far = m2 > s2;
-            refresh[i] = far ? 1 : 0;
+            far = m2 > s2;
             half = !far && m2 > 0.25f * s2;
             if (fire) {
                 ps = (double)pw[i];
                 pa = fabs(ps);
+            }
+        }
+        const uint64_t fm = __ballot(far);
+        if (fm) {
+            const int lead = __ffsll((long long)fm) - 1;
+            int at = 0;
+            if (lane == lead) {
+                at = atomicAdd(&nheld, __popcll(fm));
+            }
+            at = __shfl(at, lead, kWave);
+            if (far) {
+                held[at + __popcll(fm & lanemask_lt())] = i;
             }
         }
         // histogram: one LDS add per (wave, occupied bin)
@@ -1875,6 +1968,9 @@ __device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const
         }
     }
     __syncthreads();
+    if (nheld) {
+        list_held();
+    }
     if (tid < 32 && lh[tid]) {
         atomicAdd(&ctl->hist[tid], lh[tid]);
     }
@@ -1889,7 +1985,7 @@ __device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_stats(const float4* __restrict__ X, const float4* __restrict__ P0, const float* __restrict__ mv, const float* __restrict__ pw, int n, float skin, int fire, const float* __restrict__ thr, Ctl* __restrict__ ctl, uint8_t* __restrict__ refresh, double2* __restrict__ partials) {
+__global__ __launch_bounds__(kBlock) void k_stats(const float4* __restrict__ X, const float4* __restrict__ P0, const float* __restrict__ mv, const float* __restrict__ pw, int n, float skin, int fire, const float* __restrict__ thr, Ctl* __restrict__ ctl, int32_t* __restrict__ refresh, double2* __restrict__ partials) {
     k_stats_body(X, P0, mv, pw, n, skin, fire, thr, ctl, refresh, partials, blockIdx.x, gridDim.x);
 }
 
@@ -2051,22 +2147,6 @@ __global__ __launch_bounds__(kBlock) void k_control(CtlArgs ca, Ctl* __restrict_
     k_control_body(ca, ctl, partials, pw, slot_of, blockIdx.x, gridDim.x);
 }
 
-// clears the per-iteration counters that k_stats and k_refresh_list fill
-__device__ __forceinline__ void k_iter_begin_body(Ctl* __restrict__ ctl, int bid, int nblk) {
-    if (threadIdx.x == 0) {
-        ctl->nhalf = 0;
-        ctl->nrefresh = 0;
-        ctl->nmove = 0;
-        ctl->nmove_int = 0;
-        ctl->nmove_rest = 0;
-        ctl->nmove_def = 0;
-    }
-}
-
-__global__ void k_iter_begin(Ctl* __restrict__ ctl) {
-    k_iter_begin_body(ctl, blockIdx.x, gridDim.x);
-}
-
 // ---- grouped launches: one launch runs an iteration's kernel for many plans -------
 //
 // Each plan's arguments sit in a device table; a block finds its plan and its block
@@ -2106,12 +2186,6 @@ struct PlanIter {
     const PlanIter& P = tab[v_];                          \
     const int bid_ = (int)blockIdx.x - bfirst[v_];        \
     const int nb_ = P.nblk[shape]
-
-__global__ void kg_iter_begin(const PlanIter* __restrict__ tab, const int32_t* __restrict__ bplan,
-                              const int32_t* __restrict__ bfirst) {
-    TN_PLAN_BLOCK(kShOne);
-    k_iter_begin_body(P.ctl, bid_, nb_);
-}
 
 __global__ __launch_bounds__(kBlock) void kg_force(const PlanIter* __restrict__ tab, const int32_t* __restrict__ bplan,
                                                    const int32_t* __restrict__ bfirst) {
@@ -2162,14 +2236,7 @@ __global__ __launch_bounds__(kBlock, TN_MOVE_WAVES) void kg_move(const PlanIter*
 __global__ __launch_bounds__(kBlock) void kg_stats(const PlanIter* __restrict__ tab, const int32_t* __restrict__ bplan,
                                                    const int32_t* __restrict__ bfirst) {
     TN_PLAN_BLOCK(kShParts);
-    k_stats_body(P.X, P.P0, P.mv, P.pw, P.n, P.skin, P.fire, P.thr, P.ctl, P.flag, P.partials, bid_, nb_);
-}
-
-__global__ __launch_bounds__(kBlock) void kg_refresh_list(const PlanIter* __restrict__ tab,
-                                                          const int32_t* __restrict__ bplan,
-                                                          const int32_t* __restrict__ bfirst) {
-    TN_PLAN_BLOCK(kShNodes);
-    k_refresh_list_body(P.flag, P.n, P.ctl, P.rqueue, bid_, nb_);
+    k_stats_body(P.X, P.P0, P.mv, P.pw, P.n, P.skin, P.fire, P.thr, P.ctl, P.rqueue, P.partials, bid_, nb_);
 }
 
 __global__ __launch_bounds__(kWave) void kg_truss_node(const PlanIter* __restrict__ tab,

@@ -156,6 +156,18 @@ void hist_thresholds(float* thr) {
     }
 }
 
+// out = the exclusive scan of in[0..m) (they may be the same array); bsum: a word a tile
+void launch_scan(const int32_t* in, int32_t* out, int64_t m, int32_t* bsum, hipStream_t s) {
+    const unsigned nb = blocks_for(m, tnk::kScanTile);
+    tnk::k_scan_reduce<<<nb, tnk::kBlock, 0, s>>>(in, m, bsum);
+    if (nb <= (unsigned)tnk::kScanTiles) {
+        tnk::k_scan_down<true><<<nb, tnk::kBlock, 0, s>>>(in, out, m, bsum);
+    } else {
+        tnk::k_scan_top<<<1, tnk::kBlock, 0, s>>>(bsum, nb);
+        tnk::k_scan_down<false><<<nb, tnk::kBlock, 0, s>>>(in, out, m, bsum);
+    }
+}
+
 __global__ void k_init_nodes(tnd::Field f, const float* __restrict__ P, int n, float4* __restrict__ X) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
@@ -515,17 +527,16 @@ struct tn_plan {
     // nodes a lean move pass has handed back to the general pass in an earlier iteration
     // of this run (by slot): k_force queues them for the general pass directly
     uint8_t *dSticky = nullptr, *dStickyb = nullptr;
-    const int32_t* dKeySorted = nullptr;   // the keys in slot order after the last rebuild
+    int32_t* dPlace = nullptr;             // a node's place in its cell (a rebuild's counting)
+    int32_t* dKeySorted = nullptr;         // the keys in slot order after the last rebuild
     tnk::BrickMap bricks{};                // the K-nearest search's query order (brick positions)
     int32_t* dBrick = nullptr;             // [bricks.size + 1]: node counts, then starts, by brick position
     float *dMv = nullptr, *dPw = nullptr, *dThr = nullptr;
     int32_t *dKey = nullptr, *dCstart = nullptr, *dSorted = nullptr, *dNbrT = nullptr, *dNnb = nullptr;
-    int32_t *dQueue = nullptr, *dBhist = nullptr, *dBsum = nullptr;
+    int32_t *dQueue = nullptr, *dBsum = nullptr;
     // the move queues: interface (lean), interior (lean), general, handed back
     int32_t *dMoveQ = nullptr, *dMoveQi = nullptr, *dMoveQ2 = nullptr, *dMoveQd = nullptr;
-    uint8_t* dFlag = nullptr;   // nodes past a full skin this iteration
-    int32_t* dRk[2] = { nullptr, nullptr };
-    int32_t* dRv[2] = { nullptr, nullptr };
+    uint8_t* dFlag = nullptr;   // nodes k_force queued for the general pass this iteration
     double2* dPartials = nullptr;
     tnk::Ctl* dCtl = nullptr;
     tnk::Ctl* hCtl = nullptr;   // pinned (pageable: hctl_local, in a plan that allocates nothing)
@@ -543,7 +554,7 @@ struct tn_plan {
     // at once keep the device busy by themselves; cross-stream waits of many plans
     // would queue behind each other on the few hardware queues)
     bool overlap_moves = true;
-    int nparts = 0, radix_passes = 0, radix_nblk = 0, refresh_blocks = 1;
+    int nparts = 0, refresh_blocks = 1;
     // host-side loop state
     int rebuilds = 0;
     bool finished = false;
@@ -584,10 +595,7 @@ struct tn_plan {
     }
 
     void scan(const int32_t* in, int32_t* out, int64_t m) {
-        const unsigned nb = blocks_for(m, tnk::kScanTile);
-        tnk::k_scan_reduce<<<nb, tnk::kBlock, 0, stream>>>(in, m, dBsum);
-        tnk::k_scan_top<<<1, tnk::kBlock, 0, stream>>>(dBsum, nb);
-        tnk::k_scan_down<<<nb, tnk::kBlock, 0, stream>>>(in, out, m, dBsum);
+        launch_scan(in, out, m, dBsum, stream);
     }
 
     tnd::TrussIn truss_in() const {
@@ -611,31 +619,19 @@ struct tn_plan {
         const unsigned nb = blocks_for(n, tnk::kBlock);
         hipEvent_t t = timer.begin(KC_KEYS);
         tnk::k_fill_i32<<<blocks_for(nkeys + 1, tnk::kBlock), tnk::kBlock, 0, stream>>>(dCstart, nkeys + 1, 0);
-        tnk::k_keys<<<nb, tnk::kBlock, 0, stream>>>(H, dX, n, tskin, dKey, dCstart);
+        tnk::k_keys<<<nb, tnk::kBlock, 0, stream>>>(H, dX, n, tskin, dKey, dCstart, dPlace);
         timer.end(KC_KEYS, t);
         t = timer.begin(KC_SCAN);
         scan(dCstart, dCstart, nkeys + 1);
         timer.end(KC_SCAN, t);
         t = timer.begin(KC_RADIX);
-        if (radix_passes == 0) {
-            k_iota<<<nb, tnk::kBlock, 0, stream>>>(dSorted, n);
-        }
-        for (int p = 0; p < radix_passes; ++p) {
-            const int32_t* kin = p == 0 ? dKey : dRk[(p - 1) & 1];
-            const int32_t* vin = p == 0 ? nullptr : dRv[(p - 1) & 1];
-            int32_t* kout = dRk[p & 1];
-            int32_t* vout = p == radix_passes - 1 ? dSorted : dRv[p & 1];
-            tnk::k_radix_hist<<<radix_nblk, tnk::kBlock, 0, stream>>>(kin, n, 8 * p, radix_nblk, dBhist);
-            scan(dBhist, dBhist, (int64_t)256 * radix_nblk);
-            tnk::k_radix_scatter<<<radix_nblk, tnk::kBlock, 0, stream>>>(kin, vin, n, 8 * p, radix_nblk, dBhist, kout,
-                                                                          vout);
-        }
+        tnk::k_place<<<nb, tnk::kBlock, 0, stream>>>(dKey, dPlace, dCstart, n, dSorted);
         timer.end(KC_RADIX, t);
         t = timer.begin(KC_PERMUTE);
-        dKeySorted = radix_passes == 0 ? dKey : dRk[(radix_passes - 1) & 1];
         const tnk::NodeArrays cur{ dX, dV, dTyp, dPart, dLab, dId, dSticky },
             nxt{ dXb, dVb, dTypb, dPartb, dLabb, dIdb, dStickyb };
-        tnk::k_permute<<<nb, tnk::kBlock, 0, stream>>>(dSorted, n, cur, nxt, dPs, dP0, dMs, dSlotOf);
+        tnk::k_permute<<<nb, tnk::kBlock, 0, stream>>>(dSorted, dKey, dCstart, n, cur, nxt, dPs, dP0, dMs, dSlotOf,
+                                                       dKeySorted);
         std::swap(dX, dXb);
         std::swap(dV, dVb);
         std::swap(dTyp, dTypb);
@@ -646,9 +642,8 @@ struct tn_plan {
         timer.end(KC_PERMUTE, t);
         t = timer.begin(KC_NEIGHBORS);
         // the query order, into dSorted (free once the nodes are permuted)
-        tnk::k_fill_i32<<<blocks_for(bricks.size + 1, tnk::kBlock), tnk::kBlock, 0, stream>>>(dBrick, bricks.size + 1,
-                                                                                             0);
-        tnk::k_brick_count<<<blocks_for(nkeys, tnk::kBlock), tnk::kBlock, 0, stream>>>(H, bricks, dCstart, dBrick);
+        tnk::k_brick_count<<<blocks_for((int64_t)bricks.size + 1, tnk::kBlock), tnk::kBlock, 0, stream>>>(H, bricks, dCstart,
+                                                                                                         dBrick);
         scan(dBrick, dBrick, (int64_t)bricks.size + 1);
         tnk::k_brick_order<<<nb, tnk::kBlock, 0, stream>>>(H, bricks, dKeySorted, n, dCstart, dBrick, dSorted);
         tnk::k_truss<<<blocks_for(n, tnk::kTrussWave), tnk::kTrussWave, 0, stream>>>(H, truss_in(), n, dNbrT, dNnb);
@@ -696,7 +691,6 @@ struct tn_plan {
     // control block's copy to the host and ev_iter behind them
     void enqueue_iteration() {
         const unsigned nb = blocks_for(n, tnk::kBlock);
-        tnk::k_iter_begin<<<1, 64, 0, stream>>>(dCtl);
         hipEvent_t t = timer.begin(KC_FORCE);
         // (the junction nodes queued for the general pass, unless the move is the voxel trap's)
         tnk::k_force<<<nb, tnk::kBlock, 0, stream>>>(dX, dTyp, dNbrT, dNnb, prm.fscale, prm.fsurf, n, dF, dCtl,
@@ -712,7 +706,7 @@ struct tn_plan {
             tnk::k_move_voxel_wave<<<std::min<unsigned>(nb, tnk::kMoveGrid), tnk::kBlock, 0, stream>>>(
                 f, ma, dCtl, dMoveQ, &dCtl->nmove, dF, dX, dV, dTyp, dPart, dLab, dMv, dPw);
             timer.end(KC_MOVE, t);
-            enqueue_iteration_tail(nb);
+            enqueue_iteration_tail();
             return;
         }
         // (label volumes: the move kernels over their apron slots, with no other field mode)
@@ -771,13 +765,13 @@ struct tn_plan {
         } else {
             moves(f);
         }
-        enqueue_iteration_tail(nb);
+        enqueue_iteration_tail();
     }
 
     // stats, own-list refreshes, control, and the control block's copy to the host
-    void enqueue_iteration_tail(unsigned nb) {
+    void enqueue_iteration_tail() {
         hipEvent_t t = timer.begin(KC_STATS);
-        tnk::k_stats<<<nparts, tnk::kBlock, 0, stream>>>(dX, dP0, dMv, dPw, n, prm.skin, fire, dThr, dCtl, dFlag,
+        tnk::k_stats<<<nparts, tnk::kBlock, 0, stream>>>(dX, dP0, dMv, dPw, n, prm.skin, fire, dThr, dCtl, dQueue,
                                                          dPartials);
         timer.end(KC_STATS, t);
         // the control before the own-list refreshes, which it does not read: they are
@@ -787,7 +781,6 @@ struct tn_plan {
         tnk::k_control<<<1, tnk::kBlock, 0, stream>>>(ca, dCtl, dPartials, dPw, dSlotOf);
         timer.end(KC_CONTROL, t);
         t = timer.begin(KC_REFRESH);
-        tnk::k_refresh_list<<<nb, tnk::kBlock, 0, stream>>>(dFlag, n, dCtl, dQueue);
         tnk::k_truss_node<<<refresh_blocks, tnk::kWave, 0, stream>>>(H, truss_in(), n, dQueue, dCtl, dNbrT, dNnb, dP0);
         timer.end(KC_REFRESH, t);
         TN_HIP(hipGetLastError());
@@ -807,9 +800,9 @@ struct tn_plan {
         }
         timer.count(KC_MOVE, hCtl->nmove);
         timer.count(KC_MOVE_INT, hCtl->nmove_int);
-        timer.count(KC_MOVE_REST, hCtl->nmove_rest);
+        timer.count(KC_MOVE_REST, hCtl->moved_rest);
         timer.count(KC_MOVE_DEF, hCtl->nmove_def);
-        timer.count(KC_REFRESH, hCtl->nrefresh);
+        timer.count(KC_REFRESH, hCtl->rebuild || hCtl->done ? 0 : hCtl->nrefresh);
         timer.count(KC_CONTROL, 1);
         if (hCtl->done) {
             finished = true;
@@ -1006,15 +999,8 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
         p->dMoveQd = p->alloc<int32_t>(n);
         p->dFlag = p->alloc<uint8_t>(n);
         p->dCstart = p->alloc<int32_t>((size_t)p->nkeys + 1);
-        for (int k = 0; k < 2; ++k) {
-            p->dRk[k] = p->alloc<int32_t>(n);
-            p->dRv[k] = p->alloc<int32_t>(n);
-        }
-        // radix sort geometry: 8-bit digits over the key range [0, nkeys)
-        const int bits = p->nkeys <= 1 ? 0 : 32 - __builtin_clz((unsigned)(p->nkeys - 1));
-        p->radix_passes = (bits + 7) / 8;
-        p->radix_nblk = (int)std::max<unsigned>(1, blocks_for(n, tnk::kRadixTile));
-        p->dBhist = p->alloc<int32_t>((size_t)256 * p->radix_nblk);
+        p->dPlace = p->alloc<int32_t>(n);
+        p->dKeySorted = p->alloc<int32_t>(n);
         {   // the query order's brick positions
             int64_t pos = 0;
             for (int L = 0; L < p->H.nlev; ++L) {
@@ -1030,8 +1016,7 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
             p->bricks.size = (int)pos;
             p->dBrick = p->alloc<int32_t>((size_t)pos + 1);
         }
-        const int64_t scan_max = std::max<int64_t>(std::max<int64_t>(p->nkeys, p->bricks.size) + 1,
-                                                   (int64_t)256 * p->radix_nblk);
+        const int64_t scan_max = std::max<int64_t>(p->nkeys, p->bricks.size) + 1;
         p->dBsum = p->alloc<int32_t>(blocks_for(scan_max, tnk::kScanTile));
         p->nparts = (int)std::max<unsigned>(1, std::min<unsigned>(blocks_for(n, tnk::kBlock), tnk::kStatsBlocks));
         p->refresh_blocks = (int)std::max<int64_t>(1, std::min<int64_t>(n, 2048));   // one wave per listed node
@@ -1212,9 +1197,7 @@ struct SeedOps {
     int32_t scan(int32_t* offs, int64_t m) {
         const unsigned nb = blocks_for(m + 1, tnk::kScanTile);
         int32_t* bsum = mem.alloc<int32_t>(nb);
-        tnk::k_scan_reduce<<<nb, tnk::kBlock>>>(offs, m + 1, bsum);
-        tnk::k_scan_top<<<1, tnk::kBlock>>>(bsum, nb);
-        tnk::k_scan_down<<<nb, tnk::kBlock>>>(offs, offs, m + 1, bsum);
+        launch_scan(offs, offs, m + 1, bsum, nullptr);
         TN_HIP(hipGetLastError());
         int32_t total = 0;
         TN_HIP(hipMemcpy(&total, offs + m, sizeof total, hipMemcpyDeviceToHost));
@@ -1252,9 +1235,7 @@ struct SeedOps {
     void scan_exclusive(int32_t* a, int64_t m) {   // in place, no total
         const unsigned nb = blocks_for(m, tnk::kScanTile);
         int32_t* bsum = mem.alloc<int32_t>(nb);
-        tnk::k_scan_reduce<<<nb, tnk::kBlock>>>(a, m, bsum);
-        tnk::k_scan_top<<<1, tnk::kBlock>>>(bsum, nb);
-        tnk::k_scan_down<<<nb, tnk::kBlock>>>(a, a, m, bsum);
+        launch_scan(a, a, m, bsum, nullptr);
     }
 };
 
@@ -1911,7 +1892,6 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
     while (!active.empty()) {
         using namespace tnk;
         const bool tuning = tune_step >= 0 && tune_step < ncand * kTuneIters;
-        kg_iter_begin<<<nblocks[kShOne], 64, 0, bs>>>(dtab, bplan[kShOne], bfirst[kShOne]);
         kg_force<<<nblocks[kShNodes], kBlock, 0, bs>>>(dtab, bplan[kShNodes], bfirst[kShNodes]);
         // The general pass over every volume's junction queue runs on a side stream from
         // the forces on, beside the easy and lean passes (they move disjoint nodes, as in
@@ -1947,7 +1927,6 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
         }
         kg_stats<<<nblocks[kShParts], kBlock, 0, bs>>>(dtab, bplan[kShParts], bfirst[kShParts]);
         kg_control<<<nblocks[kShOne], kBlock, 0, bs>>>(dtab, bplan[kShOne], bfirst[kShOne]);
-        kg_refresh_list<<<nblocks[kShNodes], kBlock, 0, bs>>>(dtab, bplan[kShNodes], bfirst[kShNodes]);
         kg_truss_node<<<nblocks[kShRefresh], kWave, 0, bs>>>(dtab, bplan[kShRefresh], bfirst[kShRefresh]);
         kg_ctl_gather<<<nblocks[kShOne], 64, 0, bs>>>(dtab, bplan[kShOne], bfirst[kShOne], dctl);
         TN_HIP(hipGetLastError());
@@ -1960,7 +1939,7 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
             TN_HIP(hipEventElapsedTime(&b, tune_ev[2], tune_ev[3]));
             double queued = 0.0;
             for (const int k : active) {
-                queued += (double)hctl[k].nmove_rest + (double)hctl[k].nmove_def;
+                queued += (double)hctl[k].moved_rest + (double)hctl[k].nmove_def;
             }
             tune_ms[tune_step % ncand] += (double)a + (double)b;
             tune_nodes[tune_step % ncand] += queued;
