@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <array>
+#include <list>
 #include <map>
 #include <thread>
 #include <type_traits>
@@ -204,35 +205,81 @@ __global__ void k_iota(int32_t* __restrict__ a, int n) {
 // Freed device buffers kept for reuse, by device and size, so that creating and
 // destroying plans (a batch of 64 volumes, a loop of single calls) rarely calls
 // hipMalloc / hipFree, each of which costs tens of microseconds to milliseconds
-// and a device-wide sync. At most TN_MEM_CACHE_MB (default 8192; 0: off) are kept;
-// the buffers are never returned to the driver before the process ends.
+// and a device-wide sync. At most TN_MEM_CACHE_MB (default 8192; 0: off) are kept: past
+// that the oldest go back to the driver, and all of a device's do when an allocation on
+// it fails. Large sizes are rounded up by at most an eighth (size_class), so that
+// volumes of about one size share buffers.
 struct MemCache {
+    struct Entry {
+        int dev;
+        size_t bytes;
+        void* p;
+    };
+    using List = std::list<Entry>;   // oldest first
     std::mutex mu;
-    std::multimap<std::pair<int, size_t>, void*> free;
+    List kept;
+    std::multimap<std::pair<int, size_t>, List::iterator> by_size;
     size_t bytes = 0, cap = 0;
     MemCache() {
         const char* e = std::getenv("TN_MEM_CACHE_MB");
         cap = (e && e[0] ? (size_t)std::strtoull(e, nullptr, 10) : (size_t)8192) << 20;
     }
+    static size_t size_class(size_t b) {
+        size_t step = 1;
+        while (step * 16 <= b) {
+            step <<= 1;
+        }
+        return (b + step - 1) / step * step;   // (step: between a sixteenth and an eighth of b)
+    }
     void* take(int dev, size_t b) {
         std::lock_guard<std::mutex> g(mu);
-        const auto it = free.find({ dev, b });
-        if (it == free.end()) {
+        const auto it = by_size.find({ dev, b });
+        if (it == by_size.end()) {
             return nullptr;
         }
-        void* p = it->second;
-        free.erase(it);
+        void* p = it->second->p;
+        kept.erase(it->second);
+        by_size.erase(it);
         bytes -= b;
         return p;
     }
-    bool give(int dev, size_t b, void* p) {
+    // (the caller has synchronised the device: nothing in flight uses the buffer)
+    void give(int dev, size_t b, void* p) {
         std::lock_guard<std::mutex> g(mu);
-        if (bytes + b > cap) {
-            return false;
+        if (b > cap) {
+            (void)hipFree(p);
+            return;
         }
-        free.emplace(std::make_pair(dev, b), p);
+        while (bytes + b > cap) {
+            drop(kept.begin());
+        }
+        kept.push_back({ dev, b, p });
+        by_size.emplace(std::make_pair(dev, b), std::prev(kept.end()));
         bytes += b;
-        return true;
+    }
+    void drop_device(int dev) {
+        std::lock_guard<std::mutex> g(mu);
+        for (auto it = kept.begin(); it != kept.end();) {
+            const auto next = std::next(it);
+            if (it->dev == dev) {
+                drop(it);
+            }
+            it = next;
+        }
+    }
+
+private:
+    void drop(List::iterator e) {
+        auto r = by_size.equal_range({ e->dev, e->bytes });
+        for (auto it = r.first; it != r.second; ++it) {
+            if (it->second == e) {
+                by_size.erase(it);
+                break;
+            }
+        }
+        bytes -= e->bytes;
+        (void)hipFree(e->p);
+        kept.erase(e);
     }
 };
 
@@ -272,20 +319,23 @@ struct DevMem {
         }
         (void)hipDeviceSynchronize();   // no work in flight may still use them
         for (const Owned& o : owned) {
-            if (!mem_cache().give(o.dev, o.bytes, o.p)) {
-                (void)hipFree(o.p);
-            }
+            mem_cache().give(o.dev, o.bytes, o.p);
         }
     }
-    // a buffer of exactly `bytes` on the current device: a cached one, else a new one
+    // a buffer of `bytes` at least on the current device: a cached one, else a new one
     void* fresh(size_t bytes) {
         int dev = 0;
         TN_HIP(hipGetDevice(&dev));
-        void* p = mem_cache().take(dev, bytes);
-        if (!p) {
-            TN_HIP(hipMalloc(&p, bytes));
+        size_t b = MemCache::size_class(bytes);
+        void* p = mem_cache().take(dev, b);
+        if (!p && hipMalloc(&p, b) != hipSuccess) {
+            // no room: the kept buffers back to the driver, and no more than was asked for
+            (void)hipGetLastError();
+            mem_cache().drop_device(dev);
+            b = bytes;
+            TN_HIP(hipMalloc(&p, b));
         }
-        owned.push_back({ p, bytes, dev });
+        owned.push_back({ p, b, dev });
         return p;
     }
     void set_arena(void* base, size_t cap) {
@@ -499,10 +549,102 @@ struct KernelTimer {
     }
 };
 
+// What a plan needs of the runtime beside memory: its streams, events and the pinned
+// control block. Creating and destroying them took 3 ms a plan (a stream 0.29 and 0.44
+// ms, the pinned block 0.12 and 0.55), as long as the whole relaxation of a small volume,
+// so a plan that ends leaves them for the next on its device, at most kKits of them in
+// all; they are idle then, and a plan holds its own for as long as it lives.
+struct PlanKit {
+    hipStream_t stream = nullptr, side[2] = { nullptr, nullptr };
+    hipEvent_t events[5] = {};
+    tnk::Ctl* ctl = nullptr;
+
+    void make() {
+        TN_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        for (hipStream_t& s : side) {
+            TN_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        }
+        for (hipEvent_t& e : events) {
+            TN_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        }
+        TN_HIP(hipHostMalloc((void**)&ctl, sizeof(tnk::Ctl), hipHostMallocDefault));
+    }
+    bool whole() const {
+        return ctl != nullptr;
+    }
+    bool idle() const {   // waits for the streams; false when one of them has failed
+        bool ok = true;
+        for (hipStream_t s : { stream, side[0], side[1] }) {
+            ok = (!s || hipStreamSynchronize(s) == hipSuccess) && ok;
+        }
+        return ok;
+    }
+    void destroy() {
+        if (ctl) {
+            (void)hipHostFree(ctl);
+        }
+        for (hipEvent_t e : events) {
+            if (e) {
+                (void)hipEventDestroy(e);
+            }
+        }
+        for (hipStream_t s : { side[0], side[1], stream }) {
+            if (s) {
+                (void)hipStreamDestroy(s);
+            }
+        }
+        *this = PlanKit{};
+    }
+};
+
+struct KitPool {
+    static constexpr size_t kKits = 32;
+    std::mutex mu;
+    std::vector<std::pair<int, PlanKit>> idle;   // (device, kit)
+
+    PlanKit take(int dev) {
+        {
+            std::lock_guard<std::mutex> g(mu);
+            for (size_t k = idle.size(); k-- > 0;) {
+                if (idle[k].first == dev) {
+                    const PlanKit kit = idle[k].second;
+                    idle.erase(idle.begin() + (long)k);
+                    return kit;
+                }
+            }
+        }
+        PlanKit kit;
+        try {
+            kit.make();
+        } catch (...) {
+            kit.destroy();
+            throw;
+        }
+        return kit;
+    }
+    void give(int dev, PlanKit& kit) {
+        if (kit.idle() && kit.whole()) {
+            std::lock_guard<std::mutex> g(mu);
+            if (idle.size() < kKits) {
+                idle.emplace_back(dev, kit);
+                kit = PlanKit{};
+                return;
+            }
+        }
+        kit.destroy();
+    }
+};
+
+KitPool& kit_pool() {
+    static KitPool* p = new KitPool;   // (never destroyed: the runtime may be gone at exit)
+    return *p;
+}
+
 }  // namespace
 
 struct tn_plan {
     int device = 0;
+    PlanKit kit;   // the owner of the streams, events and pinned block below
     hipStream_t stream = nullptr;
     tn_relax_params prm{};
     int n = 0, fire = 0, rebuild_div = 300;
@@ -558,6 +700,7 @@ struct tn_plan {
     // host-side loop state
     int rebuilds = 0;
     bool finished = false;
+    bool at_seeds = false;   // as reset() leaves it: the seeds in place, the first rebuild done
 
     template <class T>
     T* alloc(size_t count) {
@@ -568,29 +711,10 @@ struct tn_plan {
         if (device >= 0) {
             (void)hipSetDevice(device);
         }
-        if (stream || noalloc) {
+        if (noalloc) {
             (void)hipStreamSynchronize(stream);
-        }
-        if (hCtl && !noalloc) {
-            (void)hipHostFree(hCtl);
-        }
-        for (hipStream_t s : side) {
-            if (s) {
-                (void)hipStreamSynchronize(s);
-            }
-        }
-        for (hipEvent_t e : { ev_iter, ev_force, ev_easy, ev_rest, ev_int }) {
-            if (e) {
-                (void)hipEventDestroy(e);
-            }
-        }
-        for (hipStream_t s : side) {
-            if (s) {
-                (void)hipStreamDestroy(s);
-            }
-        }
-        if (stream) {
-            (void)hipStreamDestroy(stream);
+        } else {
+            kit_pool().give(device, kit);
         }
     }
 
@@ -685,11 +809,13 @@ struct tn_plan {
         }
         TN_HIP(hipStreamSynchronize(stream));
         timer.collect();
+        at_seeds = true;
     }
 
     // one iteration (src/v2m_particles.cpp:828-946), enqueued: the kernels, then the
     // control block's copy to the host and ev_iter behind them
     void enqueue_iteration() {
+        at_seeds = false;
         const unsigned nb = blocks_for(n, tnk::kBlock);
         hipEvent_t t = timer.begin(KC_FORCE);
         // (the junction nodes queued for the general pass, unless the move is the voxel trap's)
@@ -943,14 +1069,16 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
             p->overlap_moves = false;
             p->mem.set_arena(arena, arena_cap);
         } else {
-            TN_HIP(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));
-            TN_HIP(hipEventCreateWithFlags(&p->ev_iter, hipEventDisableTiming));
-            for (hipStream_t& s : p->side) {
-                TN_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-            }
-            for (hipEvent_t* e : { &p->ev_force, &p->ev_easy, &p->ev_rest, &p->ev_int }) {
-                TN_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
-            }
+            p->kit = kit_pool().take(dev);
+            p->stream = p->kit.stream;
+            p->side[0] = p->kit.side[0];
+            p->side[1] = p->kit.side[1];
+            p->ev_iter = p->kit.events[0];
+            p->ev_force = p->kit.events[1];
+            p->ev_easy = p->kit.events[2];
+            p->ev_rest = p->kit.events[3];
+            p->ev_int = p->kit.events[4];
+            p->hCtl = p->kit.ctl;
         }
         p->timer.stream = p->stream;
         p->timer.mask = !p->noalloc && (prm->verbose || std::getenv("TN_KERNEL_TIMING") != nullptr) ? kAllClasses : 0u;
@@ -1025,8 +1153,6 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
         p->dCtl = p->alloc<tnk::Ctl>(1);
         if (p->noalloc) {
             p->hCtl = &p->hctl_local;
-        } else {
-            TN_HIP(hipHostMalloc((void**)&p->hCtl, sizeof(tnk::Ctl), hipHostMallocDefault));
         }
         std::memset(p->hCtl, 0, sizeof(tnk::Ctl));
         float thr[tnk::kHistThr];
@@ -1789,6 +1915,7 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
     for (int k = 0; k < count; ++k) {
         plans[k]->stream = bs;
         plans[k]->overlap_moves = false;
+        plans[k]->at_seeds = false;
     }
     DevMem gm;
     gm.device = plans[0]->device;
@@ -2494,7 +2621,12 @@ int tn_plan_reset(tn_plan* p) {
 int tn_plan_run(tn_plan* p, tn_relax_stats* st) {
     return guarded([&] {
         arg_check(p != nullptr, "null plan");
-        p->reset();
+        // (a plan just created is there already; one that is timed does it again, so that its
+        // first rebuild is counted)
+        TN_HIP(hipSetDevice(p->device));
+        if (!p->at_seeds || p->timer.mask) {
+            p->reset();
+        }
         if (p->n > 0) {
             p->run_iters(p->prm.max_iters);
         }
@@ -2563,6 +2695,7 @@ int tn_plan_rebuild(tn_plan* p, int32_t* key, int32_t* sorted, int32_t* cstart, 
         TN_HIP(hipSetDevice(p->device));
         const int n = p->n;
         if (n > 0) {
+            p->at_seeds = false;
             p->rebuild();
         }
         TN_HIP(hipStreamSynchronize(p->stream));
