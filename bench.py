@@ -101,7 +101,7 @@ CLASS_KERNELS = {
     "force": ["k_force"], "move_easy": ["k_move_easy"], "move": ["k_move<1>"], "move_int": ["k_move<2>"],
     "move_rest": ["k_move<0>"], "move_def": ["k_move<0>"],
     "stats": ["k_stats"],
-    "neighbors": ["k_truss"], "refresh": ["k_truss_node"], "permute": ["k_permute"],
+    "neighbors": ["k_truss", "k_lists"], "refresh": ["k_truss_node"], "permute": ["k_permute"],
     "keys": ["k_fill_i32", "k_keys"],
     "control": ["k_control"],
 }

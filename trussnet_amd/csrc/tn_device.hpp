@@ -17,7 +17,7 @@
 // order at every rebuild; id[t] is the node's index in the caller's arrays):
 //   X[t]    float4 (x, y, z, h at the node)  -- positions and sizes, one load per gather
 //   typ[t]  u8, lab[t] u16, part[t] u32 (partner b | partner c << 16)
-//   nbrT[k*n + t]  int32 slots, list-position-major K lists (coalesced), nnb[t] int32
+//   nbr[t*K + k]  int32 slots, a node's K list in one row of 96 bytes, nnb[t] int32
 //   Ps[t]   float4 positions and sizes as of the last rebuild (the search's candidates)
 #pragma once
 
@@ -69,6 +69,7 @@ struct Hash {
     int off[TN_MAXLEV];
     int nkeys;
     int prune;   // every node's reach fits its level's cell: the K-nearest search may skip far cells
+    float hbig;  // the largest h
 };
 
 // x / v for the voxel sizes: when they are powers of two, x * (1 / v) is the same
@@ -1230,8 +1231,8 @@ struct TrussIn {
 // v2m_force, src/opencl/v2m_particle_body.cl:161-184: the repulsive bars of node i,
 // summed in list order (the fixed order that makes the sum reproducible)
 __device__ __forceinline__ float4 bar_force(const float4* __restrict__ X, const uint8_t* __restrict__ typ,
-                                            const int32_t* __restrict__ nbrT, const int32_t* __restrict__ nnb,
-                                            float fscale, float fsurf, int i, int n_nodes) {
+                                            const int32_t* __restrict__ nbr, const int32_t* __restrict__ nnb,
+                                            float fscale, float fsurf, int i) {
     const float4 xi = X[i];
     const float px = xi.x, py = xi.y, pz = xi.z, hi = xi.w;
     const int ti = typ[i];
@@ -1243,9 +1244,14 @@ __device__ __forceinline__ float4 bar_force(const float4* __restrict__ X, const 
     constexpr int kB = 8;
     static_assert(TN_K % kB == 0, "the list length is a multiple of the batch");
     int jl[TN_K];
+    const int4* row = reinterpret_cast<const int4*>(nbr + (size_t)i * TN_K);
 #pragma unroll
-    for (int u = 0; u < TN_K; ++u) {
-        jl[u] = u < m ? nbrT[(size_t)u * n_nodes + i] : i;
+    for (int u = 0; u < TN_K; u += 4) {
+        const int4 j4 = row[u / 4];
+        jl[u] = u < m ? j4.x : i;
+        jl[u + 1] = u + 1 < m ? j4.y : i;
+        jl[u + 2] = u + 2 < m ? j4.z : i;
+        jl[u + 3] = u + 3 < m ? j4.w : i;
     }
 #pragma unroll
     for (int k0 = 0; k0 < TN_K; k0 += kB) {

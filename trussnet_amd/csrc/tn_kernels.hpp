@@ -1,12 +1,12 @@
 // tn_kernels.hpp -- the relaxation's gfx950 kernels.
 //
 // Rebuild (src/v2m_particles.cpp:771-820): k_keys (cell key + count per cell),
-// k_scan_* (exclusive scan: cell starts), k_radix_* (stable LSD radix sort of the
-// nodes by cell key), k_permute (the nodes renumbered in cell order), k_truss
-// (K-nearest lists, one wave per 64 nodes).
+// k_scan_* (exclusive scan: cell starts), k_place and k_permute (the nodes renumbered in
+// cell order), k_brick_count and k_brick_order (the order of the searches), k_truss (each
+// node's candidates, one wave per 64 nodes), k_lists (the K nearest of them in order).
 // Iteration (src/v2m_particles.cpp:828-947): k_force, k_move_easy + k_move,
 // k_stats (histogram, max, Verlet count, refresh flags, FIRE power partial sums),
-// k_refresh_list + k_truss_node (own-list refresh of the nodes past a full skin),
+// k_truss_node (own-list refresh of the nodes past a full skin, which k_stats lists),
 // k_control (one block: FIRE's update, p99, the stop and rebuild decisions).
 //
 // Node slots: at every rebuild the nodes are renumbered in cell order (slot t holds
@@ -503,9 +503,9 @@ __global__ __launch_bounds__(kBlock) void k_permute(const int32_t* __restrict__ 
 // candidates in full chunks of 64 staged in LDS: a distance prefilter on the
 // matrix cores, then for every possible hit of a lane that scans the candidate's
 // row the reference's exact test and its other checks (not the node itself, no
-// interior bar across labels). Valid candidates are appended as (distance, id) to
-// the lane's LDS buffer, which is cut back to its 24 best when it fills; at the end
-// the first 24 in (distance, id) order are kept. The list equals the reference's:
+// interior bar across labels): in k_lists, or here once a buffer fills, which is then cut
+// back to its 24 best. k_lists keeps the first 24 in (distance, id) order. The list equals
+// the reference's:
 // its K smallest valid candidates in (distance, id) order, and every valid
 // candidate lies inside the lane's own box, which the union contains. (That holds
 // when every node's reach fits its level's cell, H.prune; otherwise a lane also
@@ -514,6 +514,8 @@ __global__ __launch_bounds__(kBlock) void k_permute(const int32_t* __restrict__ 
 
 constexpr int kTrussWave = 64;   // one wave per block
 constexpr int kCollect = 32;   // per-lane candidate buffer (entries): settled by a 32-key network
+// waves a SIMD: 160 registers and no spill (at 4, 128 registers, 2.5 M nodes took longer)
+constexpr int kTrussOcc = 3;
 constexpr int kMinRoom = 4;    // a lane with less room than this (and more possible hits) settles first
 
 // ---- wave-wide reductions and scans on DPP (64 lanes, all active) ----------------
@@ -582,20 +584,25 @@ __device__ __forceinline__ uint64_t list_key(float d, int id) {
     return ((uint64_t)__float_as_uint(d) << 32) | (uint32_t)id;
 }
 
-// Sort 32 keys in registers: a bitonic network, every index known at compile time.
-__device__ __forceinline__ void bitonic32(uint64_t (&k)[32]) {
+// Sort N <= 32 keys in registers: Batcher's odd-even merge network for 32, less the
+// comparators that reach past N (K. E. Batcher, Sorting networks and their applications,
+// AFIPS 1968), every index known at compile time (24: 132 comparators, 32: 191).
+template <int N>
+__device__ __forceinline__ void merge_sort(uint64_t (&k)[32]) {
+    static_assert(N <= 32, "the network is for 32 keys");
 #pragma unroll
-    for (int size = 2; size <= 32; size <<= 1) {
+    for (int p = 1; p < 32; p <<= 1) {
 #pragma unroll
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+        for (int d = p; d > 0; d >>= 1) {
 #pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const int j = i ^ stride;
-                if (j > i) {
-                    const uint64_t x = k[i], y = k[j];
-                    const bool swap = (i & size) == 0 ? x > y : x < y;
+            for (int i = 0; i + d < N; ++i) {
+                // (i, i + d) is a comparator: i in the first half of its pair of runs of d
+                // (offset by d % p), both in one block of 2 p
+                if (i >= d % p && ((i - d % p) / d) % 2 == 0 && i / (2 * p) == (i + d) / (2 * p)) {
+                    const uint64_t x = k[i], y = k[i + d];
+                    const bool swap = x > y;
                     k[i] = swap ? y : x;
-                    k[j] = swap ? x : y;
+                    k[i + d] = swap ? x : y;
                 }
             }
         }
@@ -691,55 +698,74 @@ __device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
     return ((uint64_t)hi << 32) | lo;
 }
 
-// A slot buffer's entry e of lane `who` as its key, recomputed from the candidate's
-// position as the test formed it: (distance from the query at (x, y, z), id).
-__device__ __forceinline__ uint64_t slot_key(const float4* __restrict__ Ps, const int2* __restrict__ Ms, int slot,
-                                             float x, float y, float z) {
-    const float4 c = Ps[slot];
-    const float ex = c.x - x, ey = c.y - y, ez = c.z - z;
-    const float d2 = ex * ex + ey * ey + ez * ez;
-    return list_key(sqrtf(d2), Ms[slot].x);
-}
-
 __device__ __forceinline__ float readlane_f(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// Cut the slot buffers of the lanes in sm (wave-uniform) back to their 24 best (in
-// order); their cnt becomes 24 and kth the 24th key. All lanes take part: the keys are
-// recomputed from the slots, relative to the owner's query (px, py, pz).
+// A wave's queries, lane by lane (the search's view of its 64 nodes).
+struct WaveQueries {
+    float px, py, pz, h;   // position and size
+    int slot;
+};
+
+// Cut the slot buffers of the lanes in sm (wave-uniform) back to their best 24 bars (in
+// order); their cnt becomes the bars left and kth the 24th key when there are 24. All
+// lanes take part: the exact test and the keys are formed from the slots, relative to the
+// owner's query.
 __device__ __forceinline__ void settle_slot_lanes(uint32_t* cb, int lane, uint64_t sm, int& cnt, uint64_t& kth,
                                                   const float4* __restrict__ Ps, const int2* __restrict__ Ms,
-                                                  float px, float py, float pz) {
-    while (sm) {
-        const int a = __builtin_ctzll(sm);
+                                                  const WaveQueries& Q, float half) {
+    // the pair of lanes settled next, with its entries already on their way while the pair
+    // before it is sorted (a wave of stacked nodes settles a hundred times in a row)
+    const bool lo = lane < 32;
+    const int i = lane & 31;
+    int a = 0, b = 0, sl = 0, id = 0;
+    bool in = false;
+    float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    auto next = [&]() {
+        a = __builtin_ctzll(sm);
         sm &= sm - 1;
-        const int b = sm ? __builtin_ctzll(sm) : a;
+        b = sm ? __builtin_ctzll(sm) : a;
         sm &= sm ? sm - 1 : 0ull;
         const int ca = __builtin_amdgcn_readlane(cnt, a), cb_n = __builtin_amdgcn_readlane(cnt, b);
-        const float xa = readlane_f(px, a), ya = readlane_f(py, a), za = readlane_f(pz, a);
-        const float xb = readlane_f(px, b), yb = readlane_f(py, b), zb = readlane_f(pz, b);
-        const bool lo = lane < 32;
-        const int who = lo ? a : b, cw = lo ? ca : cb_n;
-        const int i = lane & 31;
-        int sl = 0;
-        uint64_t v = ~0ull;
-        if (i < cw) {
-            sl = (int)cb[i * kTrussWave + who];
-            v = slot_key(Ps, Ms, sl, lo ? xa : xb, lo ? ya : yb, lo ? za : zb);
+        in = i < (lo ? ca : cb_n);
+        sl = in ? (int)cb[i * kTrussWave + (lo ? a : b)] : 0;
+        c = Ps[sl];
+        id = Ms[sl].x;
+    };
+    next();
+    for (;;) {
+        const int a0 = a, b0 = b;
+        const float xa = readlane_f(Q.px, a), ya = readlane_f(Q.py, a), za = readlane_f(Q.pz, a), ha = readlane_f(Q.h, a);
+        const float xb = readlane_f(Q.px, b), yb = readlane_f(Q.py, b), zb = readlane_f(Q.pz, b), hb = readlane_f(Q.h, b);
+        const int qa = __builtin_amdgcn_readlane(Q.slot, a), qb = __builtin_amdgcn_readlane(Q.slot, b);
+        const float ex = c.x - (lo ? xa : xb), ey = c.y - (lo ? ya : yb), ez = c.z - (lo ? za : zb);
+        const float d2 = ex * ex + ey * ey + ez * ez;
+        const float rj = half * ((lo ? ha : hb) + c.w);
+        const bool bar = in && d2 < rj * rj && sl != (lo ? qa : qb);
+        uint64_t v = bar ? list_key(sqrtf(d2), id) : ~0ull;
+        int slot = sl;
+        const bool more = sm != 0;
+        if (more) {   // (of other lanes than a0 and b0: their columns are not written below)
+            next();
         }
-        half_wave_sort32_kv(v, sl, lane);
+        half_wave_sort32_kv(v, slot, lane);
         if (i < kK) {
-            cb[i * kTrussWave + who] = (uint32_t)sl;
+            cb[i * kTrussWave + (lo ? a0 : b0)] = (uint32_t)slot;
         }
+        const uint64_t bars = __ballot(v != ~0ull);
+        const int na = __popcll(bars & 0xFFFFFFFFull), nb = __popcll(bars >> 32);
         const uint64_t ka = readlane64(v, kK - 1), kb = readlane64(v, 32 + kK - 1);
-        if (lane == a) {
-            cnt = kK;
+        if (lane == a0) {
+            cnt = min(na, kK);
             kth = ka;
         }
-        if (lane == b) {
-            cnt = kK;
+        if (lane == b0) {
+            cnt = min(nb, kK);
             kth = kb;
+        }
+        if (!more) {
+            break;
         }
     }
 }
@@ -759,89 +785,134 @@ __device__ __forceinline__ void settle_slot_lanes(uint32_t* cb, int lane, uint64
 // its output register e holds D[8 (e / 4) + 4 (l / 32) + e % 4][l % 32]. So in the
 // tile of its own query's columns a lane holds half of the tile's candidate rows
 // for its query, and lane l ^ 32 holds the other half.)
+//
+// Around the twelve matrix operations a chunk costs few others. The accumulators start at
+// minus the margin, so that a possible hit is a sign bit, taken into the mask with one
+// funnel shift each. Lane l holds candidate chunk_index(l), the one whose row makes the 16
+// mask bits of either half of the wave 16 consecutive candidates. Operands and masks change
+// halves with v_permlane32_swap. (With compares and selects a bit, the operands formed
+// twice from LDS and the masks spread nibble by nibble, a chunk took about 450 vector
+// instructions instead of 190.)
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+// the candidate of the chunk that lane l holds, the lane that holds candidate k, and a
+// mask of lanes as one of candidates (bits 2, 3 and 4 of the index change places)
+__device__ __forceinline__ int chunk_index(int lane) {
+    return (lane & 0x23) | ((lane & 4) << 2) | ((lane & 0x18) >> 1);
+}
+__device__ __forceinline__ int chunk_lane(int k) {
+    return (k & 0x23) | ((k & 0x0C) << 1) | ((k & 0x10) >> 2);
+}
+__device__ __forceinline__ uint64_t by_index(uint64_t lanes) {
+    // nibbles 8 a + 4 hh of each half to 4 a + 16 hh: even ones below, odd ones above
+    const uint64_t lo = lanes & 0x0F0F0F0F0F0F0F0Full, hi = (lanes >> 4) & 0x0F0F0F0F0F0F0F0Full;
+    auto pack = [](uint64_t x) {   // the low nibble of each byte, packed within each half
+        x = (x | (x >> 4)) & 0x00FF00FF00FF00FFull;
+        return (x | (x >> 8)) & 0x0000FFFF0000FFFFull;
+    };
+    return pack(lo) | (pack(hi) << 16);
+}
+
+// lanes 32..63 of a and lanes 0..31 of b exchanged
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
 
 // this lane's B operands: queries 32 c + l % 32 (c = the column tile), three K-steps
 struct QueryOps {
     float b[2][3];
 };
 
-__device__ __forceinline__ QueryOps query_ops(float qx, float qy, float qz, float h, float Aq, int lane) {
-    const bool up = lane >= 32;
+// the six components of a lane's query, K-index 2 t + l / 32: (k0, k1), (k2, k3), (k4, k5)
+__device__ __forceinline__ QueryOps query_ops(float k0, float k1, float k2, float k3, float k4, float k5) {
     QueryOps o;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int src = 32 * c + (lane & 31);
-        const float x = __shfl(qx, src, kWave), y = __shfl(qy, src, kWave), z = __shfl(qz, src, kWave);
-        const float hh = __shfl(h, src, kWave), A = __shfl(Aq, src, kWave);
-        // K-index 2 t + l / 32: (x, y), (z, h), (|p|^2 - k^2 h^2, 1)
-        o.b[c][0] = up ? y : x;
-        o.b[c][1] = up ? hh : z;
-        o.b[c][2] = up ? 1.0f : A;
-    }
+    swap_halves(k0, k1);
+    swap_halves(k2, k3);
+    swap_halves(k4, k5);
+    o.b[0][0] = k0;
+    o.b[1][0] = k1;
+    o.b[0][1] = k2;
+    o.b[1][1] = k3;
+    o.b[0][2] = k4;
+    o.b[1][2] = k5;
     return o;
 }
 
-// The tests of one output tile, dense: bit e for register e (its difference below the
-// margin). Plain compares, so that the compiler keeps the wait states the matrix
-// cores' results need before a vector instruction may read them.
-__device__ __forceinline__ uint32_t tile_bits(const f32x16& acc, float margin) {
+// the signs of one output tile: bit e for register e
+__device__ __forceinline__ uint32_t tile_signs(const f32x16& acc) {
     uint32_t m = 0;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        m |= (acc[e] < margin ? 1u : 0u) << e;
+    for (int e = 15; e >= 0; --e) {   // (m << 1) | sign
+        m = __builtin_amdgcn_alignbit(m, __float_as_uint(acc[e]), 31);
     }
     return m;
 }
 
-// the 16 bits of a dense tile mask spread to nibbles at bits 8 k .. 8 k + 3
-__device__ __forceinline__ uint32_t spread_nibbles(uint32_t d) {
-    uint32_t x = d & 0xFFFFu;
-    x = (x | (x << 8)) & 0x00FF00FFu;
-    return (x | (x << 4)) & 0x0F0F0F0Fu;
-}
-
-// the 64-bit mask of this lane's query over the chunk's candidates (cpos) whose
-// difference, relative to the origin o, is below `margin`
-__device__ __forceinline__ uint64_t chunk_hits(const QueryOps& qo, const float4* cpos, float ox, float oy, float oz,
-                                               float k2, float margin, int lane) {
-    const bool up = lane >= 32;
-    const int h = lane >> 5;
+// The 64-bit mask of this lane's query over the chunk's candidates whose dot product is
+// below the margin, from lane l's operands of candidate chunk_index(l) (K-index 2 t and
+// 2 t + 1 in a_t[0] and a_t[1])
+__device__ __forceinline__ uint64_t tiles_below(const QueryOps& qo, float (&a0)[2], float (&a1)[2], float (&a2)[2],
+                                                float margin) {
+    swap_halves(a0[0], a0[1]);   // [r]: candidates of lanes 32 r .. 32 r + 31
+    swap_halves(a1[0], a1[1]);
+    swap_halves(a2[0], a2[1]);
+    f32x16 start;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        start[e] = -margin;
+    }
     uint32_t out[2];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {   // candidates 32 r .. 32 r + 31 (the row tile)
-        const float4 v = cpos[32 * r + (lane & 31)];
-        float a0, a1, a2;
-        if (v.x < __builtin_huge_valf()) {
-            const float cx = v.x - ox, cy = v.y - oy, cz = v.z - oz;
-            const float C = cx * cx + cy * cy + cz * cz - k2 * v.w * v.w;
-            // K-index 2 t + l / 32: (-2 cx, -2 cy), (-2 cz, -2 k^2 h), (1, |c|^2 - k^2 h^2)
-            a0 = up ? -2.0f * cy : -2.0f * cx;
-            a1 = up ? -2.0f * k2 * v.w : -2.0f * cz;
-            a2 = up ? C : 1.0f;
-        } else {   // past the row's end: a difference far above any margin
-            a0 = 0.0f;
-            a1 = 0.0f;
-            a2 = up ? 1e30f : 0.0f;
-        }
+    for (int r = 0; r < 2; ++r) {   // the row tile
         uint32_t bits[2];
 #pragma unroll
         for (int c = 0; c < 2; ++c) {   // queries 32 c .. 32 c + 31 (the column tile)
-            f32x16 acc = {};
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, qo.b[c][0], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, qo.b[c][1], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a2, qo.b[c][2], acc, 0, 0, 0);
-            bits[c] = tile_bits(acc, margin);
+            f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[r], qo.b[c][0], start, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[r], qo.b[c][1], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[r], qo.b[c][2], acc, 0, 0, 0);
+            bits[c] = tile_signs(acc);
         }
-        // my query's column tile is h: register e of lane l holds candidate
-        // 8 (e / 4) + 4 (l / 32) + e % 4 of the row tile; lane l ^ 32 has the other half
-        const uint32_t mine = h ? bits[1] : bits[0], give = h ? bits[0] : bits[1];
-        const uint32_t got = (uint32_t)__shfl_xor((int)give, 32, kWave);
-        out[r] = (spread_nibbles(mine) << (4 * h)) | (spread_nibbles(got) << (4 * (1 - h)));
+        // a lane's own column tile is l / 32: candidates 0..15 of the row tile from the lower
+        // half's registers, 16..31 from the upper half's
+        const auto x = __builtin_amdgcn_permlane32_swap(bits[0], bits[1], false, false);
+        out[r] = x[0] | (x[1] << 16);
     }
     return ((uint64_t)out[1] << 32) | out[0];
+}
+
+// the 64-bit mask of this lane's query over the chunk's candidates (lane l's own:
+// candidate chunk_index(l), at v) whose difference, relative to the origin o, is below
+// the margin
+__device__ __forceinline__ uint64_t chunk_hits(const QueryOps& qo, float4 v, float ox, float oy, float oz, float k2,
+                                               float margin) {
+    const bool some = v.x < __builtin_huge_valf();
+    const float cx = v.x - ox, cy = v.y - oy, cz = v.z - oz;
+    const float C = cx * cx + cy * cy + cz * cz - k2 * v.w * v.w;
+    // K-index 2 t + l / 32: (-2 cx, -2 cy), (-2 cz, -2 k^2 h), (1, |c|^2 - k^2 h^2); past the
+    // chunk's end a difference far above any margin
+    float a0[2] = { some ? -2.0f * cx : 0.0f, some ? -2.0f * cy : 0.0f };
+    float a1[2] = { some ? -2.0f * cz : 0.0f, some ? -2.0f * k2 * v.w : 0.0f };
+    float a2[2] = { some ? 1.0f : 0.0f, some ? C : 1e30f };
+    return tiles_below(qo, a0, a1, a2, margin);
+}
+
+// The same for d^2 < near^2, near: this lane's 24th best distance so far. The terms of d^2 -
+// near^2 are (-2c, 1, |c|^2) . (p, |p|^2 - near^2, 1), so it takes the same three steps. A
+// wave of stacked nodes meets hundreds of possible bars a node of which a tenth comes
+// before the node's 24th: only those are then tested one by one (495 k nodes moved in the
+// voxel field, 48 rebuilds: k_truss and k_lists 3.02 -> 2.40 ms a rebuild).
+__device__ __forceinline__ uint64_t chunk_near(float qx, float qy, float qz, float near2, float4 v, float ox, float oy,
+                                               float oz, float margin) {
+    const bool some = v.x < __builtin_huge_valf();
+    const float cx = v.x - ox, cy = v.y - oy, cz = v.z - oz;
+    const QueryOps qo = query_ops(qx, qy, qz, qx * qx + qy * qy + qz * qz - near2, 1.0f, 0.0f);
+    float a0[2] = { some ? -2.0f * cx : 0.0f, some ? -2.0f * cy : 0.0f };
+    float a1[2] = { some ? -2.0f * cz : 0.0f, some ? 1.0f : 0.0f };
+    float a2[2] = { some ? cx * cx + cy * cy + cz * cz : 1e35f, 0.0f };
+    return tiles_below(qo, a0, a1, a2, margin);
 }
 
 // The rows of one group, collected before any of their candidates is loaded: the
@@ -851,13 +922,19 @@ constexpr int kMaxRanges = 64;
 
 
 // The lists of all nodes at a rebuild: query q is the node in slot q. The buffers hold
-// the candidates' slots (4 bytes) and the keys are recomputed from them when a buffer
-// is cut back and at the end: 12 KB of LDS a wave (instead of 20 KB with the keys
-// themselves), so that 12 waves fit a CU.
-__global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int n, int32_t* __restrict__ nbrT,
-                                                         int32_t* __restrict__ nnb) {
+// the candidates' slots (4 bytes): 12 KB of LDS a wave, so that 13 waves fit a CU. While
+// no buffer of the wave has filled, every possible hit is appended as it is (93 of 100
+// are bars) and the exact test is left to k_lists, which forms the distances anyway: a few
+// instructions a hit, each lane its own. From the first full buffer on (nodes that stack
+// up on the voxel faces, and the grids with no reach bound) a wave tests its possible hits
+// as (query, candidate) pairs, one a lane, and takes in only what beats its query's 24th
+// best so far. Rows of up to 32 slots leave the kernel: 24 in the list's own row, the rest
+// in tail0 and tail1.
+__global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn in, int n, int32_t* __restrict__ nbr,
+                                                                      int4* __restrict__ tail0, int4* __restrict__ tail1,
+                                                                      int32_t* __restrict__ nnb) {
     __shared__ float4 cpos[kTrussWave];   // the chunk's candidates: position, h
-    __shared__ int2 cms[kTrussWave];      // their (id, typ | lab << 8)
+    __shared__ int cid[kTrussWave];       // their ids
     __shared__ int crow[kTrussWave];      // their row (index into the row table)
     // the row table of the current group: cell-start indices of the row's first cell and
     // one past its last, the lanes that scan the row, its level; after the cell starts
@@ -875,11 +952,12 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
     const float half = tskin * 0.5f;   // (t + skin) * 0.5f * (hi + hj), left to right
     const float k2 = half * half;
     const float inf = __builtin_huge_valf();
+    const int cidx = chunk_index(lane);
     for (int qb = blockIdx.x * kTrussWave; qb < n; qb += gridDim.x * kTrussWave) {
         const bool active = qb + lane < n;
         const int q = active ? in.order[qb + lane] : 0;   // the node in slot q
         float px = 0.0f, py = 0.0f, pz = 0.0f, hi = 0.0f, Ri = 0.0f;
-        int Li = 0, ti_int = 0, li = 0, myid = -1;
+        int Li = 0, ti_int = 0, li = 0;
         if (active) {   // the node in slot q (nodes are in cell order)
             const float4 xi = in.X[q];
             px = xi.x;
@@ -889,7 +967,6 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
             Ri = tskin * hi;
             Li = level_for(H, Ri);
             const int2 mi = in.Ms[q];
-            myid = mi.x;
             ti_int = (mi.y & 0xFF) == TN_INTERIOR;
             li = mi.y >> 8;
         }
@@ -907,6 +984,9 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
         // the 24th of them, and a candidate must come before it to enter.
         int cnt = 0;
         uint64_t kth = ~0ull;
+        bool near = false;   // (wave-uniform: some lane has 24 bars, and kth bounds what it still takes)
+        bool cut = !H.prune;   // (wave-uniform: some lane's buffer has been, or the pairs are needed anyway)
+        const WaveQueries Q{ px, py, pz, hi, q };
         for (;;) {
             const uint64_t pm = __ballot(pending);
             if (!pm) {
@@ -920,8 +1000,14 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
             const float gox = __shfl(px, lead, kWave), goy = __shfl(py, lead, kWave), goz = __shfl(pz, lead, kWave);
             const float qx = px - gox, qy = py - goy, qz = pz - goz;
             const float q2 = qx * qx + qy * qy + qz * qz;
-            const QueryOps qops = query_ops(qx, qy, qz, hi, q2 - k2 * hi * hi, lane);
+            const QueryOps qops = query_ops(qx, qy, qz, hi, q2 - k2 * hi * hi, 1.0f);
             const float P2 = wave_max_nonneg(ingroup ? q2 : 0.0f), HP = wave_max_nonneg(ingroup ? hi : 0.0f);
+            // The prefilter's margin, 2^-16 of a bound S on the terms of a true hit's difference:
+            // its candidate lies within the bar's reach of the query, so |c| <= |p| + k (h_p +
+            // h_c), and h_c is at most the grid's largest h. (A candidate farther off may be
+            // misjudged either way: it is no hit, and the exact test says so.)
+            const float hs = HP + H.hbig, Cmax = sqrtf(P2) + half * hs;
+            const float margin = (2.0f * (P2 + Cmax * Cmax) + 2.0f * k2 * hs * hs) * (1.0f / 65536.0f);
             int nr = 0;   // rows in the table (wave-uniform)
             // Read the cell starts of the table's rows, then test the concatenation of their
             // candidates chunk by chunk: the distance prefilter on the matrix cores, then the
@@ -953,7 +1039,7 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
                     while (rfirst + 1 < rows && r_beg[rfirst + 1] <= base) {
                         ++rfirst;
                     }
-                    const int p = base + lane;
+                    const int p = base + cidx;
                     int lo = rfirst;   // the candidate's row: the last that starts at or before p
                     if (p < total) {
                         while (lo + 1 < rows && r_beg[lo + 1] <= p) {
@@ -973,37 +1059,67 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
                 fetch(0);
                 for (int base = 0; base < total; base += kTrussWave) {
                     __syncthreads();   // the previous chunk is consumed
-                    cpos[lane] = npos;
-                    cms[lane] = nms;
-                    crow[lane] = nrow;
-                    cslot[lane] = nslot;
-                    const int lo = nrow;
+                    cslot[cidx] = nslot;
+                    const float4 mine_c = npos;
+                    const int2 mine_m = nms;
+                    if (cut) {
+                        cpos[cidx] = npos;
+                        cid[cidx] = nms.x;
+                        crow[cidx] = nrow;
+                    }
+                    const int mine_row = nrow;
                     __syncthreads();
                     if (base + kTrussWave < total) {
                         fetch(base + kTrussWave);
                     }
-                    const int cn = min(kTrussWave, total - base);
-                    // the chunk's own bound for the rounding margin
-                    const float4 mine_c = cpos[lane];
-                    const bool cval = mine_c.x < inf;
-                    const float ccx = mine_c.x - gox, ccy = mine_c.y - goy, ccz = mine_c.z - goz;
-                    const float C2 = wave_max_nonneg(cval ? ccx * ccx + ccy * ccy + ccz * ccz : 0.0f);
-                    const float HC = wave_max_nonneg(cval ? mine_c.w : 0.0f);
-                    const float hs = HP + HC;
-                    const float margin = (2.0f * (P2 + C2) + 2.0f * k2 * hs * hs) * (1.0f / 65536.0f);
-                    uint64_t hit = chunk_hits(qops, cpos, gox, goy, goz, k2, margin, lane);
-                    // the candidates of the rows this lane scans (its level range, its own box)
-                    uint64_t elig = 0;
-                    {
-                        const int r0 = __shfl(lo, 0, kWave), r1 = __shfl(lo, cn - 1, kWave);
+                    uint64_t hit = chunk_hits(qops, mine_c, gox, goy, goz, k2, margin);
+                    if (!H.prune) {
+                        // the candidates of the rows this lane scans (its level range, its own
+                        // box); where every reach fits its level's cell, a candidate that passes
+                        // the exact test is in the lane's own box without being asked
+                        const int cn = min(kTrussWave, total - base);
+                        uint64_t elig = 0;
+                        const int r0 = crow[0], r1 = crow[cn - 1];
                         for (int r = r0; r <= r1; ++r) {
                             const int a = max(r_beg[r] - base, 0), b = min(r_beg[r] + r_len[r] - base, cn);
                             if (b > a && ((r_mask[r] >> lane) & 1ull)) {
                                 elig |= (b - a == kTrussWave ? ~0ull : ((1ull << (b - a)) - 1)) << a;
                             }
                         }
+                        hit &= elig;
                     }
-                    hit = ingroup ? hit & elig : 0ull;
+                    hit = ingroup ? hit : 0ull;
+                    {   // no bar between interior nodes of two labels
+                        const bool inside = (mine_m.y & 0xFF) == TN_INTERIOR;
+                        const int cl = mine_m.y >> 8;
+                        uint64_t left = by_index(__ballot(inside && mine_m.x >= 0));
+                        while (left) {   // the labels of the chunk's interior candidates (mostly one)
+                            const int l = __builtin_amdgcn_readlane(cl, chunk_lane(__builtin_ctzll(left)));
+                            const uint64_t of = by_index(__ballot(inside && cl == l));
+                            hit = ti_int && li != l ? hit & ~of : hit;
+                            left &= ~of;
+                        }
+                    }
+                    if (near) {
+                        const float dk = kth == ~0ull ? 1e15f : __uint_as_float((uint32_t)(kth >> 32));
+                        hit &= chunk_near(qx, qy, qz, dk * dk, mine_c, gox, goy, goz, margin);
+                    }
+                    if (!cut && __ballot(cnt + __popcll(hit) > kCollect)) {   // a buffer fills
+                        cut = true;
+                        cpos[cidx] = mine_c;
+                        cid[cidx] = mine_m.x;
+                        crow[cidx] = mine_row;
+                        __syncthreads();
+                    }
+                    if (!cut) {
+                        while (hit) {   // (each lane its own)
+                            const int k = __builtin_ctzll(hit);
+                            hit &= hit - 1;
+                            cb[cnt * kTrussWave + lane] = (uint32_t)cslot[k];
+                            ++cnt;
+                        }
+                        continue;
+                    }
                     // The possible hits as (query lane, candidate) pairs, up to 64 a round, one
                     // a lane: the exact test and the reference's other checks, and the valid
                     // ones appended to their query's buffer, packed in pair order.
@@ -1012,7 +1128,8 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
                         // little room for them: keep the 24 best so far
                         const uint64_t sm = __ballot(pc > kCollect - cnt && kCollect - cnt < kMinRoom);
                         if (sm) {
-                            settle_slot_lanes(cb, lane, sm, cnt, kth, in.Ps, in.Ms, px, py, pz);
+                            settle_slot_lanes(cb, lane, sm, cnt, kth, in.Ps, in.Ms, Q, half);
+                            near = true;
                         }
                         const int want = min(pc, kCollect - cnt);
                         int npair = 0;
@@ -1030,21 +1147,18 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
                         // the owner's query, from its lane (every lane takes part in the shuffles)
                         const float ox_ = __shfl(px, o, kWave), oy_ = __shfl(py, o, kWave);
                         const float oz_ = __shfl(pz, o, kWave), oh = __shfl(hi, o, kWave);
-                        const int oid = __shfl(myid, o, kWave), otl = __shfl(ti_int | (li << 1), o, kWave);
+                        const int oslot = __shfl(q, o, kWave);
                         const int os0 = __shfl(s0, o, kWave), ocnt = __shfl(cnt, o, kWave);
                         const uint64_t okth = __shfl(kth, o, kWave);
-                        uint64_t key = 0;
+                        int cs = 0;
                         bool valid = false;
                         if (lane < npair) {
                             const float4 c = cpos[k];
-                            const int2 mt = cms[k];
+                            cs = cslot[k];
                             const float ex = c.x - ox_, ey = c.y - oy_, ez = c.z - oz_;
                             const float d2 = ex * ex + ey * ey + ez * ez;
                             const float rj = half * (oh + c.w);
-                            valid = d2 < rj * rj;
-                            // not the node itself; no interior bar across labels
-                            valid = valid && mt.x != oid &&
-                                    !((otl & 1) && (mt.y & 0xFF) == TN_INTERIOR && (mt.y >> 8) != (otl >> 1));
+                            valid = d2 < rj * rj && cs != oslot;   // a bar, and not the node itself
                             if (valid && !H.prune) {   // the reference's own scan region only
                                 const int L = r_lev[crow[k]];
                                 const float rr = 0.5f * (tskin * oh + H.b0 * (float)(1 << L));
@@ -1052,15 +1166,14 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
                                 valid = cx >= cell_coord(H, L, ox_ - rr, H.ox, 0) &&
                                         cx <= cell_coord(H, L, ox_ + rr, H.ox, 0);
                             }
-                            key = list_key(sqrtf(d2), mt.x);
-                            valid = valid && key < okth;
+                            valid = valid && list_key(sqrtf(d2), cid[k]) < okth;
                         }
                         const uint64_t vm = __ballot(valid);
                         // the owner's pairs are [s0, s0 + take) of its round: a valid pair's place is
                         // the owner's count plus the valid pairs of the owner before it
                         if (valid) {
                             const int at = ocnt + __popcll(vm & lanemask_lt() & ~((1ull << (os0 & 63)) - 1));
-                            cb[at * kTrussWave + o] = (uint32_t)cslot[k];
+                            cb[at * kTrussWave + o] = (uint32_t)cs;
                         }
                         if (take > 0) {
                             const uint64_t span = take == kTrussWave ? ~0ull : ((1ull << take) - 1);
@@ -1147,23 +1260,113 @@ __global__ __launch_bounds__(kTrussWave, 3) void k_truss(Hash H, TrussIn in, int
                 flush();
             }
         }   // the groups
-        if (active) {   // (distance, id) order; the list holds slots
-            uint64_t kk[32];
+        if (active) {   // in any order, the entries past the count read by nobody
+            nnb[q] = cnt;
+            int4* row = reinterpret_cast<int4*>(nbr + (size_t)q * kK);
 #pragma unroll
-            for (int e = 0; e < 32; ++e) {
-                kk[e] = e < cnt ? slot_key(in.Ps, in.Ms, (int)cb[e * kTrussWave + lane], px, py, pz) : ~0ull;
-            }
-            bitonic32(kk);
-            const int m = cnt < kK ? cnt : kK;
-            nnb[q] = m;
-#pragma unroll
-            for (int k = 0; k < kK; ++k) {
-                if (k < m) {
-                    nbrT[(size_t)k * n + q] = in.slot_of[(int)(uint32_t)kk[k]];
+            for (int e = 0; e < kCollect; e += 4) {
+                if (e < cnt) {
+                    const int4 v = make_int4((int)cb[e * kTrussWave + lane], (int)cb[(e + 1) * kTrussWave + lane],
+                                             (int)cb[(e + 2) * kTrussWave + lane], (int)cb[(e + 3) * kTrussWave + lane]);
+                    if (e < kK) {
+                        row[e / 4] = v;
+                    } else if (e == kK) {
+                        tail0[q] = v;
+                    } else {
+                        tail1[q] = v;
+                    }
                 }
             }
         }
         __syncthreads();   // the buffers are reused by the next block of queries
+    }
+}
+
+// The rows k_truss left (up to 32 slots, in any order) tested exactly and put in
+// (distance, id) order, the first 24 kept. In a launch of its own, a lane a node in slot
+// order, its rows and the neighbours' positions are read and written whole lines at a time;
+// at the end of k_truss, whose lanes hold nodes in brick order, the same work was a gather
+// of the ids, one of their slots and 24 scattered stores a node, its 64 key registers
+// bounding the search (2.5 M nodes: 2.25 ms in one kernel, 1.42 + 0.22 ms in two). The
+// keys are (distance, slot): the ids are read only in a wave where two distances tie, whose
+// lanes then sort by (distance, id) and look the slots up (neighbours exchanged until all
+// ids are in order took up to a pass a tied entry: 152 us instead of 80 for 495 k nodes in
+// the voxel field). Bound by the gathers of the positions.
+template <int N>
+__device__ __forceinline__ int sort_row(const float4* __restrict__ Ps, const int2* __restrict__ Ms, int t, int m, float4 xi,
+                                        float half, const int4* __restrict__ row, const int4* __restrict__ tail0,
+                                        const int4* __restrict__ tail1, const int32_t* __restrict__ slot_of,
+                                        uint64_t (&k)[32]) {
+    constexpr int kB = 8;
+    int s[N];
+#pragma unroll
+    for (int e = 0; e < N; e += 4) {
+        const int4 j4 = e < kK ? row[e / 4] : (e == kK ? tail0[t] : tail1[t]);
+        s[e] = e < m ? j4.x : t;
+        s[e + 1] = e + 1 < m ? j4.y : t;
+        s[e + 2] = e + 2 < m ? j4.z : t;
+        s[e + 3] = e + 3 < m ? j4.w : t;
+    }
+#pragma unroll
+    for (int e0 = 0; e0 < N; e0 += kB) {
+        float4 x[kB];
+#pragma unroll
+        for (int e = 0; e < kB; ++e) {
+            x[e] = Ps[s[e0 + e]];
+        }
+#pragma unroll
+        for (int e = 0; e < kB; ++e) {   // the reference's test (an entry past the row's end is the node itself)
+            const float ex = x[e].x - xi.x, ey = x[e].y - xi.y, ez = x[e].z - xi.z;
+            const float d2 = ex * ex + ey * ey + ez * ez;
+            const float rj = half * (xi.w + x[e].w);
+            const bool bar = d2 < rj * rj && s[e0 + e] != t;
+            k[e0 + e] = bar ? list_key(sqrtf(d2), s[e0 + e]) : ~0ull;
+        }
+    }
+    merge_sort<N>(k);
+    int bars = 0;
+    bool tie = false;
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+        bars += k[e] != ~0ull ? 1 : 0;
+        if (e > 0) {
+            tie = tie || (k[e] != ~0ull && (k[e - 1] >> 32) == (k[e] >> 32));
+        }
+    }
+    if (__ballot(tie)) {   // by (distance, id) then, and the slots looked up
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            k[e] = k[e] != ~0ull ? (k[e] >> 32) << 32 | (uint32_t)Ms[(int)(uint32_t)k[e]].x : ~0ull;
+        }
+        merge_sort<N>(k);
+#pragma unroll
+        for (int e = 0; e < kK; ++e) {
+            k[e] = k[e] != ~0ull ? (uint32_t)slot_of[(int)(uint32_t)k[e]] : 0ull;
+        }
+    }
+    return bars < kK ? bars : kK;
+}
+
+__global__ __launch_bounds__(kBlock) void k_lists(const float4* __restrict__ Ps, const int2* __restrict__ Ms, int n,
+                                                  float half, int32_t* __restrict__ nbr, const int4* __restrict__ tail0,
+                                                  const int4* __restrict__ tail1, const int32_t* __restrict__ slot_of,
+                                                  int32_t* __restrict__ nnb) {
+    const int g = blockIdx.x * kBlock + threadIdx.x;
+    const bool valid = g < n;
+    const int t = valid ? g : 0;
+    const int m = valid ? nnb[t] : 0;
+    int4* row = reinterpret_cast<int4*>(nbr + (size_t)t * kK);
+    const float4 xi = Ps[t];
+    uint64_t k[32];
+    const int bars = __ballot(m > kK) ? sort_row<32>(Ps, Ms, t, m, xi, half, row, tail0, tail1, slot_of, k)
+                                      : sort_row<kK>(Ps, Ms, t, m, xi, half, row, tail0, tail1, slot_of, k);
+    if (valid) {
+        nnb[t] = bars;
+#pragma unroll
+        for (int e = 0; e < kK; e += 4) {
+            row[e / 4] = make_int4((int)(uint32_t)k[e], (int)(uint32_t)k[e + 1], (int)(uint32_t)k[e + 2],
+                                   (int)(uint32_t)k[e + 3]);
+        }
     }
 }
 
@@ -1212,7 +1415,7 @@ __device__ __forceinline__ int keep_best(float* cd, int* cj, int cnt, int lane) 
     return cnt < kK ? cnt : kK;
 }
 
-__device__ __forceinline__ void k_truss_node_body(Hash H, TrussIn in, int n, const int32_t* __restrict__ list, const Ctl* __restrict__ ctl, int32_t* __restrict__ nbrT, int32_t* __restrict__ nnb, float4* __restrict__ P0, int bid, int nblk) {
+__device__ __forceinline__ void k_truss_node_body(Hash H, TrussIn in, int n, const int32_t* __restrict__ list, const Ctl* __restrict__ ctl, int32_t* __restrict__ nbr, int32_t* __restrict__ nnb, float4* __restrict__ P0, int bid, int nblk) {
     __shared__ float cd[kRefreshCap];
     __shared__ int cj[kRefreshCap];
     const int lane = threadIdx.x;
@@ -1298,7 +1501,7 @@ __device__ __forceinline__ void k_truss_node_body(Hash H, TrussIn in, int n, con
         __syncthreads();   // the appends are visible to every lane
         const int kk = keep_best(cd, cj, cnt, lane);
         if (lane < kk) {
-            nbrT[(size_t)lane * n + i] = in.slot_of[cj[lane]];
+            nbr[(size_t)i * kK + lane] = in.slot_of[cj[lane]];
         }
         if (lane == 0) {
             nnb[i] = kk;
@@ -1308,8 +1511,8 @@ __device__ __forceinline__ void k_truss_node_body(Hash H, TrussIn in, int n, con
     }
 }
 
-__global__ __launch_bounds__(kWave) void k_truss_node(Hash H, TrussIn in, int n, const int32_t* __restrict__ list, const Ctl* __restrict__ ctl, int32_t* __restrict__ nbrT, int32_t* __restrict__ nnb, float4* __restrict__ P0) {
-    k_truss_node_body(H, in, n, list, ctl, nbrT, nnb, P0, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(kWave) void k_truss_node(Hash H, TrussIn in, int n, const int32_t* __restrict__ list, const Ctl* __restrict__ ctl, int32_t* __restrict__ nbr, int32_t* __restrict__ nnb, float4* __restrict__ P0) {
+    k_truss_node_body(H, in, n, list, ctl, nbr, nnb, P0, blockIdx.x, gridDim.x);
 }
 
 // ---- node counts by type: interface, junction, interior, corner ------------------------
@@ -1377,7 +1580,7 @@ __device__ __forceinline__ void wave_append(bool flag, int i, int32_t* count, in
 // the junction nodes and, when `sticky` is given, the nodes a lean pass has handed back
 // before (their move is the same whichever pass computes it; queued here, it leaves the
 // iteration's critical path).
-__device__ __forceinline__ void k_force_body(const float4* __restrict__ X, const uint8_t* __restrict__ typ, const int32_t* __restrict__ nbrT, const int32_t* __restrict__ nnb, float fscale, float fsurf, int n, float4* __restrict__ F, Ctl* __restrict__ ctl, int32_t* __restrict__ queue_rest, uint8_t* __restrict__ skip, const uint8_t* __restrict__ sticky, int bid, int nblk) {
+__device__ __forceinline__ void k_force_body(const float4* __restrict__ X, const uint8_t* __restrict__ typ, const int32_t* __restrict__ nbr, const int32_t* __restrict__ nnb, float fscale, float fsurf, int n, float4* __restrict__ F, Ctl* __restrict__ ctl, int32_t* __restrict__ queue_rest, uint8_t* __restrict__ skip, const uint8_t* __restrict__ sticky, int bid, int nblk) {
     const int i = bid * kBlock + threadIdx.x;
     bool junction = false;
     if (i == 0) {   // the counts that the iteration's later kernels fill
@@ -1388,7 +1591,7 @@ __device__ __forceinline__ void k_force_body(const float4* __restrict__ X, const
         ctl->nmove_def = 0;
     }
     if (i < n) {
-        F[i] = bar_force(X, typ, nbrT, nnb, fscale, fsurf, i, n);
+        F[i] = bar_force(X, typ, nbr, nnb, fscale, fsurf, i);
         if (queue_rest) {
             junction = typ[i] == TN_JUNCTION || (sticky && sticky[i]);
             skip[i] = junction ? 1 : 0;
@@ -1399,8 +1602,8 @@ __device__ __forceinline__ void k_force_body(const float4* __restrict__ X, const
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_force(const float4* __restrict__ X, const uint8_t* __restrict__ typ, const int32_t* __restrict__ nbrT, const int32_t* __restrict__ nnb, float fscale, float fsurf, int n, float4* __restrict__ F, Ctl* __restrict__ ctl, int32_t* __restrict__ queue_rest, uint8_t* __restrict__ skip, const uint8_t* __restrict__ sticky) {
-    k_force_body(X, typ, nbrT, nnb, fscale, fsurf, n, F, ctl, queue_rest, skip, sticky, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(kBlock) void k_force(const float4* __restrict__ X, const uint8_t* __restrict__ typ, const int32_t* __restrict__ nbr, const int32_t* __restrict__ nnb, float fscale, float fsurf, int n, float4* __restrict__ F, Ctl* __restrict__ ctl, int32_t* __restrict__ queue_rest, uint8_t* __restrict__ skip, const uint8_t* __restrict__ sticky) {
+    k_force_body(X, typ, nbr, nnb, fscale, fsurf, n, F, ctl, queue_rest, skip, sticky, blockIdx.x, gridDim.x);
 }
 
 // ---- move (v2m_move, src/opencl/v2m_particle_body.cl:844-935) ----------------------
@@ -2165,7 +2368,7 @@ struct PlanIter {
     int n, fire, nparts, voxel;   // voxel: the voxel-trap move (no queues)
     float fscale, fsurf, skin;
     Ctl* ctl;
-    int32_t* nbrT;
+    int32_t* nbr;
     int32_t* nnb;
     float4 *X, *V, *F, *P0;
     uint8_t* typ;
@@ -2190,7 +2393,7 @@ struct PlanIter {
 __global__ __launch_bounds__(kBlock) void kg_force(const PlanIter* __restrict__ tab, const int32_t* __restrict__ bplan,
                                                    const int32_t* __restrict__ bfirst) {
     TN_PLAN_BLOCK(kShNodes);
-    k_force_body(P.X, P.typ, P.nbrT, P.nnb, P.fscale, P.fsurf, P.n, P.F, P.ctl, P.voxel ? nullptr : P.mq2, P.flag,
+    k_force_body(P.X, P.typ, P.nbr, P.nnb, P.fscale, P.fsurf, P.n, P.F, P.ctl, P.voxel ? nullptr : P.mq2, P.flag,
                  P.sticky, bid_, nb_);
 }
 
@@ -2243,7 +2446,7 @@ __global__ __launch_bounds__(kWave) void kg_truss_node(const PlanIter* __restric
                                                        const int32_t* __restrict__ bplan,
                                                        const int32_t* __restrict__ bfirst) {
     TN_PLAN_BLOCK(kShRefresh);
-    k_truss_node_body(P.H, P.tin, P.n, P.rqueue, P.ctl, P.nbrT, P.nnb, P.P0, bid_, nb_);
+    k_truss_node_body(P.H, P.tin, P.n, P.rqueue, P.ctl, P.nbr, P.nnb, P.P0, bid_, nb_);
 }
 
 __global__ __launch_bounds__(kBlock) void kg_control(const PlanIter* __restrict__ tab,

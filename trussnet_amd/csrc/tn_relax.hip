@@ -73,9 +73,11 @@ void arg_check(bool ok, const std::string& what) {
     }
 }
 
-// whether the largest size hbig's reach fits the top level's cell
-int hash_prune(const tnd::Hash& H, const tn_relax_params* prm, float hbig) {
-    return (prm->t + prm->skin) * hbig <= H.b0 * (float)(1 << (H.nlev - 1)) ? 1 : 0;
+// the K-nearest search may skip cells beyond a node's reach only if every node's reach
+// (t + skin) h fits the cell of its level, i.e. the largest h (hbig) fits the top level
+void set_largest(tnd::Hash& H, const tn_relax_params* prm, float hbig) {
+    H.hbig = hbig;
+    H.prune = (prm->t + prm->skin) * hbig <= H.b0 * (float)(1 << (H.nlev - 1)) ? 1 : 0;
 }
 
 // the hash geometry of relax_cpu (src/v2m_particles.cpp:738-761)
@@ -105,13 +107,11 @@ tnd::Hash make_hash_geom(int nx, int ny, int nz, const float* vs, float hmin, fl
     }
     H.nkeys = (int)nkeys;
     *nkeys_out = nkeys;
-    // the K-nearest search may skip cells beyond a node's reach only if every node's
-    // reach (t + skin) h fits the cell of its level, i.e. the largest h fits the top level
-    H.prune = hash_prune(H, prm, hbig);
+    set_largest(H, prm, hbig);
     return H;
 }
 
-// a host grid's hash, without its prune flag (plan_build takes the largest h on the device)
+// a host grid's hash, without its largest h (plan_build takes it on the device)
 tnd::Hash make_hash(const tn_grid_view* g, const tn_relax_params* prm, int64_t* nkeys_out) {
     return make_hash_geom(g->nx, g->ny, g->nz, g->vs, g->hmin, g->hmax, 0.0f, prm, nkeys_out);
 }
@@ -674,7 +674,7 @@ struct tn_plan {
     tnk::BrickMap bricks{};                // the K-nearest search's query order (brick positions)
     int32_t* dBrick = nullptr;             // [bricks.size + 1]: node counts, then starts, by brick position
     float *dMv = nullptr, *dPw = nullptr, *dThr = nullptr;
-    int32_t *dKey = nullptr, *dCstart = nullptr, *dSorted = nullptr, *dNbrT = nullptr, *dNnb = nullptr;
+    int32_t *dKey = nullptr, *dCstart = nullptr, *dSorted = nullptr, *dNbr = nullptr, *dNnb = nullptr;
     int32_t *dQueue = nullptr, *dBsum = nullptr;
     // the move queues: interface (lean), interior (lean), general, handed back
     int32_t *dMoveQ = nullptr, *dMoveQi = nullptr, *dMoveQ2 = nullptr, *dMoveQd = nullptr;
@@ -770,7 +770,10 @@ struct tn_plan {
                                                                                                          dBrick);
         scan(dBrick, dBrick, (int64_t)bricks.size + 1);
         tnk::k_brick_order<<<nb, tnk::kBlock, 0, stream>>>(H, bricks, dKeySorted, n, dCstart, dBrick, dSorted);
-        tnk::k_truss<<<blocks_for(n, tnk::kTrussWave), tnk::kTrussWave, 0, stream>>>(H, truss_in(), n, dNbrT, dNnb);
+        tnk::k_truss<<<blocks_for(n, tnk::kTrussWave), tnk::kTrussWave, 0, stream>>>(
+            H, truss_in(), n, dNbr, reinterpret_cast<int4*>(dXb), reinterpret_cast<int4*>(dVb), dNnb);
+        tnk::k_lists<<<nb, tnk::kBlock, 0, stream>>>(dPs, dMs, n, tskin * 0.5f, dNbr, reinterpret_cast<int4*>(dXb),
+                                                     reinterpret_cast<int4*>(dVb), dSlotOf, dNnb);
         timer.end(KC_NEIGHBORS, t);
         TN_HIP(hipGetLastError());
         for (int kc : { KC_KEYS, KC_RADIX, KC_PERMUTE, KC_NEIGHBORS }) {
@@ -819,7 +822,7 @@ struct tn_plan {
         const unsigned nb = blocks_for(n, tnk::kBlock);
         hipEvent_t t = timer.begin(KC_FORCE);
         // (the junction nodes queued for the general pass, unless the move is the voxel trap's)
-        tnk::k_force<<<nb, tnk::kBlock, 0, stream>>>(dX, dTyp, dNbrT, dNnb, prm.fscale, prm.fsurf, n, dF, dCtl,
+        tnk::k_force<<<nb, tnk::kBlock, 0, stream>>>(dX, dTyp, dNbr, dNnb, prm.fscale, prm.fsurf, n, dF, dCtl,
                                                      prm.voxel_trap ? nullptr : dMoveQ2, dFlag, dSticky);
         timer.end(KC_FORCE, t);
         t = timer.begin(KC_MOVE_EASY);
@@ -907,7 +910,7 @@ struct tn_plan {
         tnk::k_control<<<1, tnk::kBlock, 0, stream>>>(ca, dCtl, dPartials, dPw, dSlotOf);
         timer.end(KC_CONTROL, t);
         t = timer.begin(KC_REFRESH);
-        tnk::k_truss_node<<<refresh_blocks, tnk::kWave, 0, stream>>>(H, truss_in(), n, dQueue, dCtl, dNbrT, dNnb, dP0);
+        tnk::k_truss_node<<<refresh_blocks, tnk::kWave, 0, stream>>>(H, truss_in(), n, dQueue, dCtl, dNbr, dNnb, dP0);
         timer.end(KC_REFRESH, t);
         TN_HIP(hipGetLastError());
         TN_HIP(hipMemcpyAsync(hCtl, dCtl, sizeof(tnk::Ctl), hipMemcpyDeviceToHost, stream));
@@ -957,7 +960,7 @@ struct tn_plan {
         a.fsurf = prm.fsurf;
         a.skin = prm.skin;
         a.ctl = dCtl;
-        a.nbrT = dNbrT;
+        a.nbr = dNbr;
         a.nnb = dNnb;
         a.X = dX;
         a.V = dV;
@@ -1049,11 +1052,11 @@ namespace {
 
 // A plan on device dev: make_grid(mem) puts the grid into the plan's memory and
 // returns its Field; H and nkeys are the hash geometry, nslot the grid's phi slots.
-// find_prune: H.prune is still to be set, from the grid's largest h. With an arena, the plan
+// find_largest: the hash's largest h is still to be taken, from the grid on the device. With an arena, the plan
 // allocates nothing (DevMem::set_arena; tn_plan::noalloc).
 template <class MakeGrid>
 tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int dev, const tnd::Hash& H, int64_t nkeys,
-                    int64_t nslot, bool find_prune, MakeGrid make_grid, void* arena = nullptr, size_t arena_cap = 0) {
+                    int64_t nslot, bool find_largest, MakeGrid make_grid, void* arena = nullptr, size_t arena_cap = 0) {
         TN_HIP(hipSetDevice(dev));
         std::unique_ptr<tn_plan> p(new tn_plan);
         p->device = dev;
@@ -1118,7 +1121,7 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
         p->dPw = p->alloc<float>(n);
         p->dKey = p->alloc<int32_t>(n);
         p->dSorted = p->alloc<int32_t>(n);
-        p->dNbrT = p->alloc<int32_t>((size_t)n * TN_K);
+        p->dNbr = p->alloc<int32_t>((size_t)n * TN_K);
         p->dNnb = p->alloc<int32_t>(n);
         p->dQueue = p->alloc<int32_t>(n);
         p->dMoveQ = p->alloc<int32_t>(n);
@@ -1169,9 +1172,9 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
             TN_HIP(hipMemcpy(p->dTyp0, seeds->typ, n, hipMemcpyHostToDevice));
             TN_HIP(hipMemcpy(p->dLab0, seeds->lab, sizeof(uint16_t) * n, hipMemcpyHostToDevice));
         }
-        if (find_prune) {   // (the control block's memory, before its first use)
-            p->H.prune = hash_prune(H, prm, device_minmax<true>(f.h, (int64_t)f.nx * f.ny * f.nz,
-                                                                reinterpret_cast<int32_t*>(p->dCtl), p->stream).second);
+        if (find_largest) {   // (the control block's memory, before its first use)
+            set_largest(p->H, prm, device_minmax<true>(f.h, (int64_t)f.nx * f.ny * f.nz,
+                                                       reinterpret_cast<int32_t*>(p->dCtl), p->stream).second);
         }
         // (after every buffer that the plan cannot do without)
         if (n > 0 && !prm->voxel_trap) {
@@ -2733,13 +2736,13 @@ int tn_plan_rebuild(tn_plan* p, int32_t* key, int32_t* sorted, int32_t* cstart, 
                 nnb[id[t]] = cnt[t];
             }
         }
-        if (nbr) {   // slot-major by slot on the device, node-major by id (src/v2m_particles.cpp:764) here
+        if (nbr) {   // a row a slot on the device, a row an id (src/v2m_particles.cpp:764) here
             std::vector<int32_t> tr((size_t)n * TN_K);
-            TN_HIP(hipMemcpy(tr.data(), p->dNbrT, sizeof(int32_t) * n * TN_K, hipMemcpyDeviceToHost));
+            TN_HIP(hipMemcpy(tr.data(), p->dNbr, sizeof(int32_t) * n * TN_K, hipMemcpyDeviceToHost));
             for (int t = 0; t < n; ++t) {
                 const size_t i = (size_t)id[t];
                 for (int k = 0; k < TN_K; ++k) {
-                    nbr[i * TN_K + k] = k < cnt[t] ? id[tr[(size_t)k * n + t]] : -1;
+                    nbr[i * TN_K + k] = k < cnt[t] ? id[tr[(size_t)t * TN_K + k]] : -1;
                 }
             }
         }
@@ -2754,7 +2757,7 @@ int tn_plan_force(tn_plan* p, float* F) {
         if (n == 0) {
             return;
         }
-        tnk::k_force<<<blocks_for(n, tnk::kBlock), tnk::kBlock, 0, p->stream>>>(p->dX, p->dTyp, p->dNbrT, p->dNnb,
+        tnk::k_force<<<blocks_for(n, tnk::kBlock), tnk::kBlock, 0, p->stream>>>(p->dX, p->dTyp, p->dNbr, p->dNnb,
                                                                                p->prm.fscale, p->prm.fsurf, n, p->dF,
                                                                                p->dCtl, nullptr, nullptr, nullptr);
         TN_HIP(hipGetLastError());
