@@ -27,8 +27,18 @@
 // backwards from checkpoints of the positions every `ckpt_every` steps; within a
 // segment the states are recomputed, with each node's F and D, and one gather
 // pass per step forms the new adjoint from the node's own bars and the bars that
-// point at it (a reverse list built once), so no adjoint sum needs an atomic.
-// Only the sizing-grid gradient is scattered (double atomics).
+// point at it (found once), so no adjoint sum needs an atomic. Only the sizing-grid
+// gradient is scattered (integer atomics).
+//
+// Four lanes (a quad) share a node: the passes over the lists are bound by each bar's
+// arithmetic (two exponentials' worth, a logarithm, divisions) and by the gathers before
+// it, and 200 k nodes, one a lane, leave three waves a SIMD, each with one gather of one bar
+// in flight. A lane takes every fourth entry of its node's row and loads the other ends of
+// all its bars before it forms the first. 195 k nodes of 22 bars: a forward step 62 us, one
+// node a lane; 34 with quads, 1520 vector instructions a wave and these 9 tenths of the time;
+// 22 with one exponential and no correctly rounded division or root a bar, 810. A step
+// backwards 141 us; 59 with quads and the bars that two nodes share formed once; 44. Their
+// bytes would take 3 and 6 us: they stay bound by the bars' instructions.
 #pragma once
 
 namespace tnadj {
@@ -38,21 +48,52 @@ using tnk::kWave;
 
 struct AdjArgs {
     int n;
-    const int32_t* __restrict__ nbr;     // [K * n] list position-major: entry k of node i at k * n + i
+    const int32_t* __restrict__ nbr;     // [n * K] a row a node: the other end, with kMutual (entry_node, entry_mutual)
     const int32_t* __restrict__ nnb;     // [n]
     const uint8_t* __restrict__ typ;     // [n]
-    const int32_t* __restrict__ rstart;  // [n + 1] reverse lists: the bars pointing at each node
-    const int32_t* __restrict__ rsrc;    // [E] entries i * K + k
+    const int32_t* __restrict__ rstart;  // [n + 1] the bars pointing at each node from nodes it has none to
+    const int32_t* __restrict__ rsrc;    // entries i * K + k
     const int32_t* __restrict__ tet;     // [4 ntet]
     const int32_t* __restrict__ vstart;  // [n + 1] the tets at each node
     const int32_t* __restrict__ vtet;    // entries 4 t + corner
     int ntet;
     const float* __restrict__ theta;
-    const float4* __restrict__ B;        // [n] the start positions; states hold displacements from them
+    const float4* __restrict__ B;        // [n] the start positions and the type (its bits); states hold displacements
     int gx, gy, gz;
     float ox, oy, oz, dx, dy, dz;
     float dt, fscale, fsurf, beta, wq, eps_v;
+    float ibeta, ibeta_lo;   // 1 / beta, and what its rounding left out
 };
+
+// A list entry: the bar's other end j, and whether j's list holds the bar back (the r-th
+// bar from i to j and the r-th from j to i belong together where a list names a node more
+// than once). The two share length, target and rates, so their adjoints are formed at once.
+constexpr int kMutual = 1 << 30;   // (node counts stay below 2^31 / K)
+__device__ __forceinline__ int entry_node(int e) {
+    return e & (kMutual - 1);
+}
+__device__ __forceinline__ bool entry_mutual(int e) {
+    return (e & kMutual) != 0;
+}
+
+constexpr int kQuad = 4;                      // lanes a node
+constexpr int kOwn = TN_K / kQuad;            // a lane's entries of its node's row
+static_assert(TN_K % kQuad == 0, "a row is dealt to a quad");
+
+// the sum over the quad, in every lane of it (all four are active)
+__device__ __forceinline__ float quad_sum(float v) {
+    v += __int_as_float(tnk::dpp<0xB1>(__float_as_int(v), __float_as_int(v)));
+    return v + __int_as_float(tnk::dpp<0x4E>(__float_as_int(v), __float_as_int(v)));
+}
+template <int kCtrl>
+__device__ __forceinline__ double quad_perm(double v) {
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(tnk::dpp<kCtrl>(hi, hi), tnk::dpp<kCtrl>(lo, lo));
+}
+__device__ __forceinline__ double quad_sum(double v) {
+    v += quad_perm<0xB1>(v);
+    return v + quad_perm<0x4E>(v);
+}
 
 // ---- the sizing grid ---------------------------------------------------------------
 
@@ -115,74 +156,112 @@ __device__ __forceinline__ float size_of(const AdjArgs& A, float x, float y, flo
 // rounded to the unit once; a cell's sum stays far inside the +-2^19 range.
 constexpr double kThetaScale = 17592186044416.0;   // 2^44
 
-// gtheta[idx] += v for every lane of the wave (all lanes call it): lanes of one
-// run of equal cells (neighbouring nodes share cells) add once
+// gtheta[idx] += v for every lane of the wave (all lanes call it): lanes of one place in
+// their quads that follow each other with equal cells (neighbouring nodes share cells) add once
 __device__ __forceinline__ void theta_add(unsigned long long* __restrict__ gtheta, int idx, double v) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int prev = __shfl_up(idx, 1, kWave);
-    const bool head = lane == 0 || prev != idx;
-    const uint64_t heads = __ballot(head);
+    const int prev = __shfl_up(idx, kQuad, kWave);
+    const uint64_t place = 0x1111111111111111ull << (lane & (kQuad - 1));
+    const uint64_t heads = __ballot(lane < kQuad || prev != idx);
     const uint64_t upto = lane == kWave - 1 ? ~0ull : ((1ull << (lane + 1)) - 1);
-    const int seg = __popcll(heads & upto);
+    const int seg = __popcll(heads & place & upto);
 #pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
+    for (int d = kQuad; d < kWave; d <<= 1) {
         const double y = __shfl_up(v, d, kWave);
         const int sy = __shfl_up(seg, d, kWave);
         if (lane >= d && sy == seg) {
             v += y;
         }
     }
-    const int next = __shfl_down(seg, 1, kWave);
-    if ((lane == kWave - 1 || next != seg) && v != 0.0) {
+    const int next = __shfl_down(seg, kQuad, kWave);
+    if ((lane >= kWave - kQuad || next != seg) && v != 0.0) {
         atomicAdd(&gtheta[idx], (unsigned long long)__double2ll_rn(v * kThetaScale));
     }
 }
 
-// the adjoint hd of h at x: hd * dh/dx into g, hd * w_c into the grid gradient
-// (every lane of the wave calls it; hd = 0 for a lane with nothing to add)
-__device__ __forceinline__ void size_adjoint(const AdjArgs& A, float x, float y, float z, float hd, float3& g,
+// size_of by a quad, lane q of it two corners
+__device__ __forceinline__ float quad_size_of(const AdjArgs& A, float x, float y, float z, int q) {
+    const Tri t = tri_at(A, x, y, z);
+    return quad_sum(tri_weight(t, q) * A.theta[tri_index(A, t, q)] +
+                    tri_weight(t, q + 4) * A.theta[tri_index(A, t, q + 4)]);
+}
+
+// the adjoint hd of h at x: hd * dh/dx into g, hd * w_c into the grid gradient, lane q of
+// the node's quad with the corners q and q + 4 (every lane of the wave calls it; hd = 0 for
+// a quad with nothing to add)
+__device__ __forceinline__ void size_adjoint(const AdjArgs& A, float x, float y, float z, float hd, int q, float3& g,
                                              unsigned long long* __restrict__ gtheta) {
     const Tri t = tri_at(A, x, y, z);
-    float th[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        th[c] = A.theta[tri_index(A, t, c)];
-        theta_add(gtheta, tri_index(A, t, c), (double)(hd * tri_weight(t, c)));
-    }
     // d h / d f per axis (trilinear in the smoothed fractions), times d f / d x
     float hx = 0.0f, hy = 0.0f, hz = 0.0f;
+    const float wx = (q & 1) ? t.fx : 1.0f - t.fx, wy = (q >> 1) ? t.fy : 1.0f - t.fy;
+    const float sx = (q & 1) ? 1.0f : -1.0f, sy = (q >> 1) ? 1.0f : -1.0f;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const float wx = (c & 1) ? t.fx : 1.0f - t.fx, wy = ((c >> 1) & 1) ? t.fy : 1.0f - t.fy,
-                    wz = (c >> 2) ? t.fz : 1.0f - t.fz;
-        const float sx = (c & 1) ? 1.0f : -1.0f, sy = ((c >> 1) & 1) ? 1.0f : -1.0f, sz = (c >> 2) ? 1.0f : -1.0f;
-        hx += sx * wy * wz * th[c];
-        hy += wx * sy * wz * th[c];
-        hz += wx * wy * sz * th[c];
+    for (int up = 0; up < 2; ++up) {
+        const int c = q + 4 * up;
+        const float th = A.theta[tri_index(A, t, c)];
+        theta_add(gtheta, tri_index(A, t, c), (double)(hd * tri_weight(t, c)));
+        const float wz = up ? t.fz : 1.0f - t.fz, sz = up ? 1.0f : -1.0f;
+        hx += sx * wy * wz * th;
+        hy += wx * sy * wz * th;
+        hz += wx * wy * sz * th;
     }
-    g.x += hd * hx * t.gsx;
-    g.y += hd * hy * t.gsy;
-    g.z += hd * hz * t.gsz;
+    g.x += hd * quad_sum(hx) * t.gsx;
+    g.y += hd * quad_sum(hy) * t.gsy;
+    g.z += hd * quad_sum(hz) * t.gsz;
 }
 
 // ---- one bar -------------------------------------------------------------------------
-
-__device__ __forceinline__ float softplus(float u, float beta) {
-    return u > 0.0f ? u + log1pf(expf(-beta * u)) / beta : log1pf(expf(beta * u)) / beta;
-}
-
-__device__ __forceinline__ float logistic(float v) {
-    return 1.0f / (1.0f + expf(-v));
-}
 
 __device__ __forceinline__ float bar_c(const AdjArgs& A, int ti, int tj) {
     return (ti != TN_INTERIOR && tj != TN_INTERIOR) ? A.fsurf : A.fscale;
 }
 
 struct Bar {
-    float ex, ey, ez, l, sp, sg;   // e, |e|, sp(u), s(beta u)
+    float ex, ey, ez, l, inv, sp, sg;   // e, |e|, 1 / |e|, sp(u), s(beta u)
     bool ok;
 };
+
+// |e| and its inverse from its square: the hardware's reciprocal root, one Newton step on
+// each (l within 0.51 units in the last place, as measured over [2^-90, 2^90]); zeros,
+// infinities and what the hardware would flush take the library's root.
+__device__ __forceinline__ void root_and_inverse(float s, float& l, float& inv) {
+    if (s > 0x1p-90f && s < 0x1p90f) {
+        const float r = __builtin_amdgcn_rsqf(s), a = s * r;
+        l = fmaf(fmaf(-a, a, s), 0.5f * r, a);
+        inv = fmaf(fmaf(-l, r, 1.0f), r, r);
+    } else {
+        l = sqrtf(s);
+        inv = 1.0f / l;
+    }
+}
+
+// exp(-v) of v >= 0 (NaN stays NaN): the hardware's 2^x with the product's rounding put
+// back. 0 where the result would be denormal, as far below 1 as v > 87.
+__device__ __forceinline__ float exp_minus(float v) {
+    constexpr float kLog2e = 0x1.715476p+0f, kLog2eLo = 0x1.4ae0cp-26f, kLn2 = 0x1.62e43p-1f;
+    v = v > 200.0f ? 200.0f : v;
+    const float t = v * kLog2e, lo = fmaf(v, kLog2eLo, fmaf(v, kLog2e, -t));
+    const float y = __builtin_amdgcn_exp2f(-t);
+    return fmaf(y, -kLn2 * lo, y);
+}
+
+// log(1 + x) for 0 <= x <= 1: x + x^2 p(x), p of degree 9 (the least largest relative error
+// of the whole, 8e-10, by Lawson's iteration; 1.4 units in the last place at most and 0.26 on
+// average as rounded)
+__device__ __forceinline__ float log1p_unit(float x) {
+    float p = 0x1.0fb4aep-9f;
+    p = fmaf(p, x, -0x1.bead46p-7f);
+    p = fmaf(p, x, 0x1.57e95ep-5f);
+    p = fmaf(p, x, -0x1.544584p-4f);
+    p = fmaf(p, x, 0x1.fea748p-4f);
+    p = fmaf(p, x, -0x1.4a542ep-3f);
+    p = fmaf(p, x, 0x1.978278p-3f);
+    p = fmaf(p, x, -0x1.ffc42p-3f);
+    p = fmaf(p, x, 0x1.5553a6p-2f);
+    p = fmaf(p, x, -0x1.fffff8p-2f);
+    return fmaf(p * x, x, x);
+}
 
 // bar i -> j from the start positions b and the states x (displacement, h): the
 // start positions' difference is exact for neighbours (Sterbenz), so e keeps the
@@ -192,33 +271,77 @@ __device__ __forceinline__ Bar bar_at(const AdjArgs& A, float4 bi, float4 xi, fl
     b.ex = (bi.x - bj.x) + (xi.x - xj.x);
     b.ey = (bi.y - bj.y) + (xi.y - xj.y);
     b.ez = (bi.z - bj.z) + (xi.z - xj.z);
-    b.l = sqrtf(b.ex * b.ex + b.ey * b.ey + b.ez * b.ez);
+    root_and_inverse(b.ex * b.ex + b.ey * b.ey + b.ez * b.ez, b.l, b.inv);
     b.ok = b.l > 0.0f;
     const float u = c * 0.5f * (xi.w + xj.w) - b.l;
-    b.sp = softplus(u, A.beta);
-    b.sg = logistic(A.beta * u);
+    // sp(u) and s(beta u) from one exponential, of -|beta u|
+    const float v = A.beta * u, ex = exp_minus(fabsf(v)), lg = log1p_unit(ex);
+    b.sp = fmaf(lg, A.ibeta, fmaf(lg, A.ibeta_lo, u > 0.0f ? u : 0.0f));
+    const float d = 1.0f + ex, r0 = __builtin_amdgcn_rcpf(d), r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
+    b.sg = v > 0.0f ? r : ex * r;
     return b;
 }
 
-// F_i and D_i of node i at the state X (xyz, h). The bar forces of a relaxed node
-// nearly cancel, and the adjoint weighs F_i itself (kappa = mu . F / D^2): the sum
+__device__ __forceinline__ int type_of(float4 b) {
+    return __float_as_int(b.w);
+}
+
+// the other ends of up to N bars of a node, entries e[.] of its list (a negative one: none,
+// the node itself, whose bar is not ok), loaded before any is used
+template <int N>
+struct Ends {
+    int j[N];
+    float4 b[N], x[N];
+    __device__ __forceinline__ void load(const AdjArgs& A, const float4* __restrict__ X, int i, const int (&e)[N]) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            j[k] = e[k] < 0 ? i : entry_node(e[k]);
+            b[k] = A.B[j[k]];
+            x[k] = X[j[k]];
+        }
+    }
+    __device__ __forceinline__ Bar bar(const AdjArgs& A, float4 bi, float4 xi, int k, float& c) const {
+        c = bar_c(A, type_of(bi), type_of(b[k]));
+        return bar_at(A, bi, xi, b[k], x[k], c);
+    }
+};
+
+// lane q's entries of node i's row (m long), -1 past its end
+__device__ __forceinline__ void own_entries(const AdjArgs& A, int i, int q, int m, int (&e)[kOwn]) {
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) {
+        e[k] = q + kQuad * k < m ? A.nbr[(size_t)i * TN_K + q + kQuad * k] : -1;
+    }
+}
+
+// F_i and D_i of node i at the state X (xyz, h), by its quad. The bar forces of a relaxed
+// node nearly cancel, and the adjoint weighs F_i itself (kappa = mu . F / D^2): the sum
 // runs in double so F_i keeps its relative precision.
-__device__ __forceinline__ float4 force_and_stiffness(const AdjArgs& A, const float4* __restrict__ X, int i) {
-    const float4 xi = X[i], bi = A.B[i];
-    const int ti = A.typ[i], m = A.nnb[i];
+__device__ __forceinline__ float4 force_and_stiffness(const AdjArgs& A, const float4* __restrict__ X, int i, int q,
+                                                      float4 xi, float4 bi) {
+    const int m = A.nnb[i];
+    int e[kOwn];
+    own_entries(A, i, q, m, e);
+    Ends<kOwn> o;
+    o.load(A, X, i, e);
     double Fx = 0.0, Fy = 0.0, Fz = 0.0, a = 0.0;
-    for (int k = 0; k < m; ++k) {
-        const int j = A.nbr[(size_t)k * A.n + i];
-        const Bar b = bar_at(A, bi, xi, A.B[j], X[j], bar_c(A, ti, A.typ[j]));
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) {
+        float c;
+        const Bar b = o.bar(A, bi, xi, k, c);
         if (b.ok) {
-            const double w = (double)b.sp / (double)b.l;
+            const double l = b.l;   // 1 / l to the last place but one: two Newton steps
+            double r = b.inv;
+            r = fma(fma(-l, r, 1.0), r, r);
+            r = fma(fma(-l, r, 1.0), r, r);
+            const double w = b.l < __builtin_huge_valf() ? (double)b.sp * r : 0.0;
             Fx += w * b.ex;
             Fy += w * b.ey;
             Fz += w * b.ez;
             a += b.sg;
         }
     }
-    return make_float4((float)Fx, (float)Fy, (float)Fz, (float)(1.0 + a));
+    return make_float4((float)quad_sum(Fx), (float)quad_sum(Fy), (float)quad_sum(Fz), (float)(1.0 + quad_sum(a)));
 }
 
 // ---- forward ---------------------------------------------------------------------------
@@ -228,7 +351,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_load(AdjArgs A, const float* __r
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i < A.n) {
         const float x = x0[3 * (size_t)i], y = x0[3 * (size_t)i + 1], z = x0[3 * (size_t)i + 2];
-        B[i] = make_float4(x, y, z, 0.0f);
+        B[i] = make_float4(x, y, z, __int_as_float(A.typ[i]));
         X[i] = make_float4(0.0f, 0.0f, 0.0f, size_of(A, x, y, z));
     }
 }
@@ -236,24 +359,26 @@ __global__ __launch_bounds__(kBlock) void k_adj_load(AdjArgs A, const float* __r
 // X -> Xn (positions and their sizes); FD (optional): F and D of each node at X
 __global__ __launch_bounds__(kBlock) void k_adj_step(AdjArgs A, const float4* __restrict__ X, float4* __restrict__ Xn,
                                                      float4* __restrict__ FD) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const int i = (blockIdx.x * kBlock + threadIdx.x) / kQuad, q = threadIdx.x % kQuad;
     if (i >= A.n) {
         return;
     }
-    const float4 fd = force_and_stiffness(A, X, i);
-    if (FD) {
+    float4 x = X[i];
+    const float4 b = A.B[i];
+    const float4 fd = force_and_stiffness(A, X, i, q, x, b);
+    if (FD && q == 0) {
         FD[i] = fd;
     }
-    float4 x = X[i];
-    if (A.typ[i] == TN_INTERIOR) {
+    if (type_of(b) == TN_INTERIOR) {
         const float s = A.dt / fd.w;
         x.x += s * fd.x;
         x.y += s * fd.y;
         x.z += s * fd.z;
-        const float4 b = A.B[i];
-        x.w = size_of(A, b.x + x.x, b.y + x.y, b.z + x.z);
+        x.w = quad_size_of(A, b.x + x.x, b.y + x.y, b.z + x.z, q);
     }
-    Xn[i] = x;
+    if (q == 0) {
+        Xn[i] = x;
+    }
 }
 
 // out = B + X (positions), or X alone (B null: an adjoint), 3 floats per node
@@ -321,13 +446,17 @@ __global__ __launch_bounds__(kBlock) void k_adj_loss_parts(AdjArgs A, const floa
                                                            double2* __restrict__ parts) {
     __shared__ double se[kBlock / kWave], sq[kBlock / kWave];
     double e = 0.0, q = 0.0;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < A.n; i += gridDim.x * kBlock) {
+    for (int i = (blockIdx.x * kBlock + threadIdx.x) / kQuad; i < A.n; i += gridDim.x * (kBlock / kQuad)) {
         const float4 xi = X[i], bi = A.B[i];
-        const int ti = A.typ[i], m = A.nnb[i];
+        int en[kOwn];
+        own_entries(A, i, threadIdx.x % kQuad, A.nnb[i], en);
+        Ends<kOwn> o;
+        o.load(A, X, i, en);
         float s = 0.0f;
-        for (int k = 0; k < m; ++k) {
-            const int j = A.nbr[(size_t)k * A.n + i];
-            const Bar b = bar_at(A, bi, xi, A.B[j], X[j], bar_c(A, ti, A.typ[j]));
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            float c;
+            const Bar b = o.bar(A, bi, xi, k, c);
             if (b.ok) {
                 s += 0.5f * b.sp * b.sp;
             }
@@ -388,48 +517,52 @@ __global__ __launch_bounds__(kBlock) void k_adj_loss_sum(AdjArgs A, const double
 // and of the bars pointing at it, and the quality of its tets
 __global__ __launch_bounds__(kBlock) void k_adj_loss_grad(AdjArgs A, const float4* __restrict__ X,
                                                           float4* __restrict__ lam, unsigned long long* __restrict__ gtheta) {
-    int p = blockIdx.x * kBlock + threadIdx.x;
+    int p = (blockIdx.x * kBlock + threadIdx.x) / kQuad;
+    const int q = threadIdx.x % kQuad;
     const bool valid = p < A.n;   // the others stand in for node n - 1: every lane joins the scatter
     if (!valid) {
         p = A.n - 1;
     }
     const float en = 1.0f / (float)A.n;
     const float4 xp = X[p], bp = A.B[p];
-    const int tp = A.typ[p];
     float3 g = make_float3(0.0f, 0.0f, 0.0f);
     float hd = 0.0f;
-    // own bars p -> j: dE/de = -(1/n) sp s n, dE/dl0 = (1/n) sp s
-    const int m = A.nnb[p];
-    for (int k = 0; k < m; ++k) {
-        const int j = A.nbr[(size_t)k * A.n + p];
-        const float c = bar_c(A, tp, A.typ[j]);
-        const Bar b = bar_at(A, bp, xp, A.B[j], X[j], c);
+    // a bar p -> j: dE/de = -(1/n) sp s n, dE/dl0 = (1/n) sp s; a bar j -> p the same, with e
+    // from j to p: as much again to p
+    auto add = [&](const Bar& b, float c, float times) {
         if (b.ok) {
-            const float w = en * b.sp * b.sg;
+            const float w = times * (en * b.sp * b.sg);
             g.x -= w * b.ex / b.l;
             g.y -= w * b.ey / b.l;
             g.z -= w * b.ez / b.l;
             hd += 0.5f * c * w;
         }
-    }
-    // bars i -> p
-    for (int r = A.rstart[p]; r < A.rstart[p + 1]; ++r) {
-        const int i = A.rsrc[r] / TN_K;
-        const float c = bar_c(A, A.typ[i], tp);
-        const Bar b = bar_at(A, A.B[i], X[i], bp, xp, c);
-        if (b.ok) {
-            const float w = en * b.sp * b.sg;
-            g.x += w * b.ex / b.l;
-            g.y += w * b.ey / b.l;
-            g.z += w * b.ez / b.l;
-            hd += 0.5f * c * w;
+    };
+    {
+        int e[kOwn];
+        own_entries(A, p, q, A.nnb[p], e);
+        Ends<kOwn> o;
+        o.load(A, X, p, e);
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            float c;
+            const Bar b = o.bar(A, bp, xp, k, c);
+            add(b, c, entry_mutual(e[k]) ? 2.0f : 1.0f);
         }
+    }
+    for (int r = A.rstart[p] + q; r < A.rstart[p + 1]; r += kQuad) {   // bars i -> p alone
+        const int e[1] = { A.rsrc[r] / TN_K };
+        Ends<1> o;
+        o.load(A, X, p, e);
+        float c;
+        const Bar b = o.bar(A, bp, xp, 0, c);
+        add(b, c, 1.0f);
     }
     // tets: d(-wq/ntet q)/dx_p, q = 12 (3 Vs)^(2/3) / S (in double)
     const double wt = A.ntet > 0 ? -(double)A.wq / (double)A.ntet : 0.0;
     double tx = 0.0, ty = 0.0, tz = 0.0;
     const D3 pp = d3(bp, xp);
-    for (int r = A.vstart[p]; r < A.vstart[p + 1]; ++r) {
+    for (int r = A.vstart[p] + q; r < A.vstart[p + 1]; r += kQuad) {
         const int t = A.vtet[r] >> 2, corner = A.vtet[r] & 3;
         const TetQ Q = tet_quality(A, X, t);
         // d(6V)/dx_corner
@@ -462,21 +595,23 @@ __global__ __launch_bounds__(kBlock) void k_adj_loss_grad(AdjArgs A, const float
         ty += wt * (kv * dv.y - ks * ds.y);
         tz += wt * (kv * dv.z - ks * ds.z);
     }
-    g.x += (float)tx;
-    g.y += (float)ty;
-    g.z += (float)tz;
-    size_adjoint(A, bp.x + xp.x, bp.y + xp.y, bp.z + xp.z, valid ? hd : 0.0f, g, gtheta);
-    if (valid) {
+    g.x = quad_sum(g.x) + (float)quad_sum(tx);
+    g.y = quad_sum(g.y) + (float)quad_sum(ty);
+    g.z = quad_sum(g.z) + (float)quad_sum(tz);
+    hd = quad_sum(hd);
+    size_adjoint(A, bp.x + xp.x, bp.y + xp.y, bp.z + xp.z, valid ? hd : 0.0f, q, g, gtheta);
+    if (valid && q == 0) {
         lam[p] = make_float4(g.x, g.y, g.z, 0.0f);
     }
 }
 
 // ---- one step backwards ------------------------------------------------------------------
 
-// the adjoint of bar i -> j for node i's (nu, kappa): returns g_e (to x_i; -g_e to
-// x_j) and g_l0 in .w
+// The adjoint of the bar p -> j for (nu, kappa) of p, to x_p in xyz and to l0 in .w. The
+// bar j -> p for (nu_j, kappa_j) gives x_p and l0 what p -> j would for (-nu_j, kappa_j): of
+// a mutual pair, nu is nu_p - nu_j and kappa the sum.
 __device__ __forceinline__ float4 bar_adjoint(const Bar& b, float3 nu, float kappa, float beta) {
-    const float inv = 1.0f / b.l;
+    const float inv = b.inv;
     const float nx = b.ex * inv, ny = b.ey * inv, nz = b.ez * inv;
     const float vn = nu.x * nx + nu.y * ny + nu.z * nz;
     const float rho = beta * b.sg * (1.0f - b.sg);
@@ -509,56 +644,62 @@ __global__ __launch_bounds__(kBlock) void k_adj_back(AdjArgs A, const float4* __
                                                      const float4* __restrict__ nk, const float4* __restrict__ lamn,
                                                      float4* __restrict__ lam, unsigned long long* __restrict__ gtheta,
                                                      const float4* __restrict__ FDprev, float4* __restrict__ nk_prev) {
-    int p = blockIdx.x * kBlock + threadIdx.x;
+    int p = (blockIdx.x * kBlock + threadIdx.x) / kQuad;
+    const int q = threadIdx.x % kQuad;
     const bool valid = p < A.n;   // the others stand in for node n - 1: every lane joins the scatter
     if (!valid) {
         p = A.n - 1;
     }
-    const float4 xp = X[p], bp = A.B[p];
-    const int tp = A.typ[p];
-    const float4 lp = lamn[p];
-    float3 g = make_float3(lp.x, lp.y, lp.z);
+    const float4 xp = X[p], bp = A.B[p], nkp = nk[p];   // (nu and kappa of a node that stays are 0)
+    float3 g = make_float3(0.0f, 0.0f, 0.0f);
     float hd = 0.0f;
-    if (tp == TN_INTERIOR) {   // own bars p -> j
-        const float4 nkp = nk[p];
-        const float3 nu = make_float3(nkp.x, nkp.y, nkp.z);
-        const int m = A.nnb[p];
-        for (int k = 0; k < m; ++k) {
-            const int j = A.nbr[(size_t)k * A.n + p];
-            const float c = bar_c(A, tp, A.typ[j]);
-            const Bar b = bar_at(A, bp, xp, A.B[j], X[j], c);
-            if (b.ok) {
-                const float4 ge = bar_adjoint(b, nu, nkp.w, A.beta);
-                g.x += ge.x;
-                g.y += ge.y;
-                g.z += ge.z;
-                hd += 0.5f * c * ge.w;
-            }
-        }
-    }
-    for (int r = A.rstart[p]; r < A.rstart[p + 1]; ++r) {   // bars i -> p of moving nodes i
-        const int i = A.rsrc[r] / TN_K;
-        const int ti = A.typ[i];
-        if (ti != TN_INTERIOR) {
-            continue;
-        }
-        const float4 nki = nk[i];
-        const float c = bar_c(A, ti, tp);
-        const Bar b = bar_at(A, A.B[i], X[i], bp, xp, c);
+    auto add = [&](const Bar& b, float c, float3 nu, float kappa) {
         if (b.ok) {
-            const float4 ge = bar_adjoint(b, make_float3(nki.x, nki.y, nki.z), nki.w, A.beta);
-            g.x -= ge.x;
-            g.y -= ge.y;
-            g.z -= ge.z;
+            const float4 ge = bar_adjoint(b, nu, kappa, A.beta);
+            g.x += ge.x;
+            g.y += ge.y;
+            g.z += ge.z;
             hd += 0.5f * c * ge.w;
         }
+    };
+    {
+        int e[kOwn];
+        own_entries(A, p, q, A.nnb[p], e);
+        Ends<kOwn> o;
+        o.load(A, X, p, e);
+        float4 nkj[kOwn];
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            nkj[k] = nk[o.j[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            float c;
+            const Bar b = o.bar(A, bp, xp, k, c);
+            const float4 v = entry_mutual(e[k]) ? nkj[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            add(b, c, make_float3(nkp.x - v.x, nkp.y - v.y, nkp.z - v.z), nkp.w + v.w);
+        }
     }
-    size_adjoint(A, bp.x + xp.x, bp.y + xp.y, bp.z + xp.z, valid ? hd : 0.0f, g, gtheta);
-    if (valid) {
+    for (int r = A.rstart[p] + q; r < A.rstart[p + 1]; r += kQuad) {   // bars i -> p alone
+        const int e[1] = { A.rsrc[r] / TN_K };
+        Ends<1> o;
+        o.load(A, X, p, e);
+        const float4 v = nk[e[0]];
+        float c;
+        const Bar b = o.bar(A, bp, xp, 0, c);
+        add(b, c, make_float3(-v.x, -v.y, -v.z), v.w);
+    }
+    const float4 lp = lamn[p];
+    g.x = lp.x + quad_sum(g.x);
+    g.y = lp.y + quad_sum(g.y);
+    g.z = lp.z + quad_sum(g.z);
+    hd = quad_sum(hd);
+    size_adjoint(A, bp.x + xp.x, bp.y + xp.y, bp.z + xp.z, valid ? hd : 0.0f, q, g, gtheta);
+    if (valid && q == 0) {
         const float4 l = make_float4(g.x, g.y, g.z, 0.0f);
         lam[p] = l;
         if (FDprev) {
-            nk_prev[p] = nu_kappa(A, tp, l, FDprev[p]);
+            nk_prev[p] = nu_kappa(A, type_of(bp), l, FDprev[p]);
         }
     }
 }
@@ -578,22 +719,37 @@ __global__ __launch_bounds__(kBlock) void k_fill_f64(double* __restrict__ a, int
     }
 }
 
-// reverse-list keys: the target of every valid list entry (-1: none)
+// Each list entry with its mark (kMutual), and the reverse lists' keys: the target of
+// every entry that its target's list does not hold back (n, past every node: none)
 __global__ __launch_bounds__(kBlock) void k_adj_targets(int n, const int32_t* __restrict__ nbr,
-                                                        const int32_t* __restrict__ nnb, int32_t* __restrict__ key,
-                                                        int32_t* __restrict__ cnt) {
+                                                        const int32_t* __restrict__ nnb, int32_t* __restrict__ marked,
+                                                        int32_t* __restrict__ key, int32_t* __restrict__ cnt) {
     const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (e >= (int64_t)n * TN_K) {
         return;
     }
     const int i = (int)(e / TN_K), k = (int)(e % TN_K);
+    int mark = 0, to = n;
     if (k < nnb[i]) {
-        const int j = nbr[(size_t)k * n + i];
-        key[e] = j;
-        atomicAdd(&cnt[j], 1);
-    } else {
-        key[e] = n;   // sorts past every node
+        const int j = nbr[e];
+        int before = 0, back = 0;   // bars i -> j up to this one, bars j -> i
+        for (int t = 0; t <= k; ++t) {
+            before += nbr[(int64_t)i * TN_K + t] == j ? 1 : 0;
+        }
+        const int m = nnb[j];
+        for (int t = 0; t < m; ++t) {
+            back += nbr[(int64_t)j * TN_K + t] == i ? 1 : 0;
+        }
+        if (back >= before) {
+            mark = j | kMutual;
+        } else {
+            mark = j;
+            to = j;
+            atomicAdd(&cnt[j], 1);
+        }
     }
+    marked[e] = mark;
+    key[e] = to;
 }
 
 __global__ __launch_bounds__(kBlock) void k_adj_tet_keys(int ntet, const int32_t* __restrict__ tet,
@@ -707,15 +863,6 @@ int tn_adj_create(const tn_adj_problem* p, int32_t device, tn_adj** out) {
         SeedOps ops{ mem };
         tnadj::AdjArgs& A = a->A;
         A.n = n;
-        {   // the lists, list position-major (coalesced per position across nodes)
-            std::vector<int32_t> t((size_t)n * TN_K, 0);
-            for (int i = 0; i < n; ++i) {
-                for (int k = 0; k < p->nnb[i]; ++k) {
-                    t[(size_t)k * n + i] = p->nbr[(size_t)i * TN_K + k];
-                }
-            }
-            A.nbr = mem.upload(t.data(), t.size());
-        }
         A.nnb = mem.upload(p->nnb, (size_t)n);
         A.typ = mem.upload(p->typ, (size_t)n);
         A.ntet = a->ntet;
@@ -733,14 +880,20 @@ int tn_adj_create(const tn_adj_problem* p, int32_t device, tn_adj** out) {
         A.fscale = p->fscale;
         A.fsurf = p->fsurf;
         A.beta = p->beta;
+        A.ibeta = (float)(1.0 / (double)p->beta);
+        A.ibeta_lo = std::isfinite(A.ibeta) ? (float)(1.0 / (double)p->beta - (double)A.ibeta) : 0.0f;
         A.wq = p->wq;
         A.eps_v = p->eps_v;
-        // the bars pointing at each node, in (source, list position) order
+        // the lists with their marks, and the bars pointing at each node from nodes it has none
+        // to, in (source, list position) order
         {
             const int64_t m = (int64_t)n * TN_K;
+            const int32_t* nbr = mem.upload(p->nbr, (size_t)m);
+            int32_t* marked = mem.alloc<int32_t>((size_t)m);
             int32_t* key = mem.alloc<int32_t>((size_t)m);
             int32_t* cnt = ops.counts(n);
-            tnadj::k_adj_targets<<<blocks_for(m, tnk::kBlock), tnk::kBlock>>>(n, A.nbr, A.nnb, key, cnt);
+            tnadj::k_adj_targets<<<blocks_for(m, tnk::kBlock), tnk::kBlock>>>(n, nbr, A.nnb, marked, key, cnt);
+            A.nbr = marked;
             int32_t *starts = nullptr, *entries = nullptr;
             adj_csr(ops, key, m, n, cnt, starts, entries);
             A.rstart = starts;
@@ -778,7 +931,7 @@ int tn_adj_create(const tn_adj_problem* p, int32_t device, tn_adj** out) {
         a->base = mem.alloc<float4>(n);
         A.B = a->base;
         a->gtheta = mem.alloc<unsigned long long>(a->gcells);
-        a->nparts = (int)std::min<unsigned>(2048, blocks_for(std::max(n, a->ntet), tnk::kBlock));
+        a->nparts = (int)std::min<unsigned>(2048, blocks_for(std::max((int64_t)n * tnadj::kQuad, (int64_t)a->ntet), tnk::kBlock));
         a->parts = mem.alloc<double2>(a->nparts);
         a->dloss = mem.alloc<double>(3);
         TN_HIP(hipGetLastError());
@@ -793,7 +946,7 @@ int tn_adj_forward(tn_adj* a, const float* x0, const float* theta, float* xT, do
         TN_HIP(hipSetDevice(a->device));
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const int n = a->n;
-        const unsigned nb = blocks_for(n, tnk::kBlock);
+        const unsigned nb = blocks_for(n, tnk::kBlock), nq = blocks_for((int64_t)n * tnadj::kQuad, tnk::kBlock);
         tnadj::AdjArgs A = a->A;
         A.theta = theta;
         // state k lives in ckpts[k / ckpt] when k is a segment start, else in Xa / Xb
@@ -803,7 +956,7 @@ int tn_adj_forward(tn_adj* a, const float* x0, const float* theta, float* xT, do
             const int k1 = k + 1;
             float4* nxt = (k1 % a->ckpt == 0 && k1 < a->iters) ? a->ckpts + (size_t)(k1 / a->ckpt) * n
                                                                : (cur == a->Xa ? a->Xb : a->Xa);
-            tnadj::k_adj_step<<<nb, tnk::kBlock, 0, s>>>(A, cur, nxt, a->fd_all ? a->fd_all + (size_t)k * n : nullptr);
+            tnadj::k_adj_step<<<nq, tnk::kBlock, 0, s>>>(A, cur, nxt, a->fd_all ? a->fd_all + (size_t)k * n : nullptr);
             cur = nxt;
         }
         a->last = cur;
@@ -829,7 +982,7 @@ int tn_adj_backward(tn_adj* a, const float* theta, float* grad_x0, float* grad_t
         TN_HIP(hipSetDevice(a->device));
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const int n = a->n;
-        const unsigned nb = blocks_for(n, tnk::kBlock);
+        const unsigned nb = blocks_for(n, tnk::kBlock), nq = blocks_for((int64_t)n * tnadj::kQuad, tnk::kBlock);
         tnadj::AdjArgs A = a->A;
         A.theta = theta;
         tnadj::k_fill_f64<<<blocks_for(a->gcells, tnk::kBlock), tnk::kBlock, 0, s>>>(
@@ -839,16 +992,16 @@ int tn_adj_backward(tn_adj* a, const float* theta, float* grad_x0, float* grad_t
         float4* lam = a->lamA;
         float4* lamo = a->lamB;
         if (T == 0) {
-            tnadj::k_adj_loss_grad<<<nb, tnk::kBlock, 0, s>>>(A, a->ckpts, lam, a->gtheta);
+            tnadj::k_adj_loss_grad<<<nq, tnk::kBlock, 0, s>>>(A, a->ckpts, lam, a->gtheta);
         }
         if (a->fd_all) {   // every state and its F, D kept by the forward
-            tnadj::k_adj_loss_grad<<<nb, tnk::kBlock, 0, s>>>(A, a->last, lam, a->gtheta);
+            tnadj::k_adj_loss_grad<<<nq, tnk::kBlock, 0, s>>>(A, a->last, lam, a->gtheta);
             float4 *nkc = a->nk, *nkn = a->nk2;
             if (T > 0) {
                 tnadj::k_adj_nu<<<nb, tnk::kBlock, 0, s>>>(A, a->fd_all + (size_t)(T - 1) * n, lam, nkc);
             }
             for (int k = T - 1; k >= 0; --k) {   // each step also forms the next one's (nu, kappa)
-                tnadj::k_adj_back<<<nb, tnk::kBlock, 0, s>>>(A, a->ckpts + (size_t)k * n, nkc, lam, lamo, a->gtheta,
+                tnadj::k_adj_back<<<nq, tnk::kBlock, 0, s>>>(A, a->ckpts + (size_t)k * n, nkc, lam, lamo, a->gtheta,
                                                              k > 0 ? a->fd_all + (size_t)(k - 1) * n : nullptr, nkn);
                 std::swap(lam, lamo);
                 std::swap(nkc, nkn);
@@ -874,7 +1027,7 @@ int tn_adj_backward(tn_adj* a, const float* theta, float* grad_x0, float* grad_t
             }
             used[b] = true;
             for (int k = k0; k < k1; ++k) {
-                tnadj::k_adj_step<<<nb, tnk::kBlock, 0, a->side>>>(A, state(sg, k), state(sg, k + 1),
+                tnadj::k_adj_step<<<nq, tnk::kBlock, 0, a->side>>>(A, state(sg, k), state(sg, k + 1),
                                                                    a->fd[b] + (size_t)(k - k0) * n);
             }
             TN_HIP(hipEventRecord(a->ev_ready[b], a->side));
@@ -891,14 +1044,14 @@ int tn_adj_backward(tn_adj* a, const float* theta, float* grad_x0, float* grad_t
             }
             TN_HIP(hipStreamWaitEvent(s, a->ev_ready[b], 0));
             if (sg == a->nseg - 1) {   // X_T: the loss gradient starts the adjoint
-                tnadj::k_adj_loss_grad<<<nb, tnk::kBlock, 0, s>>>(A, state(sg, k1), lam, a->gtheta);
+                tnadj::k_adj_loss_grad<<<nq, tnk::kBlock, 0, s>>>(A, state(sg, k1), lam, a->gtheta);
             }
             float4 *nkc = a->nk, *nkn = a->nk2;
             // the segment's last step; the steps before get theirs from k_adj_back
             tnadj::k_adj_nu<<<nb, tnk::kBlock, 0, s>>>(A, a->fd[b] + (size_t)(k1 - 1 - k0) * n, lam, nkc);
             for (int k = k1 - 1; k >= k0; --k) {
                 const int r = k - k0;
-                tnadj::k_adj_back<<<nb, tnk::kBlock, 0, s>>>(A, state(sg, k), nkc, lam, lamo, a->gtheta,
+                tnadj::k_adj_back<<<nq, tnk::kBlock, 0, s>>>(A, state(sg, k), nkc, lam, lamo, a->gtheta,
                                                              k > k0 ? a->fd[b] + (size_t)(r - 1) * n : nullptr, nkn);
                 std::swap(lam, lamo);
                 std::swap(nkc, nkn);
