@@ -611,86 +611,12 @@ __device__ __forceinline__ void merge_sort(uint64_t (&k)[32]) {
 
 // ---- settling a few lanes' buffers with the whole wave -----------------------------------
 //
-// When only some lanes' buffers are full, the wave sorts them two at a time, one per
-// half-wave: lane i of a half holds entry i of its buffer (the key, with the slot it
-// came from) and a bitonic network runs across the 32 lanes, each compare-exchange
-// with partner lane i ^ j taken through DPP (quad_perm for j = 1, 2; row_ror:4 and
-// row_ror:12 for j = 4; row_ror:8 for j = 8) or ds_swizzle's bit mode (j = 16, xor
-// within 32 lanes). 15 steps of a few instructions against a 32-key register network
-// per settling lane.
-
-template <int kCtrl>
-__device__ __forceinline__ uint64_t dpp64(uint64_t v) {
-    const int lo = (int)(uint32_t)v, hi = (int)(uint32_t)(v >> 32);
-    return ((uint64_t)(uint32_t)dpp<kCtrl>(hi, hi) << 32) | (uint32_t)dpp<kCtrl>(lo, lo);
-}
-
-// the value of lane (i ^ J) of this lane's half-wave, i = lane % 32
-template <int J>
-__device__ __forceinline__ uint64_t xor_partner(uint64_t v, int i) {
-    if constexpr (J == 1) {
-        return dpp64<0xB1>(v);
-    } else if constexpr (J == 2) {
-        return dpp64<0x4E>(v);
-    } else if constexpr (J == 4) {
-        const uint64_t dn = dpp64<0x124>(v), up = dpp64<0x12C>(v);
-        return (i & 4) ? dn : up;
-    } else if constexpr (J == 8) {
-        return dpp64<0x128>(v);
-    } else {
-        static_assert(J == 16, "xor partners within 32 lanes");
-        const int lo = __builtin_amdgcn_ds_swizzle((int)(uint32_t)v, 0x401F);
-        const int hi = __builtin_amdgcn_ds_swizzle((int)(uint32_t)(v >> 32), 0x401F);
-        return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
-    }
-}
-
-// the 32-bit value of lane (i ^ J) of this lane's half-wave
-template <int J>
-__device__ __forceinline__ int xor_partner32(int v, int i) {
-    if constexpr (J == 1) {
-        return dpp<0xB1>(v, v);
-    } else if constexpr (J == 2) {
-        return dpp<0x4E>(v, v);
-    } else if constexpr (J == 4) {
-        const int dn = dpp<0x124>(v, v), up = dpp<0x12C>(v, v);
-        return (i & 4) ? dn : up;
-    } else if constexpr (J == 8) {
-        return dpp<0x128>(v, v);
-    } else {
-        return __builtin_amdgcn_ds_swizzle(v, 0x401F);
-    }
-}
-
-// one step of the network on (key, payload); keys are distinct or both padding
-template <int K, int J>
-__device__ __forceinline__ void half_bitonic_step_kv(uint64_t& v, int& pl, int i) {
-    const uint64_t o = xor_partner<J>(v, i);
-    const int op = xor_partner32<J>(pl, i);
-    const bool keep_min = ((i & J) == 0) == (K >= 32 || (i & K) == 0);
-    const bool take = keep_min == (o < v);
-    v = take ? o : v;
-    pl = take ? op : pl;
-}
-
-__device__ __forceinline__ void half_wave_sort32_kv(uint64_t& v, int& pl, int lane) {
-    const int i = lane & 31;
-    half_bitonic_step_kv<2, 1>(v, pl, i);
-    half_bitonic_step_kv<4, 2>(v, pl, i);
-    half_bitonic_step_kv<4, 1>(v, pl, i);
-    half_bitonic_step_kv<8, 4>(v, pl, i);
-    half_bitonic_step_kv<8, 2>(v, pl, i);
-    half_bitonic_step_kv<8, 1>(v, pl, i);
-    half_bitonic_step_kv<16, 8>(v, pl, i);
-    half_bitonic_step_kv<16, 4>(v, pl, i);
-    half_bitonic_step_kv<16, 2>(v, pl, i);
-    half_bitonic_step_kv<16, 1>(v, pl, i);
-    half_bitonic_step_kv<32, 16>(v, pl, i);
-    half_bitonic_step_kv<32, 8>(v, pl, i);
-    half_bitonic_step_kv<32, 4>(v, pl, i);
-    half_bitonic_step_kv<32, 2>(v, pl, i);
-    half_bitonic_step_kv<32, 1>(v, pl, i);
-}
+// When only some lanes' buffers are full, the wave cuts them back two at a time, one per
+// half-wave: lane i of a half holds entry i of its buffer, and its key's rank among the 32
+// (they differ) is counted against all of them, broadcast from LDS. The 32 comparisons do
+// not wait for each other, as the 15 steps of a sorting network do: waves of stacked nodes,
+// the last of a launch to end, spend most of their time here (495 k nodes in the voxel
+// field: 2.31 -> 2.23 ms a rebuild).
 
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, int l) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
@@ -712,7 +638,7 @@ struct WaveQueries {
 // order); their cnt becomes the bars left and kth the 24th key when there are 24. All
 // lanes take part: the exact test and the keys are formed from the slots, relative to the
 // owner's query.
-__device__ __forceinline__ void settle_slot_lanes(uint32_t* cb, int lane, uint64_t sm, int& cnt, uint64_t& kth,
+__device__ __forceinline__ void settle_slot_lanes(uint32_t* cb, uint64_t* keys, int lane, uint64_t sm, int& cnt, uint64_t& kth,
                                                   const float4* __restrict__ Ps, const int2* __restrict__ Ms,
                                                   const WaveQueries& Q, float half) {
     // the pair of lanes settled next, with its entries already on their way while the pair
@@ -749,13 +675,24 @@ __device__ __forceinline__ void settle_slot_lanes(uint32_t* cb, int lane, uint64
         if (more) {   // (of other lanes than a0 and b0: their columns are not written below)
             next();
         }
-        half_wave_sort32_kv(v, slot, lane);
-        if (i < kK) {
-            cb[i * kTrussWave + (lo ? a0 : b0)] = (uint32_t)slot;
+        keys[lane] = v;
+        __syncthreads();
+        const ulonglong2* mine = reinterpret_cast<const ulonglong2*>(keys + (lane & 32));
+        int rank = 0;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const ulonglong2 k = mine[e];
+            rank += (k.x < v ? 1 : 0) + (k.y < v ? 1 : 0);
         }
-        const uint64_t bars = __ballot(v != ~0ull);
+        const bool bars1 = v != ~0ull;
+        if (bars1 && rank < kK) {
+            cb[rank * kTrussWave + (lo ? a0 : b0)] = (uint32_t)slot;
+        }
+        const uint64_t bars = __ballot(bars1), last = __ballot(bars1 && rank == kK - 1);
         const int na = __popcll(bars & 0xFFFFFFFFull), nb = __popcll(bars >> 32);
-        const uint64_t ka = readlane64(v, kK - 1), kb = readlane64(v, 32 + kK - 1);
+        const uint32_t la = (uint32_t)last, lb = (uint32_t)(last >> 32);
+        const uint64_t ka = la ? readlane64(v, __ffs((int)la) - 1) : ~0ull;
+        const uint64_t kb = lb ? readlane64(v, 32 + __ffs((int)lb) - 1) : ~0ull;
         if (lane == a0) {
             cnt = min(na, kK);
             kth = ka;
@@ -764,6 +701,7 @@ __device__ __forceinline__ void settle_slot_lanes(uint32_t* cb, int lane, uint64
             cnt = min(nb, kK);
             kth = kb;
         }
+        __syncthreads();   // the keys are read
         if (!more) {
             break;
         }
@@ -939,10 +877,13 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
     // the row table of the current group: cell-start indices of the row's first cell and
     // one past its last, the lanes that scan the row, its level; after the cell starts
     // are read: the row's first slot and its position in the concatenation
-    __shared__ int r_key0[kMaxRanges], r_key1[kMaxRanges], r_lev[kMaxRanges], r_sa[kMaxRanges], r_beg[kMaxRanges],
-        r_len[kMaxRanges];
-    // a round's (query lane, candidate) pairs; the row keys are read before any round
-    static_assert(kMaxRanges >= kTrussWave, "the pairs share the row keys' array");
+    __shared__ int r_lev[kMaxRanges], r_sa[kMaxRanges], r_beg[kMaxRanges], r_len[kMaxRanges];
+    // the rows' keys are read before any round: a settling's sort keys take their place, and a
+    // round's (query lane, candidate) pairs
+    __shared__ __align__(16) uint64_t r_keys[kMaxRanges];
+    static_assert(kMaxRanges >= kTrussWave, "the pairs and sort keys share the row keys' array");
+    int* const r_key0 = reinterpret_cast<int*>(r_keys);
+    int* const r_key1 = r_key0 + kMaxRanges;
     int* const pairs = r_key0;
     __shared__ uint64_t r_mask[kMaxRanges];
     __shared__ uint32_t cb[kCollect * kTrussWave];   // the lanes' lists (candidate slots)
@@ -979,6 +920,10 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
             grow = (Li << 26) | ((cz / kBrickEdge) << 13) | (cy / kBrickEdge);
             gx = cell_coord(H, Li, px, H.ox, 0) / kBrickEdge;
         }
+        // the label of the wave's interior queries, if they have one in common
+        const uint64_t qint = __ballot(ti_int != 0);
+        const int wl = qint ? __builtin_amdgcn_readlane(li, __builtin_ctzll(qint)) : 0;
+        const bool one_label = __ballot(ti_int && li != wl) == 0ull;
         bool pending = active;
         // The lane's buffer holds cnt keys; once it has been cut back to the 24 best, kth is
         // the 24th of them, and a candidate must come before it to enter.
@@ -1030,7 +975,10 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                 const int rows = nr;
                 nr = 0;
                 __syncthreads();
-                // The candidates of chunk base + 64 are loaded while chunk base is tested.
+                // The candidates of chunk base + 64 are loaded while chunk base is tested: always,
+                // past the end slot 0's. (With the loads under a branch, the wait for the chunk's
+                // own candidates has to hold on the path without them too, and waits for the loads
+                // just issued: 2.5 M nodes 1.35 instead of 1.31 ms a rebuild.)
                 int rfirst = 0;   // the row holding the loaded chunk's first candidate
                 float4 npos;
                 int2 nms;
@@ -1041,37 +989,31 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                     }
                     const int p = base + cidx;
                     int lo = rfirst;   // the candidate's row: the last that starts at or before p
-                    if (p < total) {
-                        while (lo + 1 < rows && r_beg[lo + 1] <= p) {
-                            ++lo;
-                        }
-                        const int s = r_sa[lo] + (p - r_beg[lo]);
-                        npos = in.Ps[s];
-                        nms = in.Ms[s];
-                        nslot = s;
-                    } else {   // past the end: far away, it fails every test
-                        npos = make_float4(inf, inf, inf, 0.0f);
-                        nms = make_int2(-1, 0);
-                        nslot = 0;
+                    while (lo + 1 < rows && r_beg[lo + 1] <= p) {
+                        ++lo;
                     }
+                    const int s = p < total ? r_sa[lo] + (p - r_beg[lo]) : 0;
+                    npos = in.Ps[s];
+                    nms = in.Ms[s];
+                    nslot = s;
                     nrow = lo;
                 };
                 fetch(0);
                 for (int base = 0; base < total; base += kTrussWave) {
                     __syncthreads();   // the previous chunk is consumed
                     cslot[cidx] = nslot;
-                    const float4 mine_c = npos;
-                    const int2 mine_m = nms;
+                    // past the end: far away, it fails every test
+                    const bool some = base + cidx < total;
+                    const float4 mine_c = some ? npos : make_float4(inf, inf, inf, 0.0f);
+                    const int2 mine_m = some ? nms : make_int2(-1, 0);
                     if (cut) {
-                        cpos[cidx] = npos;
-                        cid[cidx] = nms.x;
+                        cpos[cidx] = mine_c;
+                        cid[cidx] = mine_m.x;
                         crow[cidx] = nrow;
                     }
                     const int mine_row = nrow;
                     __syncthreads();
-                    if (base + kTrussWave < total) {
-                        fetch(base + kTrussWave);
-                    }
+                    fetch(base + kTrussWave);
                     uint64_t hit = chunk_hits(qops, mine_c, gox, goy, goz, k2, margin);
                     if (!H.prune) {
                         // the candidates of the rows this lane scans (its level range, its own
@@ -1089,7 +1031,13 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                         hit &= elig;
                     }
                     hit = ingroup ? hit : 0ull;
-                    {   // no bar between interior nodes of two labels
+                    // no bar between interior nodes of two labels
+                    if (one_label) {   // (one mask then: 1.42 -> 1.35 ms for 2.5 M nodes)
+                        const uint64_t foreign = __ballot((mine_m.y & 0xFF) == TN_INTERIOR && (mine_m.y >> 8) != wl && mine_m.x >= 0);
+                        if (foreign) {
+                            hit = ti_int ? hit & ~by_index(foreign) : hit;
+                        }
+                    } else {
                         const bool inside = (mine_m.y & 0xFF) == TN_INTERIOR;
                         const int cl = mine_m.y >> 8;
                         uint64_t left = by_index(__ballot(inside && mine_m.x >= 0));
@@ -1128,7 +1076,7 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                         // little room for them: keep the 24 best so far
                         const uint64_t sm = __ballot(pc > kCollect - cnt && kCollect - cnt < kMinRoom);
                         if (sm) {
-                            settle_slot_lanes(cb, lane, sm, cnt, kth, in.Ps, in.Ms, Q, half);
+                            settle_slot_lanes(cb, r_keys, lane, sm, cnt, kth, in.Ps, in.Ms, Q, half);
                             near = true;
                         }
                         const int want = min(pc, kCollect - cnt);
@@ -1287,7 +1235,7 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
 // order, its rows and the neighbours' positions are read and written whole lines at a time;
 // at the end of k_truss, whose lanes hold nodes in brick order, the same work was a gather
 // of the ids, one of their slots and 24 scattered stores a node, its 64 key registers
-// bounding the search (2.5 M nodes: 2.25 ms in one kernel, 1.42 + 0.22 ms in two). The
+// bounding the search (2.5 M nodes: 2.25 ms in one kernel, 1.31 + 0.22 ms in two). The
 // keys are (distance, slot): the ids are read only in a wave where two distances tie, whose
 // lanes then sort by (distance, id) and look the slots up (neighbours exchanged until all
 // ids are in order took up to a pass a tied entry: 152 us instead of 80 for 495 k nodes in
