@@ -2195,7 +2195,13 @@ struct CtlArgs {
 // (n + 64) * 2^-53 * A of the exact sum, so when |S| exceeds twice that bound both
 // have the exact sum's sign. Otherwise the serial sum is recomputed here, in index
 // order, exactly as the CPU does.
-__device__ __forceinline__ void k_control_body(CtlArgs ca, Ctl* __restrict__ ctl, const double2* __restrict__ partials, const float* __restrict__ pw, const int32_t* __restrict__ slot_of, int bid, int nblk) {
+//
+// The control block goes to the host from here, by stores to pinned memory (host, if it is
+// not null), and the own-list refreshes are launched after the event that the host waits
+// for: a copy between the refreshes and the event cost each iteration its own latency, and
+// the host enqueued the next iteration only after both (75 k nodes to convergence: 45.2 ->
+// 40.5 ms, 270 iterations; 435 k nodes, 100 iterations: 42.1 -> 41.2).
+__device__ __forceinline__ void k_control_step(CtlArgs ca, Ctl* __restrict__ ctl, const double2* __restrict__ partials, const float* __restrict__ pw, const int32_t* __restrict__ slot_of, int bid, int nblk) {
     __shared__ double red[kBlock][2];
     __shared__ float chunk[kScanTile];
     __shared__ int use_serial;
@@ -2294,8 +2300,24 @@ __device__ __forceinline__ void k_control_body(CtlArgs ca, Ctl* __restrict__ ctl
     ctl->mmax_bits = 0;
 }
 
-__global__ __launch_bounds__(kBlock) void k_control(CtlArgs ca, Ctl* __restrict__ ctl, const double2* __restrict__ partials, const float* __restrict__ pw, const int32_t* __restrict__ slot_of) {
-    k_control_body(ca, ctl, partials, pw, slot_of, blockIdx.x, gridDim.x);
+// the control, then the block to the host (host may be null)
+__device__ __forceinline__ void k_control_body(CtlArgs ca, Ctl* __restrict__ ctl, const double2* __restrict__ partials, const float* __restrict__ pw, const int32_t* __restrict__ slot_of, Ctl* host, int bid, int nblk) {
+    k_control_step(ca, ctl, partials, pw, slot_of, bid, nblk);
+    if (!host) {
+        return;
+    }
+    __syncthreads();   // the first thread's stores are done
+    static_assert(sizeof(Ctl) % 4 == 0, "Ctl is copied in words");
+    const volatile uint32_t* src = reinterpret_cast<const volatile uint32_t*>(ctl);
+    volatile uint32_t* dst = reinterpret_cast<volatile uint32_t*>(host);
+    for (int k = threadIdx.x; k < (int)(sizeof(Ctl) / 4); k += kBlock) {
+        dst[k] = src[k];
+    }
+    __threadfence_system();
+}
+
+__global__ __launch_bounds__(kBlock) void k_control(CtlArgs ca, Ctl* __restrict__ ctl, const double2* __restrict__ partials, const float* __restrict__ pw, const int32_t* __restrict__ slot_of, Ctl* host) {
+    k_control_body(ca, ctl, partials, pw, slot_of, host, blockIdx.x, gridDim.x);
 }
 
 // ---- grouped launches: one launch runs an iteration's kernel for many plans -------
@@ -2399,23 +2421,9 @@ __global__ __launch_bounds__(kWave) void kg_truss_node(const PlanIter* __restric
 
 __global__ __launch_bounds__(kBlock) void kg_control(const PlanIter* __restrict__ tab,
                                                      const int32_t* __restrict__ bplan,
-                                                     const int32_t* __restrict__ bfirst) {
+                                                     const int32_t* __restrict__ bfirst, Ctl* host) {
     TN_PLAN_BLOCK(kShOne);
-    k_control_body(P.ca, P.ctl, P.partials, P.pw, P.slot_of, bid_, nb_);
-}
-
-// every plan's control block into one array (one copy to the host)
-__global__ void kg_ctl_gather(const PlanIter* __restrict__ tab, const int32_t* __restrict__ bplan,
-                              const int32_t* __restrict__ bfirst, Ctl* __restrict__ out) {
-    TN_PLAN_BLOCK(kShOne);
-    (void)bid_;
-    (void)nb_;
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(P.ctl);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(out + v_);
-    static_assert(sizeof(Ctl) % 4 == 0, "Ctl is copied in words");
-    for (int k = threadIdx.x; k < (int)(sizeof(Ctl) / 4); k += blockDim.x) {
-        dst[k] = src[k];
-    }
+    k_control_body(P.ca, P.ctl, P.partials, P.pw, P.slot_of, host + v_, bid_, nb_);
 }
 
 #undef TN_PLAN_BLOCK

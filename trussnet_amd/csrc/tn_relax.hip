@@ -526,9 +526,10 @@ struct KernelTimer {
         TN_HIP(hipEventRecord(b, s ? s : stream));
         pending.push_back({ kc, a, b });
     }
-    void collect() {   // the stream has been synchronised
+    void collect() {
         for (const Rec& r : pending) {
             float t = 0;
+            TN_HIP(hipEventSynchronize(r.b));   // (an iteration's last launch may still run)
             TN_HIP(hipEventElapsedTime(&t, r.a, r.b));
             ms[r.kc] += t;
             launches[r.kc] += 1;
@@ -897,7 +898,7 @@ struct tn_plan {
         enqueue_iteration_tail();
     }
 
-    // stats, own-list refreshes, control, and the control block's copy to the host
+    // stats, control (which hands the control block to the host), own-list refreshes
     void enqueue_iteration_tail() {
         hipEvent_t t = timer.begin(KC_STATS);
         tnk::k_stats<<<nparts, tnk::kBlock, 0, stream>>>(dX, dP0, dMv, dPw, n, prm.skin, fire, dThr, dCtl, dQueue,
@@ -907,15 +908,17 @@ struct tn_plan {
         // skipped when a rebuild or the loop's end follows
         t = timer.begin(KC_CONTROL);
         tnk::CtlArgs ca{ n, prm.max_iters, fire, rebuild_div, prm.dptol, nparts, force_serial };
-        tnk::k_control<<<1, tnk::kBlock, 0, stream>>>(ca, dCtl, dPartials, dPw, dSlotOf);
+        tnk::k_control<<<1, tnk::kBlock, 0, stream>>>(ca, dCtl, dPartials, dPw, dSlotOf, ev_iter ? hCtl : nullptr);
         timer.end(KC_CONTROL, t);
+        if (ev_iter) {   // the host goes on from here
+            TN_HIP(hipEventRecord(ev_iter, stream));
+        }
         t = timer.begin(KC_REFRESH);
         tnk::k_truss_node<<<refresh_blocks, tnk::kWave, 0, stream>>>(H, truss_in(), n, dQueue, dCtl, dNbr, dNnb, dP0);
         timer.end(KC_REFRESH, t);
         TN_HIP(hipGetLastError());
-        TN_HIP(hipMemcpyAsync(hCtl, dCtl, sizeof(tnk::Ctl), hipMemcpyDeviceToHost, stream));
-        if (ev_iter) {
-            TN_HIP(hipEventRecord(ev_iter, stream));
+        if (!ev_iter) {   // (hCtl is pageable)
+            TN_HIP(hipMemcpyAsync(hCtl, dCtl, sizeof(tnk::Ctl), hipMemcpyDeviceToHost, stream));
         }
     }
 
@@ -1923,7 +1926,6 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
     DevMem gm;
     gm.device = plans[0]->device;
     tnk::PlanIter* dtab = gm.alloc<tnk::PlanIter>(count);
-    tnk::Ctl* dctl = gm.alloc<tnk::Ctl>(count);
     // pinned host copies: the table rows, the control blocks, the block maps
     struct Pinned {
         void* p = nullptr;
@@ -2056,11 +2058,9 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
             moves(tnd::Field{});
         }
         kg_stats<<<nblocks[kShParts], kBlock, 0, bs>>>(dtab, bplan[kShParts], bfirst[kShParts]);
-        kg_control<<<nblocks[kShOne], kBlock, 0, bs>>>(dtab, bplan[kShOne], bfirst[kShOne]);
+        kg_control<<<nblocks[kShOne], kBlock, 0, bs>>>(dtab, bplan[kShOne], bfirst[kShOne], hctl);
         kg_truss_node<<<nblocks[kShRefresh], kWave, 0, bs>>>(dtab, bplan[kShRefresh], bfirst[kShRefresh]);
-        kg_ctl_gather<<<nblocks[kShOne], 64, 0, bs>>>(dtab, bplan[kShOne], bfirst[kShOne], dctl);
         TN_HIP(hipGetLastError());
-        TN_HIP(hipMemcpyAsync(hctl, dctl, sizeof(tnk::Ctl) * count, hipMemcpyDeviceToHost, bs));
         TN_HIP(hipStreamSynchronize(bs));
         ++launches;
         if (tuning) {
