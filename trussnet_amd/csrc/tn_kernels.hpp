@@ -983,16 +983,37 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                 float4 npos;
                 int2 nms;
                 int nrow, nslot;
+                bool nin;
+                // Once a buffer has filled, the chunks left take their candidates evenly spread
+                // over what is left of the concatenation, from sfirst on, sstep of them: in the
+                // rows' order the distances fall as the scan comes up to a node, so that almost
+                // every candidate beats the 24th so far and the buffers fill again and again (495 k
+                // nodes in the voxel field: 2.25 -> 1.65 ms a rebuild).
+                int sfirst = -1, sstep = 1;
                 auto fetch = [&](int base) {
-                    while (rfirst + 1 < rows && r_beg[rfirst + 1] <= base) {
-                        ++rfirst;
+                    if (sfirst < 0 && near && H.prune) {
+                        sfirst = base;
+                        sstep = (total - base + kTrussWave - 1) / kTrussWave;
                     }
-                    const int p = base + cidx;
-                    int lo = rfirst;   // the candidate's row: the last that starts at or before p
-                    while (lo + 1 < rows && r_beg[lo + 1] <= p) {
-                        ++lo;
+                    int p, lo;   // the candidate and its row: the last that starts at or before it
+                    if (sfirst < 0) {
+                        while (rfirst + 1 < rows && r_beg[rfirst + 1] <= base) {
+                            ++rfirst;
+                        }
+                        p = base + cidx;
+                        lo = rfirst;
+                        while (lo + 1 < rows && r_beg[lo + 1] <= p) {
+                            ++lo;
+                        }
+                    } else {
+                        p = sfirst + cidx * sstep + (base - sfirst) / kTrussWave;
+                        lo = 0;
+                        for (int d = kMaxRanges / 2; d > 0; d >>= 1) {
+                            lo = lo + d < rows && r_beg[lo + d] <= p ? lo + d : lo;
+                        }
                     }
-                    const int s = p < total ? r_sa[lo] + (p - r_beg[lo]) : 0;
+                    nin = p < total;
+                    const int s = nin ? r_sa[lo] + (p - r_beg[lo]) : 0;
                     npos = in.Ps[s];
                     nms = in.Ms[s];
                     nslot = s;
@@ -1003,7 +1024,7 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                     __syncthreads();   // the previous chunk is consumed
                     cslot[cidx] = nslot;
                     // past the end: far away, it fails every test
-                    const bool some = base + cidx < total;
+                    const bool some = nin;
                     const float4 mine_c = some ? npos : make_float4(inf, inf, inf, 0.0f);
                     const int2 mine_m = some ? nms : make_int2(-1, 0);
                     if (cut) {
