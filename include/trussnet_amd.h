@@ -114,7 +114,9 @@ typedef struct tn_nodes_view {
  * in RelaxStats) counts the FIRE iterations whose power sign the device could not
  * certify from its tree sum and took from the serial sum in node order, the CPU's
  * own summation (src/v2m_particles.cpp:849-855). Setting TN_SERIAL_POWER=1 in the
- * environment before a plan is created makes every FIRE iteration take that path. */
+ * environment before a plan is created makes every FIRE iteration take that path;
+ * TN_STATS_BLOCKS=b has the per-iteration statistics run in b blocks at most (a launch
+ * shape: fewer blocks walk more nodes each, and no result depends on it). */
 typedef struct tn_relax_stats {
     int32_t iters, rebuilds;
     float last_move, last_p99;

@@ -2017,16 +2017,19 @@ __device__ __forceinline__ int hist_bin(float m, const float* __restrict__ thr) 
 
 constexpr int kHistThr = 35;   // exponents -21..13
 constexpr int kStatsBlocks = 2048;   // k_stats' grid at most (8 blocks per CU)
+constexpr int kHeldChunks = 8;       // chunks of nodes after which a block writes out what it lists
 
 // Per iteration: the histogram, the largest move, the count past skin/2, the
 // nodes past a full skin (listed: their own lists are refreshed), and FIRE's
 // power partial sums (src/v2m_particles.cpp:849-937). Counts are reduced per
 // wave with ballots before any atomic, and the listed nodes gathered in LDS, so that a
 // block takes its place in the list once (a pass of its own over a flag a node, as
-// before, cost 8 us an iteration at 2.5 M nodes and a launch at any size).
+// before, cost 8 us an iteration at 2.5 M nodes and a launch at any size). LDS holds
+// every node of kHeldChunks chunks, and the block writes the list out after that many
+// whatever it holds: the chunk's number is the same in every wave, while the count held
+// may already be another wave's next, and the writing has barriers that all must reach.
 __device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const float4* __restrict__ P0, const float* __restrict__ mv, const float* __restrict__ pw, int n, float skin, int fire, const float* __restrict__ thr, Ctl* __restrict__ ctl, int32_t* __restrict__ refresh, double2* __restrict__ partials, int bid, int nblk) {
-    constexpr int kHeld = 4 * kBlock;
-    __shared__ int held[kHeld];   // nodes to list
+    __shared__ int held[kHeldChunks * kBlock];   // nodes to list
     __shared__ int nheld, held_at;
     __shared__ uint32_t lh[32];
     __shared__ uint32_t lmax;
@@ -2048,7 +2051,7 @@ __device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const
     // every thread of the block: the held nodes into the list
     auto list_held = [&]() {
         const int m = nheld;
-        if (tid == 0) {
+        if (tid == 0 && m) {
             held_at = atomicAdd(&ctl->nrefresh, m);
         }
         __syncthreads();
@@ -2062,13 +2065,16 @@ __device__ __forceinline__ void k_stats_body(const float4* __restrict__ X, const
         __syncthreads();
     };
     double bs = 0.0, ba = 0.0;   // this block's power partial sums (thread 0), chunk by chunk
+    int chunks = 0;              // chunks since the block last wrote its list out
     // chunks of kBlock nodes, grid-strided: each block adds its counts to the control
     // block once, and its partial sums have a fixed shape
     for (int c = bid; (int64_t)c * kBlock < n; c += nblk) {
-        __syncthreads();   // lps of the previous chunk has been read
-        if (nheld > kHeld - kBlock) {
+        __syncthreads();   // lps of the previous chunk has been read, its nodes are held
+        if (chunks == kHeldChunks) {
             list_held();
+            chunks = 0;
         }
+        ++chunks;
         const int i = c * kBlock + tid;
         double ps = 0.0, pa = 0.0;
         int bin = -1;

@@ -1152,7 +1152,11 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
         }
         const int64_t scan_max = std::max<int64_t>(p->nkeys, p->bricks.size) + 1;
         p->dBsum = p->alloc<int32_t>(blocks_for(scan_max, tnk::kScanTile));
-        p->nparts = (int)std::max<unsigned>(1, std::min<unsigned>(blocks_for(n, tnk::kBlock), tnk::kStatsBlocks));
+        {
+            const char* e = std::getenv("TN_STATS_BLOCKS");
+            const int most = e && e[0] ? std::atoi(e) : tnk::kStatsBlocks;
+            p->nparts = std::max(1, std::min({ (int)blocks_for(n, tnk::kBlock), tnk::kStatsBlocks, most }));
+        }
         p->refresh_blocks = (int)std::max<int64_t>(1, std::min<int64_t>(n, 2048));   // one wave per listed node
         p->dPartials = p->alloc<double2>(std::max(p->nparts, 1));
         p->dThr = p->alloc<float>(tnk::kHistThr);
