@@ -1,7 +1,8 @@
 """The K-nearest lists where their kernels change course, against the oracle's rebuild, bit
 for bit: equal distances (by id then), lists just below and above 24 and 32 candidates (the
 row, its tail, the buffers cut back), nodes that lie on each other, waves and blocks that
-are not full, and a grid with cells smaller than the bars reach.
+are not full, a grid with cells smaller than the bars reach, and bars that end past the cells
+the reference visits by a rounding.
 """
 import dataclasses
 
@@ -97,3 +98,68 @@ def test_reach_beyond_the_cells(tn, hmax, density):
     rng = np.random.default_rng(11)
     P = rng.uniform(0, 48, (int(density * 20000), 3))
     same_lists(tn, grid, nodes_at(grid, P, types=(0, 1)))
+
+
+def past_the_region(hmin, prm, want, seed):
+    """(size, place, place of the other) along an axis with voxels of 1: two nodes in the first
+    and the third row of cells of the lowest level, the lower one of that size, the upper one of
+    size hmin, such that they are a bar by the 32-bit test while the upper one's cell lies just
+    past the lower one's scan region: rounding puts the bar's reach (t + skin) (h_i + h_j) / 2 two
+    units above the region's ((t + skin) h_i + b) / 2, b the edge of the cells."""
+    f = np.float32
+    T = f(prm.t) + f(prm.skin)
+    half, b = T * f(0.5), T * hmin
+
+    def cell(x):
+        return int(np.floor((x + f(0.5)) / b))
+
+    edge = f(2) * b - f(0.5)   # the first place of the third row
+    while cell(edge) >= 2:
+        edge = np.nextafter(edge, f(-1))
+    while cell(edge) < 2:
+        edge = np.nextafter(edge, f(9))
+    rng = np.random.default_rng(seed)
+    out = []
+    while len(out) < want:
+        hi = hmin * f(rng.uniform(1.05, 1.5))
+        r, rj = f(0.5) * (T * hi + b), half * (hi + hmin)
+        if (rj - r) / np.spacing(r) < 2:
+            continue
+        p = f(np.float64(edge) - np.float64(r) - np.float64(np.spacing(r)))
+        e = edge - p
+        if e * e < rj * rj and cell(p + r) < 2:
+            out.append((hi, p, edge))
+    return out
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_bars_just_past_the_scan_region(tn, axis):
+    """A candidate that passes the test of distance by its last bit, in a cell that the
+    reference does not visit for the node: not in the list"""
+    prm = RelaxParams()
+    hmin = np.float32(1.0129207)
+    pairs = past_the_region(hmin, prm, 12, axis)
+    base = Fixture("jitter64").grid
+    grid = dataclasses.replace(base, hmin=float(hmin), hmax=float(2 * hmin), h=np.full(base.h.size, hmin, np.float32))
+    h = grid.h.reshape(grid.nz, grid.ny, grid.nx)
+    P, low, up = [], [], []
+    for k, (hi, lo, hi_place) in enumerate(pairs):
+        a, b = 6.0 + 9.0 * (k % 4), 8.0 + 9.0 * (k // 4)   # (out of the other pairs' reach)
+        for place, size in ((lo, hi), (hi_place, hmin), (np.float32(1.6), hi)):   # the third: scans that cell for its own list
+            p = np.insert(np.array([a, b], np.float32), axis, place)
+            if size == hmin:
+                up.append(len(P))
+            elif place == lo:
+                low.append(len(P))
+            if place == np.float32(1.6):
+                p[(axis + 1) % 3] += np.float32(1.0)
+            x, y, z = np.floor(p + 0.5).astype(int)
+            h[z, y, x] = size
+            P.append(p)
+    nodes = nodes_at(grid, P)
+    nodes.lab[:] = 1
+    want = orc.rebuild(grid, nodes, prm)
+    for i, j in zip(low, up):   # a bar by its length, and not in the list
+        assert j not in want["nbr"].reshape(-1, 24)[i][: want["nnb"][i]]
+        assert i in want["nbr"].reshape(-1, 24)[j][: want["nnb"][j]]
+    same_lists(tn, grid, nodes, prm)

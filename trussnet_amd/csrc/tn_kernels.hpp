@@ -506,11 +506,11 @@ __global__ __launch_bounds__(kBlock) void k_permute(const int32_t* __restrict__ 
 // interior bar across labels): in k_lists, or here once a buffer fills, which is then cut
 // back to its 24 best. k_lists keeps the first 24 in (distance, id) order. The list equals
 // the reference's:
-// its K smallest valid candidates in (distance, id) order, and every valid
-// candidate lies inside the lane's own box, which the union contains. (That holds
-// when every node's reach fits its level's cell, H.prune; otherwise a lane also
-// checks that the candidate's cell is in its own box, the reference's scan region,
-// before accepting it.)
+// its K smallest valid candidates in (distance, id) order, of those in the cells of the
+// lane's own box, the reference's scan region. Where every node's reach fits its level's
+// cell (H.prune) a bar ends inside the box but for the rounding of the two reaches, so
+// only a bar that could be past it by that (kDoubtful) is asked for its cells; otherwise
+// every one is.
 
 constexpr int kTrussWave = 64;   // one wave per block
 constexpr int kCollect = 32;   // per-lane candidate buffer (entries): settled by a 32-key network
@@ -628,6 +628,25 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
+// The reference looks for the other ends at level L in the cells from that of p - r to that
+// of p + r along each axis, r = ((t + skin) h_i + b_L) / 2. An end at most r from p has its
+// cell among them (rounding keeps order, so p + r does not round below it); past r, the
+// 32-bit difference is at least r and d^2 at least r^2 as rounded. A bar has d^2 < rj^2, rj =
+// (t + skin) / 2 (h_i + h_j), and b_L >= (t + skin) h_j as rounded: r >= rj (1 - 4 u), u =
+// 2^-24, so a bar past the cells has d^2 >= rj^2 (1 - 11 u), the squares' and the product's
+// own roundings counted. The bars from kDoubtful rj^2 on (32 u) are asked for their cells.
+constexpr float kDoubtful = 1.0f - 0x1p-19f;
+
+// whether the candidate c at level L lies in the reference's scan region of the node at
+// (x, y, z) of reach R (v2m_neighbors, src/opencl/v2m_particle_body.cl:73-151)
+__device__ __forceinline__ bool in_region(const Hash& H, int L, float x, float y, float z, float R, float4 c) {
+    const float r = 0.5f * (R + H.b0 * (float)(1 << L));
+    const int cx = cell_coord(H, L, c.x, H.ox, 0), cy = cell_coord(H, L, c.y, H.oy, 1), cz = cell_coord(H, L, c.z, H.oz, 2);
+    return cx >= cell_coord(H, L, x - r, H.ox, 0) && cx <= cell_coord(H, L, x + r, H.ox, 0) &&
+           cy >= cell_coord(H, L, y - r, H.oy, 1) && cy <= cell_coord(H, L, y + r, H.oy, 1) &&
+           cz >= cell_coord(H, L, z - r, H.oz, 2) && cz <= cell_coord(H, L, z + r, H.oz, 2);
+}
+
 // A wave's queries, lane by lane (the search's view of its 64 nodes).
 struct WaveQueries {
     float px, py, pz, h;   // position and size
@@ -640,7 +659,7 @@ struct WaveQueries {
 // owner's query.
 __device__ __forceinline__ void settle_slot_lanes(uint32_t* cb, uint64_t* keys, int lane, uint64_t sm, int& cnt, uint64_t& kth,
                                                   const float4* __restrict__ Ps, const int2* __restrict__ Ms,
-                                                  const WaveQueries& Q, float half) {
+                                                  const WaveQueries& Q, const Hash& H, float half) {
     // the pair of lanes settled next, with its entries already on their way while the pair
     // before it is sorted (a wave of stacked nodes settles a hundred times in a row)
     const bool lo = lane < 32;
@@ -667,8 +686,12 @@ __device__ __forceinline__ void settle_slot_lanes(uint32_t* cb, uint64_t* keys, 
         const int qa = __builtin_amdgcn_readlane(Q.slot, a), qb = __builtin_amdgcn_readlane(Q.slot, b);
         const float ex = c.x - (lo ? xa : xb), ey = c.y - (lo ? ya : yb), ez = c.z - (lo ? za : zb);
         const float d2 = ex * ex + ey * ey + ez * ez;
-        const float rj = half * ((lo ? ha : hb) + c.w);
-        const bool bar = in && d2 < rj * rj && sl != (lo ? qa : qb);
+        const float rj = half * ((lo ? ha : hb) + c.w), rj2 = rj * rj;
+        bool bar = in && d2 < rj2 && sl != (lo ? qa : qb);
+        if (bar && d2 >= kDoubtful * rj2) {
+            const float T = 2.0f * half;
+            bar = in_region(H, level_for(H, T * c.w), lo ? xa : xb, lo ? ya : yb, lo ? za : zb, T * (lo ? ha : hb), c);
+        }
         uint64_t v = bar ? list_key(sqrtf(d2), id) : ~0ull;
         int slot = sl;
         const bool more = sm != 0;
@@ -1038,8 +1061,8 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                     uint64_t hit = chunk_hits(qops, mine_c, gox, goy, goz, k2, margin);
                     if (!H.prune) {
                         // the candidates of the rows this lane scans (its level range, its own
-                        // box); where every reach fits its level's cell, a candidate that passes
-                        // the exact test is in the lane's own box without being asked
+                        // box); where every reach fits its level's cell, only the bars that could
+                        // be past the box by rounding are asked, where their lengths are formed
                         const int cn = min(kTrussWave, total - base);
                         uint64_t elig = 0;
                         const int r0 = crow[0], r1 = crow[cn - 1];
@@ -1097,7 +1120,7 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                         // little room for them: keep the 24 best so far
                         const uint64_t sm = __ballot(pc > kCollect - cnt && kCollect - cnt < kMinRoom);
                         if (sm) {
-                            settle_slot_lanes(cb, r_keys, lane, sm, cnt, kth, in.Ps, in.Ms, Q, half);
+                            settle_slot_lanes(cb, r_keys, lane, sm, cnt, kth, in.Ps, in.Ms, Q, H, half);
                             near = true;
                         }
                         const int want = min(pc, kCollect - cnt);
@@ -1126,14 +1149,10 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                             cs = cslot[k];
                             const float ex = c.x - ox_, ey = c.y - oy_, ez = c.z - oz_;
                             const float d2 = ex * ex + ey * ey + ez * ez;
-                            const float rj = half * (oh + c.w);
-                            valid = d2 < rj * rj && cs != oslot;   // a bar, and not the node itself
-                            if (valid && !H.prune) {   // the reference's own scan region only
-                                const int L = r_lev[crow[k]];
-                                const float rr = 0.5f * (tskin * oh + H.b0 * (float)(1 << L));
-                                const int cx = cell_coord(H, L, c.x, H.ox, 0);
-                                valid = cx >= cell_coord(H, L, ox_ - rr, H.ox, 0) &&
-                                        cx <= cell_coord(H, L, ox_ + rr, H.ox, 0);
+                            const float rj = half * (oh + c.w), rj2 = rj * rj;
+                            valid = d2 < rj2 && cs != oslot;   // a bar, and not the node itself
+                            if (valid && (!H.prune || d2 >= kDoubtful * rj2)) {   // the reference's own scan region only
+                                valid = in_region(H, r_lev[crow[k]], ox_, oy_, oz_, tskin * oh, c);
                             }
                             valid = valid && list_key(sqrtf(d2), cid[k]) < okth;
                         }
@@ -1262,12 +1281,13 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
 // ids are in order took up to a pass a tied entry: 152 us instead of 80 for 495 k nodes in
 // the voxel field). Bound by the gathers of the positions.
 template <int N>
-__device__ __forceinline__ int sort_row(const float4* __restrict__ Ps, const int2* __restrict__ Ms, int t, int m, float4 xi,
-                                        float half, const int4* __restrict__ row, const int4* __restrict__ tail0,
+__device__ __forceinline__ int sort_row(const Hash& H, const float4* __restrict__ Ps, const int2* __restrict__ Ms, int t,
+                                        int m, float4 xi, float half, const int4* __restrict__ row, const int4* __restrict__ tail0,
                                         const int4* __restrict__ tail1, const int32_t* __restrict__ slot_of,
                                         uint64_t (&k)[32]) {
     constexpr int kB = 8;
     int s[N];
+    uint32_t doubt = 0;   // the bars that could be past the scan region by rounding
 #pragma unroll
     for (int e = 0; e < N; e += 4) {
         const int4 j4 = e < kK ? row[e / 4] : (e == kK ? tail0[t] : tail1[t]);
@@ -1287,9 +1307,28 @@ __device__ __forceinline__ int sort_row(const float4* __restrict__ Ps, const int
         for (int e = 0; e < kB; ++e) {   // the reference's test (an entry past the row's end is the node itself)
             const float ex = x[e].x - xi.x, ey = x[e].y - xi.y, ez = x[e].z - xi.z;
             const float d2 = ex * ex + ey * ey + ez * ez;
-            const float rj = half * (xi.w + x[e].w);
-            const bool bar = d2 < rj * rj && s[e0 + e] != t;
+            const float rj = half * (xi.w + x[e].w), rj2 = rj * rj;
+            const bool bar = d2 < rj2 && s[e0 + e] != t;
             k[e0 + e] = bar ? list_key(sqrtf(d2), s[e0 + e]) : ~0ull;
+            doubt |= bar && d2 >= kDoubtful * rj2 ? 1u << (e0 + e) : 0u;
+        }
+    }
+#pragma clang loop unroll(disable)
+    while (doubt) {   // (rare)
+        const int at = __builtin_ctz(doubt);
+        doubt &= doubt - 1;
+        int j = t;
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            j = e == at ? (int)(uint32_t)k[e] : j;
+        }
+        const float4 c = Ps[j];
+        const float T = 2.0f * half;
+        if (!in_region(H, level_for(H, T * c.w), xi.x, xi.y, xi.z, T * xi.w, c)) {
+#pragma unroll
+            for (int e = 0; e < N; ++e) {
+                k[e] = e == at ? ~0ull : k[e];
+            }
         }
     }
     merge_sort<N>(k);
@@ -1316,7 +1355,7 @@ __device__ __forceinline__ int sort_row(const float4* __restrict__ Ps, const int
     return bars < kK ? bars : kK;
 }
 
-__global__ __launch_bounds__(kBlock) void k_lists(const float4* __restrict__ Ps, const int2* __restrict__ Ms, int n,
+__global__ __launch_bounds__(kBlock) void k_lists(Hash H, const float4* __restrict__ Ps, const int2* __restrict__ Ms, int n,
                                                   float half, int32_t* __restrict__ nbr, const int4* __restrict__ tail0,
                                                   const int4* __restrict__ tail1, const int32_t* __restrict__ slot_of,
                                                   int32_t* __restrict__ nnb) {
@@ -1327,8 +1366,8 @@ __global__ __launch_bounds__(kBlock) void k_lists(const float4* __restrict__ Ps,
     int4* row = reinterpret_cast<int4*>(nbr + (size_t)t * kK);
     const float4 xi = Ps[t];
     uint64_t k[32];
-    const int bars = __ballot(m > kK) ? sort_row<32>(Ps, Ms, t, m, xi, half, row, tail0, tail1, slot_of, k)
-                                      : sort_row<kK>(Ps, Ms, t, m, xi, half, row, tail0, tail1, slot_of, k);
+    const int bars = __ballot(m > kK) ? sort_row<32>(H, Ps, Ms, t, m, xi, half, row, tail0, tail1, slot_of, k)
+                                      : sort_row<kK>(H, Ps, Ms, t, m, xi, half, row, tail0, tail1, slot_of, k);
     if (valid) {
         nnb[t] = bars;
 #pragma unroll

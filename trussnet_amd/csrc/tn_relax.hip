@@ -773,7 +773,7 @@ struct tn_plan {
         tnk::k_brick_order<<<nb, tnk::kBlock, 0, stream>>>(H, bricks, dKeySorted, n, dCstart, dBrick, dSorted);
         tnk::k_truss<<<blocks_for(n, tnk::kTrussWave), tnk::kTrussWave, 0, stream>>>(
             H, truss_in(), n, dNbr, reinterpret_cast<int4*>(dXb), reinterpret_cast<int4*>(dVb), dNnb);
-        tnk::k_lists<<<nb, tnk::kBlock, 0, stream>>>(dPs, dMs, n, tskin * 0.5f, dNbr, reinterpret_cast<int4*>(dXb),
+        tnk::k_lists<<<nb, tnk::kBlock, 0, stream>>>(H, dPs, dMs, n, tskin * 0.5f, dNbr, reinterpret_cast<int4*>(dXb),
                                                      reinterpret_cast<int4*>(dVb), dSlotOf, dNnb);
         timer.end(KC_NEIGHBORS, t);
         TN_HIP(hipGetLastError());
