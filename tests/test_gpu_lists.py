@@ -2,7 +2,7 @@
 for bit: equal distances (by id then), lists just below and above 24 and 32 candidates (the
 row, its tail, the buffers cut back), nodes that lie on each other, waves and blocks that
 are not full, a grid with cells smaller than the bars reach, and bars that end past the cells
-the reference visits by a rounding.
+the reference visits by a rounding; in any unit of length.
 """
 import dataclasses
 
@@ -163,3 +163,19 @@ def test_bars_just_past_the_scan_region(tn, axis):
         assert j not in want["nbr"].reshape(-1, 24)[i][: want["nnb"][i]]
         assert i in want["nbr"].reshape(-1, 24)[j][: want["nnb"][j]]
     same_lists(tn, grid, nodes, prm)
+
+
+@pytest.mark.parametrize("power", [-62, -40, 40, 49, 54])
+@pytest.mark.parametrize("per", [20, 100])
+def test_any_unit_of_length(tn, power, per):
+    """Lengths scaled by a power of two: the same lists, down to squares near the smallest
+    normal number and up to squares near the largest; 20 nodes a place fill no buffer, 100 do"""
+    u = np.float32(2.0 ** power)
+    base = Fixture("jitter64").grid
+    grid = dataclasses.replace(base, vs=tuple(float(u * v) for v in base.vs), h=base.h * u, hmin=float(u * np.float32(base.hmin)),
+                               hmax=float(u * np.float32(base.hmax)))
+    rng = np.random.default_rng(per)
+    P = np.concatenate([np.repeat(rng.uniform(8, 14, (7, 3)), per, 0), rng.uniform(6, 20, (333, 3)), rng.uniform(40, 50, (5, 3))])
+    nodes = nodes_at(base, P[rng.permutation(len(P))])
+    nodes.P *= u
+    assert same_lists(tn, grid, nodes).max() == 24

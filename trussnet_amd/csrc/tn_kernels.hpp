@@ -853,10 +853,10 @@ __device__ __forceinline__ uint64_t chunk_hits(const QueryOps& qo, float4 v, flo
     const float cx = v.x - ox, cy = v.y - oy, cz = v.z - oz;
     const float C = cx * cx + cy * cy + cz * cz - k2 * v.w * v.w;
     // K-index 2 t + l / 32: (-2 cx, -2 cy), (-2 cz, -2 k^2 h), (1, |c|^2 - k^2 h^2); past the
-    // chunk's end a difference far above any margin
+    // chunk's end an infinite difference, above the margin in any unit of length
     float a0[2] = { some ? -2.0f * cx : 0.0f, some ? -2.0f * cy : 0.0f };
     float a1[2] = { some ? -2.0f * cz : 0.0f, some ? -2.0f * k2 * v.w : 0.0f };
-    float a2[2] = { some ? 1.0f : 0.0f, some ? C : 1e30f };
+    float a2[2] = { some ? 1.0f : 0.0f, some ? C : __builtin_huge_valf() };
     return tiles_below(qo, a0, a1, a2, margin);
 }
 
@@ -872,7 +872,7 @@ __device__ __forceinline__ uint64_t chunk_near(float qx, float qy, float qz, flo
     const QueryOps qo = query_ops(qx, qy, qz, qx * qx + qy * qy + qz * qz - near2, 1.0f, 0.0f);
     float a0[2] = { some ? -2.0f * cx : 0.0f, some ? -2.0f * cy : 0.0f };
     float a1[2] = { some ? -2.0f * cz : 0.0f, some ? 1.0f : 0.0f };
-    float a2[2] = { some ? cx * cx + cy * cy + cz * cz : 1e35f, 0.0f };
+    float a2[2] = { some ? cx * cx + cy * cy + cz * cz : __builtin_huge_valf(), 0.0f };
     return tiles_below(qo, a0, a1, a2, margin);
 }
 
@@ -1093,8 +1093,10 @@ __global__ __launch_bounds__(kTrussWave, kTrussOcc) void k_truss(Hash H, TrussIn
                         }
                     }
                     if (near) {
-                        const float dk = kth == ~0ull ? 1e15f : __uint_as_float((uint32_t)(kth >> 32));
-                        hit &= chunk_near(qx, qy, qz, dk * dk, mine_c, gox, goy, goz, margin);
+                        const bool full = kth != ~0ull;   // (a lane with fewer bars takes any)
+                        const float dk = full ? __uint_as_float((uint32_t)(kth >> 32)) : 0.0f;
+                        const uint64_t nearer = chunk_near(qx, qy, qz, dk * dk, mine_c, gox, goy, goz, margin);
+                        hit = full ? hit & nearer : hit;
                     }
                     if (!cut && __ballot(cnt + __popcll(hit) > kCollect)) {   // a buffer fills
                         cut = true;
