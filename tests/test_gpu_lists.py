@@ -179,3 +179,28 @@ def test_any_unit_of_length(tn, power, per):
     nodes = nodes_at(base, P[rng.permutation(len(P))])
     nodes.P *= u
     assert same_lists(tn, grid, nodes).max() == 24
+
+
+@pytest.mark.parametrize("counts", [(127, 128, 129), (255, 1, 256), (383, 384, 385), (640, 641), (2000, 3000, 700)])
+@pytest.mark.parametrize("ahead", [0, 1, 200])
+def test_cells_longer_than_a_block(tn, counts, ahead):
+    """Cells of so many nodes that renumbering reads them past a block's window, to one side or
+    both, in a row and from any place in a block (`ahead` nodes in cells before them)"""
+    grid = Fixture("jitter64").grid
+    b = float(np.float32(1.6) * np.float32(grid.hmin))
+    rng = np.random.default_rng(sum(counts) + ahead)
+    cell = [rng.uniform(0.02, 0.98, (c, 3)) * b + [(4 + k) * b - 0.5, 6 * b - 0.5, 6 * b - 0.5] for k, c in enumerate(counts)]
+    P = np.concatenate([rng.uniform(0.5, 2 * b, (ahead, 3)), *cell])
+    same_lists(tn, grid, nodes_at(grid, P[rng.permutation(len(P))]))
+
+
+def test_renumbering_a_long_cell_costs_less_than_its_search(tn):
+    """100 k nodes in a few cells: both grow with the square of a cell's nodes, the search with
+    by far the larger factor"""
+    grid = Fixture("jitter64").grid
+    P = 30.0 + 4.0 * np.random.default_rng(1).uniform(0, 1, (100000, 3))
+    with tn.Plan(grid, nodes_at(grid, P), RelaxParams(max_iters=0)) as plan:
+        plan.set_timing(True)
+        plan.run()
+        ms = {k: v[1] for k, v in plan.timings().items()}
+    assert ms["permute"] < 0.2 * ms["neighbors"], ms

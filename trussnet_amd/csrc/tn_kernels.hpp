@@ -429,8 +429,11 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const int32_t* __restr
 // among them (read from LDS) is its place: two launches where the radix sort this
 // replaces took three passes of five (2.5 M nodes: 126 us of sorting and 66 of renumbering
 // a rebuild before, 11 and 80 now; 3 k nodes: 37 and 6, now 6 and 7). The rank costs a
-// read for every node of the cell: where the voxel trap stacks nodes up (hundreds in a
-// cell) the two take 131 us at 495 k nodes against 97 before, of 2.9 ms a rebuild.
+// comparison for every node of the cell, so it grows with the square of a cell's nodes as
+// their search does. A cell longer than the window is read by the block together, tile by
+// tile, which keeps it a tenth of the search's time or less: 495 k nodes that the voxel
+// trap stacks up (hundreds in a cell) 103 -> 29 us, each node reading the cell's places by
+// itself -> tiles; 100 k nodes of a few cells 4.24 -> 0.66 ms, their search 7.0.
 // Ps and P0 (the positions as of this rebuild) and Ms (id, typ | lab << 8) are written in
 // the new order, and keyS the nodes' keys.
 struct NodeArrays {
@@ -449,29 +452,57 @@ __global__ __launch_bounds__(kBlock) void k_permute(const int32_t* __restrict__ 
                                                     NodeArrays out, float4* __restrict__ Ps,
                                                     float4* __restrict__ P0, int2* __restrict__ Ms,
                                                     int32_t* __restrict__ slot_of, int32_t* __restrict__ keyS) {
-    constexpr int kSide = kBlock / 2;
-    __shared__ int near[2 * kBlock];   // bycell around the block: most cells' slots
-    const int p = blockIdx.x * kBlock + threadIdx.x, n0 = blockIdx.x * kBlock - kSide, n1 = n0 + 2 * kBlock;
-    for (int j = threadIdx.x; j < 2 * kBlock; j += kBlock) {
+    constexpr int kSide = kBlock / 2, kTile = 2 * kBlock;
+    __shared__ __align__(16) int near[kTile];   // bycell around the block: most cells' slots; then tiles
+    __shared__ int reach[2];                    // where the first node's cell begins, where the last one's ends
+    const int tid = threadIdx.x, p0 = blockIdx.x * kBlock, p = p0 + tid, n0 = p0 - kSide, n1 = n0 + kTile;
+    for (int j = tid; j < kTile; j += kBlock) {
         near[j] = n0 + j >= 0 && n0 + j < n ? bycell[n0 + j] : 0;
     }
     __syncthreads();
+    int s = 0, k = 0, b = 0, e = 0, t = 0;
     if (p < n) {
-        const int s = near[kSide + threadIdx.x];
-        const int k = key[s];
-        const int b = cstart[k], e = cstart[k + 1];
+        s = near[kSide + tid];
+        k = key[s];
+        b = cstart[k];
+        e = cstart[k + 1];
         const int b1 = max(b, n0), e1 = min(e, n1);
-        int t = b;
+        t = b;
 #pragma unroll 4
         for (int q = b1; q < e1; ++q) {
             t += near[q - n0] < s ? 1 : 0;
         }
-        for (int q = b; q < b1; ++q) {   // a long cell's slots beyond the window
-            t += bycell[q] < s ? 1 : 0;
+    }
+    if (tid == 0) {
+        reach[0] = b;
+    }
+    if (p == min(n, p0 + kBlock) - 1) {
+        reach[1] = e;
+    }
+    __syncthreads();
+    // the slots of a long cell at places q0 .. q1 - 1, outside the window (all threads of the
+    // block; mine: of this node's cell, the one that reaches out of the window on that side)
+    auto beyond = [&](int q0, int q1, bool mine) {
+        for (int at = q0; at < q1; at += kTile) {
+            for (int j = tid; j < kTile; j += kBlock) {
+                near[j] = at + j < q1 ? bycell[at + j] : INT_MAX;
+            }
+            __syncthreads();
+            if (mine) {
+                const int4* tile = reinterpret_cast<const int4*>(near);
+                const int m = (min(kTile, q1 - at) + 3) / 4;
+#pragma unroll 4
+                for (int j = 0; j < m; ++j) {
+                    const int4 v = tile[j];
+                    t += (v.x < s ? 1 : 0) + (v.y < s ? 1 : 0) + (v.z < s ? 1 : 0) + (v.w < s ? 1 : 0);
+                }
+            }
+            __syncthreads();
         }
-        for (int q = e1; q < e; ++q) {
-            t += bycell[q] < s ? 1 : 0;
-        }
+    };
+    beyond(reach[0], n0, b < n0);
+    beyond(n1, reach[1], e > n1);
+    if (p < n) {
         keyS[t] = k;
         const float4 x = in.X[s];
         out.X[t] = x;
