@@ -38,6 +38,11 @@ struct TnError : std::runtime_error {
     TnError(int c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
 
+// device memory has run out (TN_ERR_HIP to the caller)
+struct NoMemory : TnError {
+    explicit NoMemory(const std::string& m) : TnError(TN_ERR_HIP, m) {}
+};
+
 #define TN_HIP(call)                                                                                   \
     do {                                                                                               \
         const hipError_t e_ = (call);                                                                  \
@@ -208,7 +213,9 @@ __global__ void k_iota(int32_t* __restrict__ a, int n) {
 // and a device-wide sync. At most TN_MEM_CACHE_MB (default 8192; 0: off) are kept: past
 // that the oldest go back to the driver, and all of a device's do when an allocation on
 // it fails. Large sizes are rounded up by at most an eighth (size_class), so that
-// volumes of about one size share buffers.
+// volumes of about one size share buffers. TN_MEM_LIMIT_MB (read at each allocation; unset
+// or 0: none) bounds what the library holds in all, in use and kept: past it an allocation
+// fails as on a device of that size.
 struct MemCache {
     struct Entry {
         int dev;
@@ -219,7 +226,8 @@ struct MemCache {
     std::mutex mu;
     List kept;
     std::multimap<std::pair<int, size_t>, List::iterator> by_size;
-    size_t bytes = 0, cap = 0;
+    size_t bytes = 0, cap = 0;   // kept, and at most
+    size_t held = 0;             // allocated, in use or kept
     MemCache() {
         const char* e = std::getenv("TN_MEM_CACHE_MB");
         cap = (e && e[0] ? (size_t)std::strtoull(e, nullptr, 10) : (size_t)8192) << 20;
@@ -231,8 +239,16 @@ struct MemCache {
         }
         return (b + step - 1) / step * step;   // (step: between a sixteenth and an eighth of b)
     }
+    static size_t limit() {
+        const char* v = std::getenv("TN_MEM_LIMIT_MB");
+        return v && v[0] ? (size_t)std::strtoull(v, nullptr, 10) << 20 : 0;
+    }
     void* take(int dev, size_t b) {
+        const size_t most = limit();
         std::lock_guard<std::mutex> g(mu);
+        while (most && held > most && !kept.empty()) {
+            drop(kept.begin());
+        }
         const auto it = by_size.find({ dev, b });
         if (it == by_size.end()) {
             return nullptr;
@@ -243,11 +259,41 @@ struct MemCache {
         bytes -= b;
         return p;
     }
+    // a new buffer, or null and the error
+    void* grab(size_t b, hipError_t* e) {
+        const size_t most = limit();
+        {
+            std::lock_guard<std::mutex> g(mu);
+            if (most && held + b > most) {
+                *e = hipErrorOutOfMemory;
+                return nullptr;
+            }
+            held += b;
+        }
+        void* p = nullptr;
+        *e = hipMalloc(&p, b);
+        if (*e != hipSuccess) {
+            (void)hipGetLastError();
+            std::lock_guard<std::mutex> g(mu);
+            held -= b;
+            return nullptr;
+        }
+        return p;
+    }
+    size_t kept_on(int dev) {
+        std::lock_guard<std::mutex> g(mu);
+        size_t b = 0;
+        for (const Entry& e : kept) {
+            b += e.dev == dev ? e.bytes : 0;
+        }
+        return b;
+    }
     // (the caller has synchronised the device: nothing in flight uses the buffer)
     void give(int dev, size_t b, void* p) {
         std::lock_guard<std::mutex> g(mu);
         if (b > cap) {
             (void)hipFree(p);
+            held -= b;
             return;
         }
         while (bytes + b > cap) {
@@ -278,6 +324,7 @@ private:
             }
         }
         bytes -= e->bytes;
+        held -= e->bytes;
         (void)hipFree(e->p);
         kept.erase(e);
     }
@@ -323,27 +370,40 @@ struct DevMem {
         }
     }
     // a buffer of `bytes` at least on the current device: a cached one, else a new one
-    void* fresh(size_t bytes) {
+    // (optional: its caller can do without)
+    void* fresh(size_t bytes, bool optional) {
         int dev = 0;
         TN_HIP(hipGetDevice(&dev));
+        hipError_t e = hipSuccess;
         size_t b = MemCache::size_class(bytes);
         void* p = mem_cache().take(dev, b);
-        if (!p && hipMalloc(&p, b) != hipSuccess) {
+        if (!p) {
+            p = mem_cache().grab(b, &e);
+        }
+        if (!p && !(optional && mem_cache().kept_on(dev) < bytes)) {
             // no room: the kept buffers back to the driver, and no more than was asked for
-            (void)hipGetLastError();
             mem_cache().drop_device(dev);
             b = bytes;
-            TN_HIP(hipMalloc(&p, b));
+            p = mem_cache().grab(b, &e);
+        }
+        if (!p) {
+            throw NoMemory("hipMalloc of " + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
         }
         owned.push_back({ p, b, dev });
         return p;
+    }
+    // the other's buffers, to be freed with this one's
+    void adopt(DevMem& o) {
+        owned.insert(owned.end(), o.owned.begin(), o.owned.end());
+        o.owned.clear();
+        o.chunk_left = 0;
     }
     void set_arena(void* base, size_t cap) {
         arena = static_cast<char*>(base);
         arena_cap = cap;
         arena_used = 0;
     }
-    void* raw(size_t bytes) {
+    void* raw(size_t bytes, bool optional = false) {
         bytes = (std::max<size_t>(bytes, 1) + kAlign - 1) / kAlign * kAlign;
         if (arena) {
             if (bytes > arena_cap - arena_used) {
@@ -357,10 +417,10 @@ struct DevMem {
             return p;
         }
         if (bytes > kChunk / 4) {   // a buffer of its own
-            return fresh(bytes);
+            return fresh(bytes, optional);
         }
         if (bytes > chunk_left) {
-            chunk = static_cast<char*>(fresh(kChunk));
+            chunk = static_cast<char*>(fresh(kChunk, optional));
             chunk_left = kChunk;
         }
         void* p = chunk;
@@ -371,9 +431,8 @@ struct DevMem {
     // raw() for a buffer that its caller can do without: null where there is no room
     void* spare(size_t bytes) {
         try {
-            return raw(bytes);
+            return raw(bytes, true);
         } catch (const TnError&) {
-            (void)hipGetLastError();
             return nullptr;
         }
     }
@@ -447,12 +506,14 @@ void add_apron(tnd::Field& f, int64_t nslot, DevMem& mem, hipStream_t s, bool ow
         return;
     }
     const int64_t nb = (int64_t)f.nbx * f.nby * f.nbz;
-    const size_t slots = (size_t)std::max<int64_t>(nslot, 1) * tnd::kApSlot * sizeof(float);
-    float* ap = static_cast<float*>(mem.spare(slots));
-    uint4* rec = ap ? static_cast<uint4*>(mem.spare((size_t)nb * 4 * sizeof(uint4))) : nullptr;
-    if (!rec) {
+    // (one buffer, whole lines of it for either)
+    const size_t values = (size_t)std::max<int64_t>(nslot, 1) * tnd::kApSlot;
+    static_assert(tnd::kApSlot * sizeof(float) % 64 == 0, "the records begin with a line");
+    float* ap = static_cast<float*>(mem.spare(values * sizeof(float) + (size_t)nb * 4 * sizeof(uint4)));
+    if (!ap) {
         return;
     }
+    uint4* rec = reinterpret_cast<uint4*>(ap + values);
     tnd::k_brick_rec<<<blocks_for(nb, 256), 256, 0, s>>>(f.bl_cnt, f.bl_lab, f.bl_slot, (int)nb, rec);
     tnd::k_apron<<<(unsigned)nb, 256, 0, s>>>(f, ap);
     TN_HIP(hipGetLastError());
@@ -1807,18 +1868,19 @@ Seeds run_seeding(const tn_grid_view* g, const uint8_t* grade, const tn_relax_pa
     return g->nfeat > 0 ? add_feature_nodes(g, f, s, mem) : s;
 }
 
-// seed_cpu on a grid already on the device (f, its grades d_grade), scratch in mem
-Seeds seeding_core(const tnd::Field& stored, int64_t nslot, const uint8_t* d_grade, float hmin, float hmax,
-                   const tn_relax_params* prm, DevMem& mem) {
+// seed_cpu on a grid already on the device (stored, its grades d_grade), the nodes and the
+// scratch in mem, the slots (none without) in a memory of their own
+Seeds seeding_pass(const tnd::Field& stored, int64_t nslot, const uint8_t* d_grade, float hmin, float hmax,
+                   const tn_relax_params* prm, DevMem& mem, DevMem* slots) {
     arg_check(prm != nullptr, "seeding: null argument");
     arg_check(prm->nseed >= 1 && prm->nseed <= 64, "seeding: nseed out of range");
     arg_check(prm->jseed >= 0.0f && std::isfinite(prm->jseed), "seeding: jseed must be finite and >= 0");
     SeedOps ops{ mem };
     // (the copy of the Field in device memory, which other calls share, keeps no slots: they
-    // go with this call's memory, and only kernels without out-of-line calls read them)
+    // go with this call, and only kernels without out-of-line calls read them)
     tnd::Field f = stored;
-    if (!prm->voxel_trap) {
-        add_apron(f, nslot, mem, nullptr, false);
+    if (slots && !prm->voxel_trap) {
+        add_apron(f, nslot, *slots, nullptr, false);
     }
     // run k(F): over the apron slots where there are any
     auto over_field = [&](auto&& k) {
@@ -1893,6 +1955,23 @@ Seeds seeding_core(const tnd::Field& stored, int64_t nslot, const uint8_t* d_gra
     }
     TN_HIP(hipDeviceSynchronize());
     return s;
+}
+
+// The seeding with the slots, which come before the arrays whose sizes only the seeding
+// tells; once more without them where these then find no room.
+Seeds seeding_core(const tnd::Field& stored, int64_t nslot, const uint8_t* d_grade, float hmin, float hmax,
+                   const tn_relax_params* prm, DevMem& mem) {
+    {
+        DevMem work, slots;
+        work.device = slots.device = mem.device;
+        try {
+            const Seeds s = seeding_pass(stored, nslot, d_grade, hmin, hmax, prm, work, &slots);
+            mem.adopt(work);
+            return s;
+        } catch (const NoMemory&) {
+        }
+    }
+    return seeding_pass(stored, nslot, d_grade, hmin, hmax, prm, mem, nullptr);
 }
 
 // Every plan's iterations as grouped launches on one stream: each of an iteration's
