@@ -65,3 +65,18 @@ def test_seeding(tn, monkeypatch, volume):
 def test_plan(tn, monkeypatch, volume):
     seeds, prm = tn.seed(volume, RelaxParams(), device=0), RelaxParams(max_iters=3, dptol=0.0)
     smallest_limit(tn, monkeypatch, lambda: tn.relax(volume, seeds, prm, device=0)[0], lambda a, b: a.equal(b), 300)
+
+
+def test_batch(tn, monkeypatch, volume):
+    """Three volumes take no more than three times what one takes alone, and the batch's tables"""
+    seeds, prm = tn.seed(volume, RelaxParams(), device=0), RelaxParams(max_iters=3, dptol=0.0)
+
+    def batch(count):
+        return [x for x, _ in tn.relax_batch([volume] * count, [seeds] * count, [prm] * count, device=0)]
+
+    def same(a, b):
+        return all(x.equal(y) for x, y in zip(a, b))
+
+    one = smallest_limit(tn, monkeypatch, lambda: batch(1), same, 40)
+    three = smallest_limit(tn, monkeypatch, lambda: batch(3), same, 600)
+    assert three <= 3 * one + STEP

@@ -763,6 +763,7 @@ struct tn_plan {
     int rebuilds = 0;
     bool finished = false;
     bool at_seeds = false;   // as reset() leaves it: the seeds in place, the first rebuild done
+    int64_t nslot = 0;       // the grid's phi slots
 
     template <class T>
     T* alloc(size_t count) {
@@ -777,6 +778,14 @@ struct tn_plan {
             (void)hipStreamSynchronize(stream);
         } else {
             kit_pool().give(device, kit);
+        }
+    }
+
+    // the corner slots, where the moves read them: optional, so after every buffer that the
+    // plan, and a batch of plans, cannot do without
+    void lay_slots() {
+        if (n > 0 && !prm.voxel_trap) {
+            add_apron(f, nslot, mem, stream, true);
         }
     }
 
@@ -1117,10 +1126,12 @@ namespace {
 // A plan on device dev: make_grid(mem) puts the grid into the plan's memory and
 // returns its Field; H and nkeys are the hash geometry, nslot the grid's phi slots.
 // find_largest: the hash's largest h is still to be taken, from the grid on the device. With an arena, the plan
-// allocates nothing (DevMem::set_arena; tn_plan::noalloc).
+// allocates nothing (DevMem::set_arena; tn_plan::noalloc). slots: lay_slots() is called here,
+// not left to the caller.
 template <class MakeGrid>
 tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int dev, const tnd::Hash& H, int64_t nkeys,
-                    int64_t nslot, bool find_largest, MakeGrid make_grid, void* arena = nullptr, size_t arena_cap = 0) {
+                    int64_t nslot, bool find_largest, MakeGrid make_grid, bool slots = true, void* arena = nullptr,
+                    size_t arena_cap = 0) {
         TN_HIP(hipSetDevice(dev));
         std::unique_ptr<tn_plan> p(new tn_plan);
         p->device = dev;
@@ -1131,6 +1142,7 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
         p->tskin = prm->t + prm->skin;
         p->H = H;
         p->nkeys = nkeys;
+        p->nslot = nslot;
         p->noalloc = arena != nullptr;
         if (p->noalloc) {   // the null stream, the passes one after another, no timing
             p->overlap_moves = false;
@@ -1244,9 +1256,8 @@ tn_plan* plan_build(const tn_relax_params* prm, const tn_nodes_view* seeds, int 
             set_largest(p->H, prm, device_minmax<true>(f.h, (int64_t)f.nx * f.ny * f.nz,
                                                        reinterpret_cast<int32_t*>(p->dCtl), p->stream).second);
         }
-        // (after every buffer that the plan cannot do without)
-        if (n > 0 && !prm->voxel_trap) {
-            add_apron(f, nslot, p->mem, p->stream, true);
+        if (slots) {
+            p->lay_slots();
         }
         p->reset();
         return p.release();
@@ -1372,6 +1383,20 @@ void check_nodes(const tn_nodes_view* nd) {
     if (nd->n > 0) {
         arg_check(nd->P && nd->lab && nd->typ && nd->part, "nodes: null array");
     }
+}
+
+// a plan over a host grid (tn_plan_create)
+void plan_over(const tn_grid_view* g, const tn_relax_params* prm, const tn_nodes_view* seeds, int32_t device, bool slots,
+               tn_plan** out) {
+    arg_check(out != nullptr, "null plan pointer");
+    *out = nullptr;
+    check_grid(g);
+    check_params(prm);
+    check_nodes(seeds);
+    const int dev = pick_device(device);
+    int64_t nkeys = 0;
+    const tnd::Hash H = make_hash(g, prm, &nkeys);
+    *out = plan_build(prm, seeds, dev, H, nkeys, g->nslot, true, [&](DevMem& mem) { return upload_grid(g, mem); }, slots);
 }
 
 // The seeding of seed_cpu_body (src/v2m_particles.cpp:637-726) on one device: the
@@ -1983,10 +2008,6 @@ template <class Plans>
 void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
     const int count = (int)plans.size();
     hipStream_t bs = plans[0]->stream;
-    bool all_plain = true;   // every smooth move over a label volume's apron slots
-    for (int k = 0; k < count; ++k) {
-        all_plain = all_plain && (plans[k]->f.ap || (plans[k]->prm.voxel_trap && plans[k]->f.gm == 0));
-    }
     std::vector<hipStream_t> own(count);
     for (int k = 0; k < count; ++k) {
         own[k] = plans[k]->stream;
@@ -2026,7 +2047,6 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
     for (int k = 0; k < count; ++k) {
         htab[k] = plans[k]->iter_args();
     }
-    TN_HIP(hipMemcpyAsync(dtab, htab, sizeof(tnk::PlanIter) * count, hipMemcpyHostToDevice, bs));
     // block maps: for each grid shape, the plan of every block and each plan's first block
     int64_t map_total = 0;
     for (int k = 0; k < count; ++k) {
@@ -2038,6 +2058,13 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
     TN_HIP(hipHostMalloc(&pmap.p, sizeof(int32_t) * map_total, hipHostMallocDefault));
     int32_t* hmap = static_cast<int32_t*>(pmap.p);
     int32_t* dmap = gm.alloc<int32_t>((size_t)map_total);
+    bool all_plain = true;   // every smooth move over a label volume's apron slots
+    for (int k = 0; k < count; ++k) {
+        plans[k]->lay_slots();
+        htab[k].f = plans[k]->f;
+        all_plain = all_plain && (plans[k]->f.ap || (plans[k]->prm.voxel_trap && plans[k]->f.gm == 0));
+    }
+    TN_HIP(hipMemcpyAsync(dtab, htab, sizeof(tnk::PlanIter) * count, hipMemcpyHostToDevice, bs));
     const int32_t* bplan[tnk::kShapes];
     const int32_t* bfirst[tnk::kShapes];
     unsigned nblocks[tnk::kShapes];
@@ -2655,17 +2682,7 @@ int tn_device_count(int32_t* count) {
 
 int tn_plan_create(const tn_grid_view* g, const tn_relax_params* prm, const tn_nodes_view* seeds, int32_t device,
                    tn_plan** out) {
-    return guarded([&] {
-        arg_check(out != nullptr, "null plan pointer");
-        *out = nullptr;
-        check_grid(g);
-        check_params(prm);
-        check_nodes(seeds);
-        const int dev = pick_device(device);
-        int64_t nkeys = 0;
-        const tnd::Hash H = make_hash(g, prm, &nkeys);
-        *out = plan_build(prm, seeds, dev, H, nkeys, g->nslot, true, [&](DevMem& mem) { return upload_grid(g, mem); });
-    });
+    return guarded([&] { plan_over(g, prm, seeds, device, true, out); });
 }
 
 int tn_plan_set_timing(tn_plan* p, int32_t on) {
@@ -2991,7 +3008,7 @@ int tn_relax_noalloc(const tn_grid_view* g, const tn_relax_params* prm, tn_nodes
         int64_t nkeys = 0;
         const tnd::Hash H = make_hash(g, prm, &nkeys);
         std::unique_ptr<tn_plan> p(plan_build(prm, nd, dev, H, nkeys, g->nslot, true, [&](DevMem& mem) { return upload_grid(g, mem); },
-                                              base, TN_NOALLOC_SCRATCH_BYTES));
+                                              true, base, TN_NOALLOC_SCRATCH_BYTES));
         if (p->n > 0) {   // plan_build left it reset: seeds in place, first rebuild done
             p->run_iters(p->prm.max_iters);
         }
@@ -3015,9 +3032,9 @@ int tn_relax_batch(const tn_grid_view* grids, const tn_relax_params* prms, tn_no
         };
         std::vector<std::unique_ptr<tn_plan, Destroy>> plans;
         plans.reserve(count);
-        for (int k = 0; k < count; ++k) {   // each plan: grid and seeds uploaded, first rebuild done
+        for (int k = 0; k < count; ++k) {   // each plan: grid and seeds uploaded, first rebuild done; no slots yet
             tn_plan* p = nullptr;
-            const int rc = tn_plan_create(&grids[k], &prms[k], &nodes[k], device, &p);
+            const int rc = guarded([&] { plan_over(&grids[k], &prms[k], &nodes[k], device, false, &p); });
             if (rc != TN_OK) {
                 throw TnError(rc, "volume " + std::to_string(k) + ": " + g_err);
             }
