@@ -2058,11 +2058,15 @@ void run_grouped(Plans& plans, int64_t& launches, int64_t& steps) {
     TN_HIP(hipHostMalloc(&pmap.p, sizeof(int32_t) * map_total, hipHostMallocDefault));
     int32_t* hmap = static_cast<int32_t*>(pmap.p);
     int32_t* dmap = gm.alloc<int32_t>((size_t)map_total);
-    bool all_plain = true;   // every smooth move over a label volume's apron slots
+    // every smooth move over a label volume's corner slots (a plan with no nodes has no moves)
+    bool all_plain = true;
     for (int k = 0; k < count; ++k) {
         plans[k]->lay_slots();
         htab[k].f = plans[k]->f;
-        all_plain = all_plain && (plans[k]->f.ap || (plans[k]->prm.voxel_trap && plans[k]->f.gm == 0));
+        all_plain = all_plain && (plans[k]->n == 0 || plans[k]->f.ap || (plans[k]->prm.voxel_trap && plans[k]->f.gm == 0));
+    }
+    if (std::getenv("TN_BATCH_VERBOSE")) {
+        std::fprintf(stderr, "[tn_relax_batch] moves over the %s\n", all_plain ? "corner slots" : "stored layout");
     }
     TN_HIP(hipMemcpyAsync(dtab, htab, sizeof(tnk::PlanIter) * count, hipMemcpyHostToDevice, bs));
     const int32_t* bplan[tnk::kShapes];
