@@ -3,6 +3,8 @@ the oracle, which reads the stored layout voxel by voxel: every query the same b
 points in brick interiors, on brick faces and edges, at the grid's sides and outside it,
 for labels the cell's brick lists and labels it does not.
 """
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -58,6 +60,34 @@ def test_queries_equal_the_oracle(tn, oracle_lib, shape, vs, blocks, nlab):
             want = oracle_lib.field_points(grid, a, b, X)
             for g, w, name in zip(got, want, ("phi", "psi", "grad", "label", "second")):
                 assert np.array_equal(bits(g), bits(w)), (shape, a, b, name)
+
+
+@pytest.mark.parametrize("name", ["sectors48", "ellipsoids56"])
+def test_bricks_that_share_slots(tn, oracle_lib, name):
+    """A grid whose bricks of the same labels refer to one brick's slots: the values beyond a
+    slot's upper faces are each brick's own, so such a grid is read as stored. The same nodes
+    as of the grid that holds the shared values once for every brick."""
+    case = Fixture(name)
+    grid = case.grid
+    slot, phi, first = grid.bl_slot.copy(), grid.phi.reshape(-1, 512).copy(), {}
+    lab = grid.bl_lab.reshape(-1, 16)
+    for b in np.flatnonzero(slot >= 0):
+        n = int(grid.bl_cnt[b])
+        a = first.setdefault(tuple(lab[b, :n].tolist()), b)
+        phi[grid.bl_slot[b]:grid.bl_slot[b] + n] = phi[grid.bl_slot[a]:grid.bl_slot[a] + n]
+        slot[b] = grid.bl_slot[a]
+    assert (slot != grid.bl_slot).sum() > 10
+    shared, own = dataclasses.replace(grid, bl_slot=slot), dataclasses.replace(grid, phi=phi.ravel())
+    X = _points((grid.nz, grid.ny, grid.nx), grid.vs, 3)
+    with tn.Plan(shared, case.seeds, RelaxParams()) as plan:
+        for a, b in ((0, 1), (1, 2)):
+            for g, w in zip(plan.field_points(a, b, X), oracle_lib.field_points(shared, a, b, X)):
+                assert np.array_equal(bits(g), bits(w))
+    prm = RelaxParams(max_iters=30, dptol=0.0)
+    want = oracle_lib.relax(shared, case.seeds, prm)[0]
+    for g in (shared, own):
+        assert tn.relax(g, case.seeds, prm, device=0)[0].equal(want)
+    assert tn.seed(shared, prm, device=0).equal(tn.seed(own, prm, device=0))
 
 
 def test_stored_layout_where_the_slots_do_not_fit(tn):

@@ -495,14 +495,35 @@ tnd::Field upload_grid(const tn_grid_view* g, DevMem& mem) {
     return f;
 }
 
+// The phi slots of a checked host grid if each is one brick's own, else -1: a slot that two
+// bricks refer to has two sets of values beyond its upper faces.
+int64_t own_slots(const tn_grid_view* g) {
+    if (g->gm != 0) {
+        return g->nslot;
+    }
+    std::vector<bool> taken((size_t)g->nslot);
+    const int64_t nb = (int64_t)g->nbx * g->nby * g->nbz;
+    for (int64_t b = 0; b < nb; ++b) {
+        const int64_t s0 = g->bl_slot[b], s1 = s0 < 0 ? s0 : s0 + std::min<int64_t>(g->bl_cnt[b], TN_BL);
+        for (int64_t s = s0; s < s1; ++s) {
+            if (taken[(size_t)s]) {
+                return -1;
+            }
+            taken[(size_t)s] = true;
+        }
+    }
+    return g->nslot;
+}
+
 // The apron slots and brick records of a label volume's grid (tn_apron.hpp), put into mem
-// and f (f.self's copy too, on the stream s). Nothing for the other field modes, nor where
-// mem has no room for them: the kernels over the stored layout then run.
+// and f (f.self's copy too, on the stream s). Nothing for the other field modes, for bricks
+// that share slots (nslot < 0), nor where mem has no room for them: the kernels over the
+// stored layout then run.
 // own_self: f.self is this Field's alone.
 void add_apron(tnd::Field& f, int64_t nslot, DevMem& mem, hipStream_t s, bool own_self) {
     f.ap = nullptr;
     f.rec = nullptr;
-    if (f.gm != 0) {
+    if (f.gm != 0 || nslot < 0) {
         return;
     }
     const int64_t nb = (int64_t)f.nbx * f.nby * f.nbz;
@@ -763,7 +784,7 @@ struct tn_plan {
     int rebuilds = 0;
     bool finished = false;
     bool at_seeds = false;   // as reset() leaves it: the seeds in place, the first rebuild done
-    int64_t nslot = 0;       // the grid's phi slots
+    int64_t nslot = 0;       // the grid's phi slots (-1: bricks share some)
 
     template <class T>
     T* alloc(size_t count) {
@@ -1124,7 +1145,7 @@ struct tn_plan {
 namespace {
 
 // A plan on device dev: make_grid(mem) puts the grid into the plan's memory and
-// returns its Field; H and nkeys are the hash geometry, nslot the grid's phi slots.
+// returns its Field; H and nkeys are the hash geometry, nslot the grid's phi slots (own_slots).
 // find_largest: the hash's largest h is still to be taken, from the grid on the device. With an arena, the plan
 // allocates nothing (DevMem::set_arena; tn_plan::noalloc). slots: lay_slots() is called here,
 // not left to the caller.
@@ -1396,7 +1417,7 @@ void plan_over(const tn_grid_view* g, const tn_relax_params* prm, const tn_nodes
     const int dev = pick_device(device);
     int64_t nkeys = 0;
     const tnd::Hash H = make_hash(g, prm, &nkeys);
-    *out = plan_build(prm, seeds, dev, H, nkeys, g->nslot, true, [&](DevMem& mem) { return upload_grid(g, mem); }, slots);
+    *out = plan_build(prm, seeds, dev, H, nkeys, own_slots(g), true, [&](DevMem& mem) { return upload_grid(g, mem); }, slots);
 }
 
 // The seeding of seed_cpu_body (src/v2m_particles.cpp:637-726) on one device: the
@@ -1888,7 +1909,7 @@ Seeds run_seeding(const tn_grid_view* g, const uint8_t* grade, const tn_relax_pa
     mem.device = dev;
     const tnd::Field f = upload_grid(g, mem);
     const uint8_t* d_grade = mem.upload(grade, (size_t)g->nx * g->ny * g->nz);
-    const Seeds s = seeding_core(f, g->nslot, d_grade, g->hmin, g->hmax, prm, mem);
+    const Seeds s = seeding_core(f, own_slots(g), d_grade, g->hmin, g->hmax, prm, mem);
     // seed_cpu (src/v2m_particles.cpp:625-635): the shape input's feature nodes last
     return g->nfeat > 0 ? add_feature_nodes(g, f, s, mem) : s;
 }
@@ -3011,7 +3032,7 @@ int tn_relax_noalloc(const tn_grid_view* g, const tn_relax_params* prm, tn_nodes
         TN_HIP(hipGetLastError());
         int64_t nkeys = 0;
         const tnd::Hash H = make_hash(g, prm, &nkeys);
-        std::unique_ptr<tn_plan> p(plan_build(prm, nd, dev, H, nkeys, g->nslot, true, [&](DevMem& mem) { return upload_grid(g, mem); },
+        std::unique_ptr<tn_plan> p(plan_build(prm, nd, dev, H, nkeys, own_slots(g), true, [&](DevMem& mem) { return upload_grid(g, mem); },
                                               true, base, TN_NOALLOC_SCRATCH_BYTES));
         if (p->n > 0) {   // plan_build left it reset: seeds in place, first rebuild done
             p->run_iters(p->prm.max_iters);
