@@ -62,6 +62,25 @@ def test_queries_equal_the_oracle(tn, oracle_lib, shape, vs, blocks, nlab):
                 assert np.array_equal(bits(g), bits(w)), (shape, a, b, name)
 
 
+@pytest.mark.parametrize("name,voxel", [("sectors48", False), ("sectors48", True), ("aniso40", False), ("aniso40", True),
+                                        ("gray40", False), ("tpm32", False)])
+def test_points_far_out(tn, oracle_lib, name, voxel):
+    """Points whose voxel coordinates leave the range of an integer along any of the axes, as a
+    corner's Newton steps can: outside the grid, in the slots and in the stored layout (which a
+    voxel-trap plan reads)"""
+    case = Fixture(name)
+    grid = case.grid
+    rng = np.random.default_rng(2)
+    near = rng.uniform(0, 1, (4000, 3)) * np.array([grid.nx, grid.ny, grid.nz]) * np.array(grid.vs)
+    far = rng.choice([2.0 ** 31, 2.0 ** 31 - 128, 2.0 ** 32, 1e10, 1e20, -2.0 ** 31, -1e10, -1e20], (4000, 3)) * rng.choice([1.0, 1.5], (4000, 3))
+    X = np.where(rng.random((4000, 3)) < 0.6, far, near).astype(np.float32)
+    with tn.Plan(grid, case.seeds, RelaxParams(voxel_trap=voxel)) as plan:
+        for a, b in ((0, 1), (1, 0), (1, 2)):
+            for g, w, what in zip(plan.field_points(a, b, X), oracle_lib.field_points(grid, a, b, X),
+                                  ("phi", "psi", "grad", "label", "second")):
+                assert np.array_equal(g, w), (a, b, what)
+
+
 @pytest.mark.parametrize("name", ["sectors48", "ellipsoids56"])
 def test_bricks_that_share_slots(tn, oracle_lib, name):
     """A grid whose bricks of the same labels refer to one brick's slots: the values beyond a

@@ -90,10 +90,6 @@ __device__ __forceinline__ BrickList brick_list(const PlainField& f, int b) {
     return r;
 }
 
-__device__ __forceinline__ bool in_grid(const PlainField& f, int i, int j, int k) {
-    return (uint32_t)i < (uint32_t)f.nx && (uint32_t)j < (uint32_t)f.ny && (uint32_t)k < (uint32_t)f.nz;
-}
-
 // the first of the cell's corners in slot s
 __device__ __forceinline__ const float* apron_cell(const PlainField& f, int s, int i0, int j0, int k0) {
     return f.ap + (size_t)s * kApSlot + (size_t)((i0 & 7) + kApRow * (j0 & 7) + kApPlane * (k0 & 7));
@@ -125,7 +121,7 @@ __device__ __forceinline__ void corners_by_voxel(const Field& f, int l, int m, i
     }
 #pragma clang loop unroll(disable)
     for (int q = 0; q < 8; ++q) {
-        const int i = i0 + (q & 1), j = j0 + ((q >> 1) & 1), k = k0 + (q >> 2);
+        const int i = step_by(i0, q & 1), j = step_by(j0, (q >> 1) & 1), k = step_by(k0, q >> 2);
         float v = phi_voxel(f, l, i, j, k);
         if (m >= 0) {
             v = v - phi_voxel(f, m, i, j, k);
@@ -145,7 +141,7 @@ __device__ __forceinline__ void psi_cell_load(const PlainField& f, int a, int b,
     pc.j0 = j0;
     pc.k0 = k0;
     bool slots = false;
-    if (in_grid(f, i0, j0, k0)) {
+    if (in_range(f, i0, j0, k0)) {
         const int bk = brick_at(f, i0, j0, k0);
         if (bk != pc.bk) {
             pc.bk = bk;
@@ -193,7 +189,7 @@ __device__ __forceinline__ BrickLabels brick_labels_at(const PlainField& f, P3 p
     const int i = (int)floorf(over_vx(f, p.x) + 0.5f), j = (int)floorf(over_vy(f, p.y) + 0.5f),
               k = (int)floorf(over_vz(f, p.z) + 0.5f);
     BrickLabels r;
-    if (!in_grid(f, i, j, k)) {
+    if (!in_range(f, i, j, k)) {
         r.b = -1;
         r.n = 1;
         r.list.lo = r.list.hi = make_uint4(0u, 0u, 0u, 0u);
@@ -226,7 +222,7 @@ __device__ __forceinline__ ApronCell apron_point(const PlainField& f, P3 p, cons
     c.fx = u - (float)c.i0;
     c.fy = v - (float)c.j0;
     c.fz = w - (float)c.k0;
-    c.in = in_grid(f, c.i0, c.j0, c.k0);
+    c.in = in_range(f, c.i0, c.j0, c.k0);
     const int bk = c.in ? brick_at(f, c.i0, c.j0, c.k0) : -1;
     c.same = c.in && bk == bl.b;
     c.list = bl.list;

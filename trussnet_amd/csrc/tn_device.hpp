@@ -107,6 +107,20 @@ __device__ __forceinline__ size_t vox(const Field& f, int i, int j, int k) {
     return (size_t)i + (size_t)f.nx * ((size_t)j + (size_t)f.ny * (size_t)k);
 }
 
+// A point's cell along an axis is (int)floorf(u), which saturates: of a point that ran
+// far out (a corner's Newton steps from nearly dependent gradients reach 1e9 voxels and
+// more) it is INT_MAX, and the cell's upper corner one more. Such sums wrap, so they are
+// formed without sign, and compared so (in_range) or against the bound less one: the
+// compiler takes a signed i + 1 < 0 for i < -1, and the wrapped corner for one inside.
+__device__ __forceinline__ int step_by(int i, int d) {
+    return (int)((uint32_t)i + (uint32_t)d);
+}
+
+// voxel (i, j, k) lies in the grid
+__device__ __forceinline__ bool in_range(const Field& f, int i, int j, int k) {
+    return (uint32_t)i < (uint32_t)f.nx && (uint32_t)j < (uint32_t)f.ny && (uint32_t)k < (uint32_t)f.nz;
+}
+
 // v2m_brick_of, src/opencl/v2m_grid_body.cl:116-118
 __device__ __forceinline__ int brick_at(const Field& f, int i, int j, int k) {
     return (i >> 3) + f.nbx * ((j >> 3) + f.nby * (k >> 3));
@@ -156,7 +170,7 @@ __device__ __forceinline__ int slot_in(const Field& f, int b, int l, int* has) {
 
 // v2m_phi_vox, src/opencl/v2m_grid_body.cl:137-153
 __device__ __forceinline__ float phi_voxel(const Field& f, int l, int i, int j, int k) {
-    if (i < 0 || j < 0 || k < 0 || i >= f.nx || j >= f.ny || k >= f.nz) {
+    if (!in_range(f, i, j, k)) {
         return l == 0 ? 1.0f : 0.0f;
     }
     int has;
@@ -170,8 +184,8 @@ __device__ __forceinline__ float phi_voxel(const Field& f, int l, int i, int j, 
 // v2m_phi_cell's single-brick case (src/opencl/v2m_grid_body.cl:161-180): the cell
 // (i0,j0,k0) lies in one brick inside the grid
 __device__ __forceinline__ bool cell_in_one_brick(const Field& f, int i0, int j0, int k0) {
-    return i0 >= 0 && j0 >= 0 && k0 >= 0 && i0 + 1 < f.nx && j0 + 1 < f.ny && k0 + 1 < f.nz &&
-           (i0 >> 3) == ((i0 + 1) >> 3) && (j0 >> 3) == ((j0 + 1) >> 3) && (k0 >> 3) == ((k0 + 1) >> 3);
+    return i0 >= 0 && j0 >= 0 && k0 >= 0 && i0 < f.nx - 1 && j0 < f.ny - 1 && k0 < f.nz - 1 && (i0 & 7) != 7 &&
+           (j0 & 7) != 7 && (k0 & 7) != 7;
 }
 
 // the 8 corners of phi_l in a single-brick cell, given l's slot s in that brick
@@ -212,8 +226,8 @@ __device__ __forceinline__ void corners_split(const Field& f, int la, int lb, in
     int b0 = -1, b1 = -1, sa0 = -1, sb0 = -1, ha0 = 0, hb0 = 0, sa1 = -1, sb1 = -1, ha1 = 0, hb1 = 0;
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
-        const int i = i0 + (m & 1), j = j0 + ((m >> 1) & 1), k = k0 + (m >> 2);
-        if (i < 0 || j < 0 || k < 0 || i >= f.nx || j >= f.ny || k >= f.nz) {   // outside the grid: label 0
+        const int i = step_by(i0, m & 1), j = step_by(j0, (m >> 1) & 1), k = step_by(k0, m >> 2);
+        if (!in_range(f, i, j, k)) {   // outside the grid: label 0
             ca[m] = la == 0 ? 1.0f : 0.0f;
             if (kPair) {
                 cb[m] = lb == 0 ? 1.0f : 0.0f;
@@ -686,7 +700,7 @@ __device__ __forceinline__ float4 gray_at(const Field& f, P3 p) {
     const float fx = u - (float)i0, fy = v - (float)j0, fz = w - (float)k0;
     const float out = f.gTW[0] - f.gTW[f.gm];
     float c[8];
-    if (i0 >= 0 && j0 >= 0 && k0 >= 0 && i0 + 1 < f.nx && j0 + 1 < f.ny && k0 + 1 < f.nz) {
+    if (i0 >= 0 && j0 >= 0 && k0 >= 0 && i0 < f.nx - 1 && j0 < f.ny - 1 && k0 < f.nz - 1) {
         const float* b0 = f.gI + vox(f, i0, j0, k0);
         const size_t sy = (size_t)f.nx, sz = (size_t)f.nx * (size_t)f.ny;
         c[0] = b0[0];
@@ -700,8 +714,8 @@ __device__ __forceinline__ float4 gray_at(const Field& f, P3 p) {
     } else {
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
-            const int i = i0 + (m & 1), j = j0 + ((m >> 1) & 1), k = k0 + (m >> 2);
-            c[m] = (i < 0 || j < 0 || k < 0 || i >= f.nx || j >= f.ny || k >= f.nz) ? out : f.gI[vox(f, i, j, k)];
+            const int i = step_by(i0, m & 1), j = step_by(j0, (m >> 1) & 1), k = step_by(k0, m >> 2);
+            c[m] = in_range(f, i, j, k) ? f.gI[vox(f, i, j, k)] : out;
         }
     }
     return trilerp_grad(f, c, fx, fy, fz);
@@ -790,7 +804,7 @@ __device__ __forceinline__ BrickLabels brick_labels_at(const Field& f, P3 p) {
     const int i = (int)floorf(over_vx(f, p.x) + 0.5f), j = (int)floorf(over_vy(f, p.y) + 0.5f),
               k = (int)floorf(over_vz(f, p.z) + 0.5f);
     BrickLabels r;
-    if (i < 0 || j < 0 || k < 0 || i >= f.nx || j >= f.ny || k >= f.nz) {
+    if (!in_range(f, i, j, k)) {
         r.b = -1;
         r.n = 1;
         r.list.lo = r.list.hi = make_uint4(0u, 0u, 0u, 0u);
@@ -1626,10 +1640,13 @@ __device__ __forceinline__ float trapped_step(const F& f, float h, P3 s, float m
 
 // v2m_label_at, src/opencl/v2m_grid_body.cl:72-78 (0 outside the grid)
 __device__ __forceinline__ int label_or_zero(const Field& f, int i, int j, int k) {
-    if (i < 0 || j < 0 || k < 0 || i >= f.nx || j >= f.ny || k >= f.nz) {
-        return 0;
-    }
-    return f.L[vox(f, i, j, k)];
+    return in_range(f, i, j, k) ? f.L[vox(f, i, j, k)] : 0;
+}
+
+// the voxel coordinate floor(u) for the walks and boxes below, kept where a few steps
+// from it cannot wrap (a grid has far fewer voxels along an axis)
+__device__ __forceinline__ int voxel_coord(float u) {
+    return (int)fminf(fmaxf(floorf(u), -0x1p30f), 0x1p30f);
 }
 
 __device__ __forceinline__ float over_v(const Field& f, float x, int ax) {
@@ -1644,7 +1661,7 @@ __device__ float dda_hit(const Field& f, int a, const float* p, const float* s, 
     for (int k = 0; k < 3; ++k) {
         u[k] = over_v(f, p[k], k) + 0.5f;
         w[k] = over_v(f, s[k], k);
-        id[k] = (int)floorf(u[k]);
+        id[k] = voxel_coord(u[k]);
     }
     int l = label_or_zero(f, id[0], id[1], id[2]);
     if (l != a) {
@@ -1690,7 +1707,7 @@ __device__ float vox_nearest(const Field& f, int a, int b, int c, const float* q
     int ci[3];
     for (int k = 0; k < 3; ++k) {
         u[k] = over_v(f, q[k], k) + 0.5f;
-        ci[k] = (int)floorf(u[k]);
+        ci[k] = voxel_coord(u[k]);
     }
     float best = -1.0f;
     for (int vk = ci[2] - R; vk <= ci[2] + R; ++vk) {
@@ -1785,7 +1802,7 @@ __device__ float vox_nearest_wave(const Field& f, int a, int b, int c, const flo
     int ci[3];
     for (int k = 0; k < 3; ++k) {
         u[k] = over_v(f, q[k], k) + 0.5f;
-        ci[k] = (int)floorf(u[k]);
+        ci[k] = voxel_coord(u[k]);
         qc[k] = q[k];
     }
     const int W = 2 * R + 1, total = W * W * W, nsub = c == kNoLab ? 2 : 4;
@@ -1927,8 +1944,7 @@ __device__ float vox_nearest_wave(const Field& f, int a, int b, int c, const flo
 
 // v2m_vox_third, src/opencl/v2m_particle_body.cl:533-545
 __device__ __forceinline__ int vox_third(const Field& f, int a, int b, const float* p) {
-    const int i0 = (int)floorf(over_vx(f, p[0])), j0 = (int)floorf(over_vy(f, p[1])),
-              k0 = (int)floorf(over_vz(f, p[2]));
+    const int i0 = voxel_coord(over_vx(f, p[0])), j0 = voxel_coord(over_vy(f, p[1])), k0 = voxel_coord(over_vz(f, p[2]));
     for (int m = 0; m < 8; ++m) {
         const int l = label_or_zero(f, i0 + (m & 1), j0 + ((m >> 1) & 1), k0 + (m >> 2));
         if (l != a && l != b) {
@@ -1985,8 +2001,8 @@ __device__ float voxel_step(const Field& f, float h, float snap, int a, const fl
             ty = TN_INTERFACE;
         } else if (snap > 0.0f) {   // close to any wall: snap onto it
             const int Rs = 1 + (int)ceilf(snap * h / vmin);
-            const int qx = (int)floorf(over_vx(f, q[0]) + 0.5f), qy = (int)floorf(over_vy(f, q[1]) + 0.5f),
-                      qz = (int)floorf(over_vz(f, q[2]) + 0.5f);
+            const int qx = voxel_coord(over_vx(f, q[0]) + 0.5f), qy = voxel_coord(over_vy(f, q[1]) + 0.5f),
+                      qz = voxel_coord(over_vz(f, q[2]) + 0.5f);
             // the label Rs voxels away in direction d (dz, dy, dx = d / 9, d / 3 % 3, d % 3, less 1)
             auto dir_label = [&](int d) {
                 return label_or_zero(f, qx + (d % 3 - 1) * Rs, qy + (d / 3 % 3 - 1) * Rs, qz + (d / 9 - 1) * Rs);
