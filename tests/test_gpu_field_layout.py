@@ -131,3 +131,31 @@ def test_stored_layout_where_the_slots_do_not_fit(tn):
     got, _ = run(lo)
     want, _ = tn.relax(case.grid, Nodes(P[:lo], lab[:lo], typ[:lo], part[:lo]), prm, device=0)
     assert got.equal(want)
+
+
+@pytest.mark.parametrize("shape,nlab,blocks,vs,seed", [
+    ((23, 27, 45), 3, 2, (0.976, 0.993, 1.223), 1168), ((15, 36, 21), 3, 2, (0.596, 1.492, 1.432), 1173)])
+def test_corner_steps_that_run_away(tn, shape, nlab, blocks, vs, seed):
+    """Volumes of small blocks, among whose corners are some with nearly dependent gradients:
+    their Newton steps go 3e9 and 8e9 voxels out (with the voxel sizes' further digits) and are
+    then dropped for the vertex itself"""
+    from trussnet_amd import gridbuild
+    from trussnet_amd._abi import GridParams
+
+    rng = np.random.default_rng(seed)
+    assert shape == tuple(int(v) for v in rng.integers(5, 56, 3))
+    assert nlab == int(rng.integers(1, 6)) and blocks == int(rng.choice([2, 3, 5, 9, 16]))
+    lab = rng.integers(0, nlab + 1, [(s + blocks - 1) // blocks for s in shape]).astype(np.uint16)
+    for ax in range(3):
+        lab = np.repeat(lab, blocks, axis=ax)
+    lab = np.ascontiguousarray(lab[:shape[0], :shape[1], :shape[2]])
+    rng.random()
+    size = tuple(float(v) for v in rng.uniform(0.5, 2, 3))
+    assert np.allclose(size, vs, atol=1e-3)
+    h = float(rng.uniform(0.8, 2.5)) * min(size)
+    grid = gridbuild.build(lab, size, GridParams(hbase=h, hmin=h, hmax=h), device=0)
+    seeds = tn.seed(grid, RelaxParams(), device=0)
+    corner = seeds.P[seeds.typ == 3] / np.array(size, np.float32)
+    off = corner - (np.floor(corner) + 0.5)
+    assert len(corner) > 100 and (off ** 2).sum(1).max() < 0.76 and ((off ** 2).sum(1) <= 0.2501).mean() > 0.9
+    assert tn.seed(grid, RelaxParams(), device=0).equal(seeds)
