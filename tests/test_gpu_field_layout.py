@@ -125,9 +125,13 @@ def test_stored_layout_where_the_slots_do_not_fit(tn):
             return None
 
     lo, hi = 1000, s.n * reps
+    assert run(hi) is None
     while hi - lo > 500:   # the largest count that fits, to 0.25 MB
         mid = (lo + hi) // 2
         lo, hi = (mid, hi) if run(mid) is not None else (lo, mid)
+    # 500 nodes more were refused: less is left than these take (328 bytes each, about 50 buffers
+    # in steps of 256), and the slots take more than that
+    assert 4 * 736 * case.grid.nslot > 500 * 400 + 50 * 256
     got, _ = run(lo)
     want, _ = tn.relax(case.grid, Nodes(P[:lo], lab[:lo], typ[:lo], part[:lo]), prm, device=0)
     assert got.equal(want)
