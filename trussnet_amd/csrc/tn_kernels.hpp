@@ -544,7 +544,7 @@ __global__ __launch_bounds__(kBlock) void k_permute(const int32_t* __restrict__ 
 // every one is.
 
 constexpr int kTrussWave = 64;   // one wave per block
-constexpr int kCollect = 32;   // per-lane candidate buffer (entries): settled by a 32-key network
+constexpr int kCollect = 32;   // per-lane candidate buffer (entries): half a wave's lanes hold one when it is cut back
 // waves a SIMD: 160 registers and no spill (at 4, 128 registers, 2.5 M nodes took longer)
 constexpr int kTrussOcc = 3;
 constexpr int kMinRoom = 4;    // a lane with less room than this (and more possible hits) settles first
@@ -2096,7 +2096,7 @@ constexpr int kHeldChunks = 8;       // chunks of nodes after which a block writ
 // power partial sums (src/v2m_particles.cpp:849-937). Counts are reduced per
 // wave with ballots before any atomic, and the listed nodes gathered in LDS, so that a
 // block takes its place in the list once (a pass of its own over a flag a node, as
-// before, cost 8 us an iteration at 2.5 M nodes and a launch at any size). LDS holds
+// before, cost 8 us an iteration at 2.5 M nodes and a launch at any size; 57 us there). LDS holds
 // every node of kHeldChunks chunks, and the block writes the list out after that many
 // whatever it holds: the chunk's number is the same in every wave, while the count held
 // may already be another wave's next, and the writing has barriers that all must reach.
@@ -2298,8 +2298,8 @@ struct CtlArgs {
 // The control block goes to the host from here, by stores to pinned memory (host, if it is
 // not null), and the own-list refreshes are launched after the event that the host waits
 // for: a copy between the refreshes and the event cost each iteration its own latency, and
-// the host enqueued the next iteration only after both (75 k nodes to convergence: 45.2 ->
-// 40.5 ms, 270 iterations; 435 k nodes, 100 iterations: 42.1 -> 41.2).
+// the host enqueued the next iteration only after both (435 k nodes, 100 iterations: 42.1 ->
+// 41.2 ms; at 75 k nodes to convergence the runs of one side differ by more than the gain).
 __device__ __forceinline__ void k_control_step(CtlArgs ca, Ctl* __restrict__ ctl, const double2* __restrict__ partials, const float* __restrict__ pw, const int32_t* __restrict__ slot_of, int bid, int nblk) {
     __shared__ double red[kBlock][2];
     __shared__ float chunk[kScanTile];
